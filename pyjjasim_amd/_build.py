@@ -2,17 +2,20 @@
 
 The shared library holds the HIP kernels, the device plan and the host-side
 Cholesky factorisation. It is built next to this file so that it travels with the
-source tree; nothing is installed elsewhere.
+source tree; nothing is installed elsewhere. The sources compile side by side
+(each to an object in a temporary folder) and are linked once.
 """
 import os
 import subprocess
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libjja.so")
 
 HIPCC_FLAGS = [
-    "-O3", "--offload-arch=gfx950", "-fPIC", "-shared", "-std=c++17",
+    "-O3", "--offload-arch=gfx950", "-fPIC", "-std=c++17",
     # the step expressions keep the reference's operation order: no FMA contraction
     "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -21,17 +24,24 @@ HIPCC_FLAGS = [
 
 
 def sources():
-    return [os.path.join(CSRC, "jja_evolve.hip"), os.path.join(CSRC, "jja_factor.cpp")]
+    return [os.path.join(CSRC, name) for name in ("jja_evolve.hip", "jja_factor.cpp")]
 
 
 def build_library(verbose=False):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-    tmp = LIB + ".tmp"
-    cmd = [hipcc, *HIPCC_FLAGS, *sources(), "-o", tmp]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    subprocess.run(cmd, check=True)
-    os.replace(tmp, LIB)
+
+    def run(cmd):
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        subprocess.run(cmd, check=True)
+
+    with tempfile.TemporaryDirectory() as tmp:
+        objects = [os.path.join(tmp, os.path.basename(src) + ".o") for src in sources()]
+        with ThreadPoolExecutor(len(objects)) as pool:
+            list(pool.map(lambda so: run([hipcc, *HIPCC_FLAGS, "-c", so[0], "-o", so[1]]), zip(sources(), objects)))
+        out = LIB + ".tmp"
+        run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *objects, "-o", out])
+    os.replace(out, LIB)
     return LIB
 
 
