@@ -217,6 +217,7 @@ typedef struct jja_problem_desc {
    * x_r = d_r - ((-g) inv[r][k]) x_{r+1} */
   const double* lattice_inv;
   double lattice_g;            /* g */
+  double lattice_gc;           /* g_c */
 } jja_problem_desc;
 
 /*

@@ -99,7 +99,36 @@ struct DevProblem {
   const double* lat_sine_p;    // [ES][2][CP/2]: the same table, even and odd modes apart (matrix-core B operands)
   const double* lat_inv;       // [R][CP] inverse Thomas pivots
   double lat_g;
+  // LDS store of a lattice whose padded form fits (lat_ld 0: it does not): two
+  // copies of the face vector with rows of lat_ld doubles, the second at
+  // lat_buf, then the sine tables of both sides at lat_tab (DstShape)
+  int32_t lat_ld, lat_buf, lat_tab;
+  int32_t store_doubles;       // LDS store: doubles a column's store takes
+  const double* lat_table;     // the sine tables (C's, then R's unless R == C)
+  const double* lat_lam;       // [padded rows][lat_ld] inverse eigenvalues, 0 in the padding
+  const int32_t* face_addr;    // [n_slice_rows]: store address of a face record's row slot
 };
+
+// The sine matrix of n modes as operands of v_mfma_f64_16x16x4f64: modes of one
+// parity in blocks of 16, the folded index i in steps of 4 (an even count). Lane l
+// of (pair of blocks b, step k, parity p) holds S[4k + l/16][2 (16 b + l%16) + p]
+// at ((b * steps + k) * 2 + p) * 64 + l, 0 past the matrix; the middle element of
+// an odd n, which the fold adds to itself, is halved.
+struct DstShape {
+  int32_t n, h, pairs, steps;
+  __host__ __device__ __forceinline__ explicit DstShape(int32_t modes)
+      : n(modes), h((modes + 1) >> 1), pairs((h + 15) >> 4), steps((((h + 3) >> 2) + 1) & ~1) {}
+  __host__ __device__ __forceinline__ int32_t entries() const { return pairs * steps * 2 * 64; }
+  // rows or columns that outputs of all blocks take
+  __host__ __device__ __forceinline__ int32_t padded() const { return 32 * pairs; }
+};
+
+// Store address of solve position q (an LDS store; the global one is linear).
+__device__ __forceinline__ int32_t store_address(const DevProblem& P, int32_t q) {
+  if (!P.lat_ld) return q;
+  const int32_t r = q / P.lat_cols;
+  return r * P.lat_ld + (q - r * P.lat_cols);
+}
 
 // The current-phase relation's sum at one argument: sin(arg) for the default
 // relation, else sum_k a_k sin((k+1) arg) accumulated in ascending k (each
@@ -634,6 +663,114 @@ __device__ __forceinline__ void lattice_transform_lds(const DevProblem& P, const
   }
 }
 
+// The solve of an LDS store with room for padding: both sides of the lattice by
+// sine transforms, X = S_R ((S_R B S_C) / lambda) S_C with lambda = g mu_R +
+// g_c mu_C, as four products on the matrix cores between two copies of the face
+// vector. A wave takes 16 x 16 tiles of v_mfma_f64_16x16x4f64 (lane l holds
+// A[l%16][l/16] and B[l/16][l%16], result register q D[l/16 + 4q][l%16]): one
+// operand comes from the sine table in LDS, the other is the sum (even modes) or
+// difference (odd modes) of two mirrored elements, folded as they are read
+// (S[n-1-i][j] = (-1)^j S[i][j]); a wave takes an even and an odd block of modes
+// together. Rows and columns are padded to whole blocks of zeros, so nothing is
+// clamped or masked.
+//   Small lattices are bound by latency: one wave issues an instruction in 4 to 8
+// cycles, so what counts is the instructions of a stage and the number of
+// barriers (four here, against ten with folds, transforms of the rows only and
+// blocked recurrences along them).
+
+// dst[r][j] = sum_i src[r][i] S[i][j] (LEFT false), or dst[i][c] = lam[i][c]
+// sum_r S[i][r] src[r][c] (LEFT true; lam may be NULL)
+template <bool LEFT>
+__device__ __forceinline__ void dst_product(const LAS double* src, LAS double* dst, const LAS double* table,
+                                            const GAS double* lam, int32_t n, int32_t other, int32_t ld, int32_t tid,
+                                            int32_t nt) {
+  const DstShape D(n);
+  const int lane = tid & (kWave - 1), lr = lane & 15, lk = lane >> 4;
+  const int32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave), NW = nt / kWave;
+  const int32_t tasks = D.pairs * ((other + 15) >> 4);
+  // task = block of the other side * pairs + mode pair, split by subtraction (a
+  // division costs more than the few rounds)
+  for (int32_t task = wave, mb = wave, ob = 0; task < tasks; task += NW, mb += NW) {
+    while (mb >= D.pairs) {
+      mb -= D.pairs;
+      ob += 16;
+    }
+    const LAS double* f = table + mb * D.steps * 2 * kWave + lane;
+    // element i of the folded side at s0 + i * si, its mirror at s1 - i * si
+    const int32_t si = LEFT ? ld : 1, o = LEFT ? ob + lr : (ob + lr) * ld;
+    const LAS double* s0 = src + o + lk * si;
+    const LAS double* s1 = src + o + (n - 1 - lk) * si;
+    const int32_t out = LEFT ? 2 * (16 * mb + lk) * ld + ob + lr : (ob + lk) * ld + 2 * (16 * mb + lr);
+    double scale[4][2];
+    if (LEFT && lam) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        scale[r][0] = lam[out + 8 * r * ld];
+        scale[r][1] = lam[out + (8 * r + 1) * ld];
+      }
+    }
+    vdouble4 ae{0.0, 0.0, 0.0, 0.0}, ao{0.0, 0.0, 0.0, 0.0};
+    for (int32_t k = 0; k < D.steps; k += 2) {
+      double p[2], q[2], v[2][2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        p[u] = s0[4 * u * si];
+        q[u] = s1[-4 * u * si];
+        v[u][0] = f[(2 * u) * kWave];
+        v[u][1] = f[(2 * u + 1) * kWave];
+      }
+      s0 += 8 * si;
+      s1 -= 8 * si;
+      f += 4 * kWave;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const double e = p[u] + q[u], d = p[u] - q[u];
+        if constexpr (LEFT) {
+          ae = __builtin_amdgcn_mfma_f64_16x16x4f64(v[u][0], e, ae, 0, 0, 0);
+          ao = __builtin_amdgcn_mfma_f64_16x16x4f64(v[u][1], d, ao, 0, 0, 0);
+        } else {
+          ae = __builtin_amdgcn_mfma_f64_16x16x4f64(e, v[u][0], ae, 0, 0, 0);
+          ao = __builtin_amdgcn_mfma_f64_16x16x4f64(d, v[u][1], ao, 0, 0, 0);
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if constexpr (LEFT) {
+        dst[out + 8 * r * ld] = lam ? ae[r] * scale[r][0] : ae[r];
+        dst[out + (8 * r + 1) * ld] = lam ? ao[r] * scale[r][1] : ao[r];
+      } else {
+        *reinterpret_cast<LAS vdouble2*>(dst + out + 4 * r * ld) = vdouble2{ae[r], ao[r]};
+      }
+    }
+  }
+}
+
+__device__ __forceinline__ void solve_lattice_padded(const DevProblem& P, const FaceStore<false>& zs) {
+  const int32_t R = P.lat_rows, C = P.lat_cols, ld = P.lat_ld;
+  LAS double* z = (LAS double*)zs.p;
+  LAS double* t = z + P.lat_buf;
+  const LAS double* tc = z + P.lat_tab;
+  const LAS double* tr = R == C ? tc : tc + DstShape(C).entries();
+  dst_product<false>(z, t, tc, nullptr, C, R, ld, zs.vt, zs.vbs);
+  zs.barrier();
+  dst_product<true>(t, z, tr, gbl(P.lat_lam), R, C, ld, zs.vt, zs.vbs);
+  zs.barrier();
+  dst_product<true>(z, t, tr, nullptr, R, C, ld, zs.vt, zs.vbs);
+  zs.barrier();
+  dst_product<false>(t, z, tc, nullptr, C, R, ld, zs.vt, zs.vbs);
+  zs.barrier();
+}
+
+// Zeros in both copies of the face vector (their padding stays zero) and the sine
+// tables: every kernel with an LDS store, before it writes its first face value.
+__device__ __forceinline__ void init_store(const DevProblem& P, double* lds, int32_t tid, int32_t nt) {
+  if (!P.lat_ld) return;
+  for (int32_t i = tid; i < P.lat_tab; i += nt) lds[i] = 0.0;
+  for (int32_t i = P.lat_tab + tid; i < P.store_doubles; i += nt) lds[i] = gbl(P.lat_table)[i - P.lat_tab];
+  __syncthreads();
+}
+
 // The same sums for a global store, on the matrix cores: for each parity p,
 // out[r][2m+p] = sum_i F_p[r][i] S[i][2m+p] (F_0 = E, F_1 = O) is a product
 // of an R x ES and an ES x (modes of parity p) matrix. A wave takes a tile of
@@ -1020,6 +1157,12 @@ template <class Z>
 __device__ __forceinline__ void solve_face_system(const DevProblem& P, const Z& zs) {
   if constexpr (RunsLattice<Z>::value) {
     if (P.lat_rows) {
+      if constexpr (!Z::kGlobal) {
+        if (P.lat_ld) {
+          solve_lattice_padded(P, zs);
+          return;
+        }
+      }
       solve_lattice(P, zs);
       return;
     }
@@ -1138,7 +1281,7 @@ __device__ __forceinline__ double term_at(const TermView& v, int32_t i) {
 // so a group costs two memory round trips.
 struct FaceRec {
   int32_t cd[kFaceIter];  // +-junction codes, -1 past the face's length
-  int32_t pos;            // solve position written at FINISH, or -1
+  int32_t pos;            // store address written at FINISH, or -1
   int32_t fid;            // face index of that position (flux input), or -1
   bool finish;
 };
@@ -1152,7 +1295,7 @@ __device__ __forceinline__ void face_rec_load(const DevProblem& P, int32_t k, bo
   for (int i = 0; i < kFaceIter; ++i) r.cd[i] = (live && i < m.n_iter) ? code[i * vbs] : -1;
   r.finish = present && (m.flags & JJA_SLICE_FINISH);
   const bool rowed = live && r.finish;
-  r.pos = rowed ? gbl(P.slice_rows)[m.rowbase + tid] : -1;
+  r.pos = rowed ? gbl(P.face_addr)[m.rowbase + tid] : -1;
   r.fid = rowed ? gbl(P.face_fid)[m.rowbase + tid] : -1;
 }
 
@@ -1587,6 +1730,7 @@ __device__ __forceinline__ void evolve_column(const DevProblem& P, const jja_pro
     zs.p = lds;
   zs.vt = threadIdx.x;
   zs.vbs = BS;
+  if constexpr (!GLOBAL) init_store(P, lds, threadIdx.x, BS);
   evolve_steps<BS, SW>(P, R, w, zs, n_steps, step0);
 }
 
@@ -1712,7 +1856,8 @@ __device__ __forceinline__ void adjoint_steps(const DevProblem& P, const jja_adj
       zs.barrier();
       solve_face_system(P, zs);
     }
-    for (int32_t p = zs.vt; p < P.Nf; p += zs.vbs) gf[p] = gf[p] - kTwoPi * zs.rd(p);
+    for (int32_t p = zs.vt; p < P.Nf; p += zs.vbs)
+      gf[p] = gf[p] - kTwoPi * zs.rd(Z::kGlobal ? p : store_address(P, p));
     adjoint_junctions(P, A, C, zs, k, w);
     zs.sync();
   }

@@ -37,6 +37,7 @@
 
 #include "../../include/jja.h"
 #include "jja_device.h"
+#include "jja_resident.h"
 
 // Device scratch of jja_solve_noalloc (a global face store for its columns):
 // 2^21 doubles (16 MiB) per GPU, held until the process ends. Calls on one
@@ -130,6 +131,7 @@ __global__ __launch_bounds__(BS) void adjoint_kernel(const DevProblem* __restric
     zs.p = lds;
   zs.vt = threadIdx.x;
   zs.vbs = BS;
+  if constexpr (!GLOBAL) init_store(P, lds, threadIdx.x, BS);
   adjoint_steps<BS>(P, A, w, zs, k_hi, k_lo);
 }
 
@@ -217,15 +219,16 @@ __global__ __launch_bounds__(BS) void spd_solve_kernel(const DevProblem* __restr
   const GAS double* __restrict__ bc = gbl(b) + col * ldb;
   GAS double* __restrict__ xc = gblw(x) + col * ldx;
   const GAS int32_t* __restrict__ fop = gbl(P.face_of_pos);
+  if constexpr (!GLOBAL) init_store(P, lds, threadIdx.x, BS);
   for (int32_t q = threadIdx.x; q < P.Nf; q += BS) {
     const double v = bc[fop[q]];
-    zs.wr(q, v);
+    zs.wr(GLOBAL ? q : store_address(P, q), v);
     if (q < P.copy_rows) zs.wr(P.Nf + q, v);
   }
   zs.sync();
   solve_face_system(P, zs);
   zs.sync();
-  for (int32_t q = threadIdx.x; q < P.Nf; q += BS) xc[fop[q]] = zs.rd(q);
+  for (int32_t q = threadIdx.x; q < P.Nf; q += BS) xc[fop[q]] = zs.rd(GLOBAL ? q : store_address(P, q));
 }
 
 struct Plan {
@@ -267,6 +270,33 @@ struct Plan {
   std::vector<std::pair<const void*, int>> lds_attr;
   std::vector<std::pair<const void*, int>> per_cu;
 };
+
+// The sine matrix of n modes in DstShape's layout, and T_n's eigenvalues
+// 4 sin^2(pi (k + 1) / (2 (n + 1))); angles reduced to a period in integers
+std::vector<double> dst_table(int32_t n) {
+  const DstShape D(n);
+  std::vector<double> t(static_cast<size_t>(D.entries()), 0.0);
+  const double pi = 3.14159265358979323846, norm = std::sqrt(2.0 / (n + 1));
+  for (size_t e = 0; e < t.size(); ++e) {
+    const int64_t l = e % kWave, par = e / kWave % 2, k = e / (2 * kWave) % D.steps, b = e / (2 * kWave) / D.steps;
+    const int64_t j = 2 * (16 * b + l % 16) + par, i = 4 * k + l / 16;
+    if (i >= D.h || j >= n) continue;
+    const int64_t m = (i + 1) * (j + 1) % (2 * (static_cast<int64_t>(n) + 1));
+    if (m % (n + 1) == 0) continue;  // the sine of a multiple of pi
+    const double v = norm * std::sin(pi * static_cast<double>(m) / (n + 1));
+    t[e] = 2 * i + 1 == n ? 0.5 * v : v;
+  }
+  return t;
+}
+
+std::vector<double> dst_eigenvalues(int32_t n) {
+  std::vector<double> mu(n);
+  for (int32_t k = 0; k < n; ++k) {
+    const double s = std::sin(3.14159265358979323846 * (k + 1) / (2.0 * (n + 1)));
+    mu[k] = 4.0 * s * s;
+  }
+  return mu;
+}
 
 template <typename T>
 int upload(Plan* plan, const T* host, size_t n, const T** out) {
@@ -464,6 +494,8 @@ int validate(const jja_problem_desc& d) {
     if (ms < (Nf & 1) + std::max(2 * R * EF, 4 * B * C))
       return fail(JJA_EINVAL, "max_stage_rows too small for the lattice solve");
     if (!(d.lattice_g > 0.0) || !std::isfinite(d.lattice_g)) return fail(JJA_EINVAL, "lattice_g must be finite and > 0");
+    if (!(d.lattice_gc > 0.0) || !std::isfinite(d.lattice_gc))
+      return fail(JJA_EINVAL, "lattice_gc must be finite and > 0");
     return JJA_OK;
   }
   // solve programs: one per wave of 64 lanes; each runs a multiple of three
@@ -597,6 +629,50 @@ int launch_evolve_sw(Plan* plan, const WorkItem* work, int32_t n, int64_t lds, i
     case 4: return launch_evolve<BS, 4, STORE>(plan, work, n, lds, n_steps, step0, stream);
     default: return launch_evolve<BS, 5, STORE>(plan, work, n, lds, n_steps, step0, stream);
   }
+}
+
+// How a launch can keep every column's state on chip (jja_resident.hip): the
+// junction pairs each thread keeps in registers (1, 2), 0 for the state in LDS,
+// or -1 when some problem or run needs the general kernel. *lds receives the
+// dynamic LDS bytes of the widest column. The resident kernels take the usual
+// step: stencil 3, no voltage sources, noise from Philox with a given
+// amplitude or none.
+int resident_form(const Plan* plan, const jja_problem_run* runs, int64_t* lds) {
+  if (plan->stencil_width != 3 || plan->block_size > 512) return -1;
+  const int32_t BS = plan->block_size;
+  int32_t form = 1;
+  for (size_t p = 0; p < plan->problems.size(); ++p) {
+    const DevProblem& d = plan->problems[p];
+    const jja_problem_run& r = runs[p];
+    if (d.index_bytes != 2 || !r.Vs.zero || r.noise || (!r.T.zero && !r.sigma.base)) return -1;
+    const int32_t per = ((d.Nj + 1) / 2 + BS - 1) / BS;
+    const int32_t need = d.n_face_slices <= kResidentFaces * kResidentPairs && per <= kResidentPairs
+                             ? std::max(per, (d.n_face_slices + kResidentFaces - 1) / kResidentFaces)
+                             : 0;
+    if (need == 0 && d.n_face_slices > kResidentRecords) return -1;
+    form = form == 0 || need == 0 ? 0 : std::max(form, need);
+  }
+  *lds = 8;
+  for (const DevProblem& d : plan->problems) {
+    // face vector and scratch, then u (registers) or x, theta_{t-1} and, when
+    // each junction has its own 1/c0, u
+    const int64_t store = d.store_doubles;
+    const int64_t arrays = form > 0 ? 1 : d.coef_si == 0 ? 2 : 3;
+    *lds = std::max(*lds, 8 * (store + arrays * 2 * ((static_cast<int64_t>(d.Nj) + 1) / 2)));
+  }
+  return *lds <= plan->lds_limit ? form : -1;
+}
+
+int launch_resident(Plan* plan, int32_t n, int form, int64_t lds, int32_t n_steps, int64_t step0, hipStream_t stream) {
+  const void* kern = resident_evolve_kernel(plan->block_size, form);
+  if (!kern) return fail(JJA_EUNSUPPORTED, "no resident kernel for this workgroup size");
+  if (int rc = set_lds_limit(plan, kern, static_cast<int>(lds))) return rc;
+  const DevProblem* probs = plan->d_problems;
+  const jja_problem_run* runs = plan->d_runs;
+  const WorkItem* work = plan->d_work;
+  void* argv[] = {&probs, &runs, &work, &n_steps, &step0};
+  JJA_HIP(hipLaunchKernel(kern, dim3(n), dim3(plan->block_size), argv, static_cast<size_t>(lds), stream));
+  return JJA_OK;
 }
 
 template <int STORE>
@@ -883,6 +959,29 @@ int jja_plan_create(int32_t n_problems, const jja_problem_desc* descs, jja_plan*
         if ((rc = upload(plan, split.data(), n, &dp.lat_sine_p))) break;
       }
       if ((rc = upload(plan, d.lattice_inv, static_cast<size_t>(R) * dp.lat_cp, &dp.lat_inv))) break;
+      // padded LDS form: the table steps and their mirrors stay inside sides of 8
+      // a side; rows of 32 k + 4 doubles put the 16 rows of a tile on all banks
+      const DstShape dc(C), dr(R);
+      const int32_t ld = dc.padded() + 4;
+      const int64_t buf = static_cast<int64_t>(dr.padded()) * ld;
+      const int64_t tables = dc.entries() + (R == C ? 0 : dr.entries());
+      if (d.index_bytes == 2 && R >= 8 && C >= 8 && 8 * (2 * buf + tables) <= plan->lds_limit) {
+        dp.lat_ld = ld;
+        dp.lat_buf = static_cast<int32_t>(buf);
+        dp.lat_tab = static_cast<int32_t>(2 * buf);
+        dp.store_doubles = static_cast<int32_t>(2 * buf + tables);
+        std::vector<double> t = dst_table(C), lam(static_cast<size_t>(buf), 0.0);
+        if (R != C) {
+          const std::vector<double> tr = dst_table(R);
+          t.insert(t.end(), tr.begin(), tr.end());
+        }
+        const std::vector<double> mc = dst_eigenvalues(C), mr = dst_eigenvalues(R);
+        for (size_t i = 0; i < static_cast<size_t>(R); ++i)
+          for (size_t j = 0; j < static_cast<size_t>(C); ++j)
+            lam[i * ld + j] = 1.0 / (d.lattice_g * mr[i] + d.lattice_gc * mc[j]);
+        if ((rc = upload(plan, t.data(), t.size(), &dp.lat_table))) break;
+        if ((rc = upload(plan, lam.data(), lam.size(), &dp.lat_lam))) break;
+      }
     }
     const size_t Nj = d.n_junctions, Nf = d.n_faces;
     if ((rc = upload(plan, d.Ic, Nj, &dp.Ic))) break;
@@ -900,7 +999,14 @@ int jja_plan_create(int32_t n_problems, const jja_problem_desc* descs, jja_plan*
       for (size_t j = 0; j < Nj; ++j) rc0[j] = 1.0 / d.coef[j];
       if ((rc = upload(plan, rc0.data(), Nj, &dp.rc0))) break;
     }
-    if ((rc = upload(plan, d.junc_code, 2 * Nj, &dp.junc_code))) break;
+    // incidence codes and face rows by store address
+    auto address = [&](int32_t q) { return dp.lat_ld ? q / dp.lat_cols * dp.lat_ld + q % dp.lat_cols : q; };
+    {
+      std::vector<int32_t> code(d.junc_code, d.junc_code + 2 * Nj);
+      for (int32_t& c : code)
+        if (c >= 0) c = 2 * address(c >> 1) + (c & 1);
+      if ((rc = upload(plan, code.data(), code.size(), &dp.junc_code))) break;
+    }
     if (Nf) {
       if ((rc = upload(plan, d.face_of_pos, Nf, &dp.face_of_pos))) break;
       if ((rc = upload(plan, d.face_slices, static_cast<size_t>(d.n_face_slices), &dp.face_slices))) break;
@@ -908,6 +1014,13 @@ int jja_plan_create(int32_t n_problems, const jja_problem_desc* descs, jja_plan*
       if ((rc = upload(plan, d.solve_wave_ptr, static_cast<size_t>(d.block_size / kWave + 1), &dp.wave_ptr))) break;
       if ((rc = upload(plan, d.face_code, static_cast<size_t>(d.n_face_entries), &dp.face_code))) break;
       if ((rc = upload(plan, d.slice_rows, static_cast<size_t>(d.n_slice_rows), &dp.slice_rows))) break;
+      dp.face_addr = dp.slice_rows;
+      if (dp.lat_ld) {
+        std::vector<int32_t> at(d.slice_rows, d.slice_rows + d.n_slice_rows);
+        for (int32_t& q : at)
+          if (q >= 0) q = address(q);
+        if ((rc = upload(plan, at.data(), at.size(), &dp.face_addr))) break;
+      }
       {
         // face index of every row slot a face record finishes (the flux input)
         std::vector<int32_t> fid(static_cast<size_t>(d.n_slice_rows), -1);
@@ -936,9 +1049,9 @@ int jja_plan_create(int32_t n_problems, const jja_problem_desc* descs, jja_plan*
       static const double zeros[8] = {0, 0, 0, 0, 0, 0, 0, 0};
       if ((rc = upload(plan, zeros, 8, &dp.zero))) break;
     }
+    if (!dp.lat_ld) dp.store_doubles = (d.n_faces + d.max_stage_rows + 1) & ~1;
     plan->problems.push_back(dp);
-    const int64_t store = (static_cast<int64_t>(d.n_faces) + d.max_stage_rows) * static_cast<int64_t>(sizeof(double));
-    plan->lds_bytes.push_back(d.index_bytes == 2 ? store : 0);
+    plan->lds_bytes.push_back(d.index_bytes == 2 ? static_cast<int64_t>(dp.store_doubles) * 8 : 0);
     // work of one column step in factor-entry units (a lattice solve: its multiply-adds)
     const int64_t solve_work = d.lattice_rows ? static_cast<int64_t>(d.n_faces) * (d.lattice_cols + 1) : d.n_entries;
     plan->cost.push_back(solve_work + d.n_face_entries + 8 * static_cast<int64_t>(d.n_junctions));
@@ -1095,7 +1208,11 @@ int jja_evolve(jja_plan* p, const jja_problem_run* runs, int32_t n_steps, int64_
     if ((rc = upload_work(plan, work, stream))) return rc;
     if (lds < 8) lds = 8;
     const int32_t n = n_lds + n_g;
-    if (n_g == 0)
+    int64_t resident_lds = 0;
+    const int form = n_g == 0 ? resident_form(plan, runs, &resident_lds) : -1;
+    if (form >= 0)
+      rc = launch_resident(plan, n, form, resident_lds, n_steps, step0, stream);
+    else if (n_g == 0)
       rc = launch_evolve_bs<0>(plan, plan->d_work, n, lds, n_steps, step0, stream);
     else if (n_lds == 0)
       rc = launch_evolve_bs<1>(plan, plan->d_work, n, 8, n_steps, step0, stream);

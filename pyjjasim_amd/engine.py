@@ -121,12 +121,18 @@ def set_cpr(desc, cpr):
         desc.cpr_coef[k] = float(coef[k])
 
 
+# junctions up to which a column's whole state fits in one workgroup's LDS
+# beside the face vector (or in registers): the kernels for that take at most
+# 512 threads, which then have 256 registers each
+RESIDENT_JUNCTIONS = 6144
+
+
 def default_block_size(Nj, Nf):
     work = max(Nj, Nf)
     for bs in (64, 128, 256, 512):
         if work <= 2 * bs:
             return bs
-    return 1024
+    return 512 if work <= RESIDENT_JUNCTIONS else 1024
 
 
 def device_compute_units():

@@ -178,7 +178,7 @@ class LatticeSolve:
         d.lattice_rows, d.lattice_cols = self.R, self.C
         d.lattice_sine = P(self.sine, _native.C.c_double)
         d.lattice_inv = P(self.inv, _native.C.c_double)
-        d.lattice_g = self.g_r
+        d.lattice_g, d.lattice_gc = self.g_r, self.g_c
 
     # ------------------------------------------------------ host emulation
     def _fold(self, Z):
