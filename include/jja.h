@@ -193,7 +193,13 @@ typedef struct jja_problem_desc {
    * (static_problem.py:77-85); n terms for Ic * sum_{k<n} cpr_coef[k] sin((k+1) theta),
    * the device form of a sine-series relation (jja_adjoint: default only) */
   int32_t cpr_terms;
-  int32_t cpr_pad_;
+  /* 1: a split lattice column may run as row slabs: each part keeps the junctions
+   * of its face rows on chip and the parts exchange their end rows once a step.
+   * Needs lattice_rows, parts >= 2, workgroups of 512 threads and a plan of this
+   * problem alone; runs it does not take (voltage sources, given normals, noise
+   * whose temperature varies in time) and lattices whose slabs do not fit run as
+   * other split columns. Changes the rounding of the lattice solve only. */
+  int32_t lattice_slabs;
   double cpr_coef[JJA_CPR_MAX_TERMS];
   /* Lattice solve: 0 rows, or the face system of a rectangular lattice of
    * R x C faces at positions r*C + c whose face matrix is the Kronecker sum

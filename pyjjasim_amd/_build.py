@@ -19,12 +19,12 @@ HIPCC_FLAGS = [
     # the step expressions keep the reference's operation order: no FMA contraction
     "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-    "-Wall", "-Wno-unused-result",
+    "-Wall", "-Wno-unused-result", "-mllvm", "-disable-machine-licm",
 ]
 
 
 def sources():
-    return [os.path.join(CSRC, name) for name in ("jja_evolve.hip", "jja_resident.hip", "jja_factor.cpp")]
+    return [os.path.join(CSRC, name) for name in ("jja_evolve.hip", "jja_resident.hip", "jja_slab.hip", "jja_factor.cpp")]
 
 
 def build_library(verbose=False):

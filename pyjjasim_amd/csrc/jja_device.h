@@ -151,6 +151,31 @@ __device__ __forceinline__ double rc0_at(const DevProblem& P, int32_t j) {
   return gbl(P.rc0)[static_cast<int64_t>(j) * P.coef_si];
 }
 
+// A value the compiler must assume changed: what is computed from it inside a loop
+// is then formed there instead of being hoisted into registers that live through
+// the whole loop (addresses of every array and constants spill otherwise).
+__device__ __forceinline__ int32_t opaque(int32_t v) {
+  __asm__ volatile("" : "+v"(v));
+  return v;
+}
+// The same for a wave-uniform value: a zero to add to an index.
+__device__ __forceinline__ int32_t opaque_zero() {
+  int32_t z = 0;
+  __asm__ volatile("" : "+s"(z));
+  return z;
+}
+
+// 16-bit incidence codes (2 * address + sign, 0xffff empty) of the kernels that
+// keep them in registers, two to a word: +-v by the sign bit, 0 for an empty slot
+__device__ __forceinline__ double signed_value(double v, uint32_t code) {
+  const long long b = __builtin_bit_cast(long long, v) ^ (static_cast<long long>(code & 1u) << 63);
+  return code == 0xffffu ? 0.0 : __builtin_bit_cast(double, b);
+}
+__device__ __forceinline__ uint32_t code_address(uint32_t code) { return code == 0xffffu ? 0u : code >> 1; }
+__device__ __forceinline__ uint32_t pack_codes(int32_t a, int32_t b) {
+  return static_cast<uint32_t>(a & 0xffff) | (static_cast<uint32_t>(b & 0xffff) << 16);
+}
+
 struct WorkItem {
   int32_t problem;
   int32_t column;  // column (times the problem's parts, plus the part, in a split launch)

@@ -38,6 +38,7 @@
 #include "../../include/jja.h"
 #include "jja_device.h"
 #include "jja_resident.h"
+#include "jja_slab.h"
 
 // Device scratch of jja_solve_noalloc (a global face store for its columns):
 // 2^21 doubles (16 MiB) per GPU, held until the process ends. Calls on one
@@ -255,6 +256,13 @@ struct Plan {
                                      // [1] workgroups whose column ran on one XCD
   int32_t n_cu = 0;                  // compute units of the device
   uint32_t wait_limit = kWaitLimit;  // split launches: polls before a column barrier gives up
+  // a lattice column as row slabs (one problem): the device descriptor, dynamic LDS
+  // doubles, pairs a thread holds and the sequence number of the last step
+  SlabDev slab{};
+  SlabDev* d_slab = nullptr;
+  int64_t slab_lds = 0;
+  int32_t slab_pairs = 0;
+  uint32_t slab_seq = 0;
   int64_t split_lds = 0;             // split launches: dynamic LDS bytes (part-local lattice solves)
   // what the device copies of the launch descriptors hold: a launch uploads
   // only what changed since the previous one
@@ -308,6 +316,40 @@ int upload(Plan* plan, const T* host, size_t n, const T** out) {
   plan->allocations.push_back(d);
   JJA_HIP(hipMemcpy(d, host, n * sizeof(T), hipMemcpyHostToDevice));
   *out = static_cast<const T*>(d);
+  return JJA_OK;
+}
+
+// The slab form of a split lattice problem, where it asks for it and fits.
+int create_slabs(Plan* plan, const jja_problem_desc& d) {
+  if (!d.lattice_slabs || !d.lattice_rows || plan->parts < 2 || plan->block_size != kSlabBlock) return JJA_OK;
+  SlabHost h;
+  if (!build_slabs(d, plan->parts, kSplitLdsMax, &h)) return JJA_OK;
+  plan->slab_pairs = (h.d.pairs + plan->block_size - 1) / plan->block_size;
+  if (plan->slab_pairs > kSlabPairs) return JJA_OK;
+  const std::vector<double> table = dst_table(d.lattice_cols);
+  int rc;
+  if ((rc = upload(plan, h.pair.data(), h.pair.size(), &h.d.pair))) return rc;
+  if ((rc = upload(plan, h.pair_code.data(), h.pair_code.size(), &h.d.pair_code))) return rc;
+  if ((rc = upload(plan, h.face_code.data(), h.face_code.size(), &h.d.face_code))) return rc;
+  if ((rc = upload(plan, h.face_id.data(), h.face_id.size(), &h.d.face_id))) return rc;
+  if ((rc = upload(plan, h.face_at.data(), h.face_at.size(), &h.d.face_at))) return rc;
+  if ((rc = upload(plan, table.data(), table.size(), &h.d.table))) return rc;
+  if ((rc = upload(plan, h.inv.data(), h.inv.size(), &h.d.inv))) return rc;
+  if ((rc = upload(plan, h.spike.data(), h.spike.size(), &h.d.spike))) return rc;
+  if ((rc = upload(plan, h.reduced.data(), h.reduced.size(), &h.d.reduced))) return rc;
+  const std::vector<double> ends(static_cast<size_t>(d.max_columns) * 4 * plan->parts * d.lattice_cols, 0.0);
+  const std::vector<uint32_t> flags(static_cast<size_t>(d.max_columns) * plan->parts * h.d.mode_waves, 0u);
+  const double* e = nullptr;
+  const uint32_t* f = nullptr;
+  if ((rc = upload(plan, ends.data(), ends.size(), &e))) return rc;
+  if ((rc = upload(plan, flags.data(), flags.size(), &f))) return rc;
+  h.d.ends = const_cast<double*>(e);
+  h.d.flags = const_cast<uint32_t*>(f);
+  plan->slab = h.d;
+  plan->slab_lds = 8 * slab_lds_doubles(h.d, d.lattice_cols);
+  const SlabDev* dev = nullptr;
+  if ((rc = upload(plan, &plan->slab, 1, &dev))) return rc;
+  plan->d_slab = const_cast<SlabDev*>(dev);
   return JJA_OK;
 }
 
@@ -632,47 +674,62 @@ int launch_evolve_sw(Plan* plan, const WorkItem* work, int32_t n, int64_t lds, i
 }
 
 // How a launch can keep every column's state on chip (jja_resident.hip): the
-// junction pairs each thread keeps in registers (1, 2), 0 for the state in LDS,
-// or -1 when some problem or run needs the general kernel. *lds receives the
-// dynamic LDS bytes of the widest column. The resident kernels take the usual
-// step: stencil 3, no voltage sources, noise from Philox with a given
-// amplitude or none.
-int resident_form(const Plan* plan, const jja_problem_run* runs, int64_t* lds) {
-  if (plan->stencil_width != 3 || plan->block_size > 512) return -1;
+// junction pairs each thread keeps in registers, 0 for the state in LDS, or -1 when
+// some problem needs the general kernels. *lds receives the dynamic LDS bytes of
+// the widest column.
+int resident_layout(const Plan* plan, int64_t* lds) {
+  if (plan->stencil_width != 3 || plan->block_size > kResidentBlock) return -1;
   const int32_t BS = plan->block_size;
   int32_t form = 1;
-  for (size_t p = 0; p < plan->problems.size(); ++p) {
-    const DevProblem& d = plan->problems[p];
-    const jja_problem_run& r = runs[p];
-    if (d.index_bytes != 2 || !r.Vs.zero || r.noise || (!r.T.zero && !r.sigma.base)) return -1;
-    const int32_t per = ((d.Nj + 1) / 2 + BS - 1) / BS;
-    const int32_t need = d.n_face_slices <= kResidentFaces * kResidentPairs && per <= kResidentPairs
-                             ? std::max(per, (d.n_face_slices + kResidentFaces - 1) / kResidentFaces)
-                             : 0;
-    if (need == 0 && d.n_face_slices > kResidentRecords) return -1;
-    form = form == 0 || need == 0 ? 0 : std::max(form, need);
+  for (const DevProblem& d : plan->problems) {
+    if (d.index_bytes != 2) return -1;
+    const int32_t need = std::max(((d.Nj + 1) / 2 + BS - 1) / BS, (d.n_face_slices + kResidentFaces - 1) / kResidentFaces);
+    if (need > kResidentPairs && d.n_face_slices > kResidentRecords) return -1;
+    form = form == 0 || need > kResidentPairs ? 0 : std::max(form, need);
   }
   *lds = 8;
   for (const DevProblem& d : plan->problems) {
-    // face vector and scratch, then u (registers) or x, theta_{t-1} and, when
-    // each junction has its own 1/c0, u
-    const int64_t store = d.store_doubles;
+    // the face vector's store, then u (registers) or two phases per junction and,
+    // when each junction has its own 1/c0, u
     const int64_t arrays = form > 0 ? 1 : d.coef_si == 0 ? 2 : 3;
-    *lds = std::max(*lds, 8 * (store + arrays * 2 * ((static_cast<int64_t>(d.Nj) + 1) / 2)));
+    *lds = std::max(*lds, 8 * (d.store_doubles + arrays * 2 * ((static_cast<int64_t>(d.Nj) + 1) / 2)));
   }
   return *lds <= plan->lds_limit ? form : -1;
 }
 
-int launch_resident(Plan* plan, int32_t n, int form, int64_t lds, int32_t n_steps, int64_t step0, hipStream_t stream) {
-  const void* kern = resident_evolve_kernel(plan->block_size, form);
+// The resident kernels take the usual step: stencil 3, no voltage sources, noise
+// from Philox with a given amplitude or none.
+bool resident_runs(const Plan* plan, const jja_problem_run* runs) {
+  for (size_t p = 0; p < plan->problems.size(); ++p)
+    if (!runs[p].Vs.zero || runs[p].noise || (!runs[p].T.zero && !runs[p].sigma.base)) return false;
+  return true;
+}
+
+template <typename... Args>
+int launch_resident(Plan* plan, const void* kern, int32_t n, int64_t lds, hipStream_t stream, Args... args) {
   if (!kern) return fail(JJA_EUNSUPPORTED, "no resident kernel for this workgroup size");
   if (int rc = set_lds_limit(plan, kern, static_cast<int>(lds))) return rc;
+  void* argv[] = {static_cast<void*>(&args)...};
+  JJA_HIP(hipLaunchKernel(kern, dim3(n), dim3(plan->block_size), argv, static_cast<size_t>(lds), stream));
+  return JJA_OK;
+}
+
+int launch_resident_evolve(Plan* plan, int32_t n, int form, int64_t lds, int32_t n_steps, int64_t step0,
+                           hipStream_t stream) {
   const DevProblem* probs = plan->d_problems;
   const jja_problem_run* runs = plan->d_runs;
   const WorkItem* work = plan->d_work;
-  void* argv[] = {&probs, &runs, &work, &n_steps, &step0};
-  JJA_HIP(hipLaunchKernel(kern, dim3(n), dim3(plan->block_size), argv, static_cast<size_t>(lds), stream));
-  return JJA_OK;
+  return launch_resident(plan, resident_evolve_kernel(plan->block_size, form), n, lds, stream, probs, runs, work, n_steps,
+                         step0);
+}
+
+int launch_resident_adjoint(Plan* plan, int32_t n, int form, int64_t lds, int64_t k_hi, int64_t k_lo,
+                            hipStream_t stream) {
+  const DevProblem* probs = plan->d_problems;
+  const jja_adjoint_run* runs = plan->d_adj;
+  const WorkItem* work = plan->d_work;
+  return launch_resident(plan, resident_adjoint_kernel(plan->block_size, form), n, lds, stream, probs, runs, work, k_hi,
+                         k_lo);
 }
 
 template <int STORE>
@@ -762,10 +819,11 @@ int reset_counters(Plan* plan, size_t n, hipStream_t stream) {
 
 // Cooperative launch of a split kernel: all n workgroups resident at once (the
 // column barriers need every part of a column running), or an error. Each
-// workgroup gets the plan's split_lds bytes of dynamic LDS.
+// workgroup gets lds_bytes of dynamic LDS.
 template <typename... Args>
-int launch_cooperative(Plan* plan, const void* kern, int BS, int32_t n, hipStream_t stream, Args... args) {
-  const int lds = static_cast<int>(plan->split_lds);
+int launch_cooperative(Plan* plan, const void* kern, int BS, int32_t n, int64_t lds_bytes, hipStream_t stream,
+                       Args... args) {
+  const int lds = static_cast<int>(lds_bytes);
   int per_cu = -1;
   for (const auto& a : plan->per_cu)
     if (a.first == kern) per_cu = a.second;
@@ -790,7 +848,7 @@ int launch_evolve_split_bs(Plan* plan, int32_t n, int32_t n_steps, int64_t step0
   const WorkItem* work = plan->d_work;
   const void* kern = plan->pairs ? reinterpret_cast<const void*>(evolve_split_kernel<BS, 3, BS <= 512>)
                                  : reinterpret_cast<const void*>(evolve_split_kernel<BS, 3, false>);
-  return launch_cooperative(plan, kern, BS, n, stream, probs, runs, work, n_steps, step0, plan->d_ctrs,
+  return launch_cooperative(plan, kern, BS, n, plan->split_lds, stream, probs, runs, work, n_steps, step0, plan->d_ctrs,
                             plan->d_err, plan->wait_limit);
 }
 
@@ -804,6 +862,37 @@ int launch_evolve_split(Plan* plan, int32_t n, int32_t n_steps, int64_t step0, h
   }
 }
 
+// Whether a run can go to the slab kernels: the usual step (stencil 3, no voltage
+// sources, noise from Philox with a given amplitude or none).
+bool slab_run(const Plan* plan, const jja_problem_run& r) {
+  return plan->d_slab && plan->stencil_width == 3 && r.Vs.zero && !r.noise && (r.T.zero || r.sigma.base);
+}
+
+int launch_evolve_slab(Plan* plan, int32_t n, int32_t n_steps, int64_t step0, hipStream_t stream) {
+  const DevProblem* probs = plan->d_problems;
+  const jja_problem_run* runs = plan->d_runs;
+  const WorkItem* work = plan->d_work;
+  const SlabDev* slabs = plan->d_slab;
+  const uint32_t seq = plan->slab_seq;
+  const int rc = launch_cooperative(plan, slab_evolve_kernel(plan->slab_pairs), plan->block_size, n,
+                                    plan->slab_lds, stream, probs, runs, work, slabs, n_steps, step0, seq, plan->d_err,
+                                    plan->wait_limit);
+  if (rc == JJA_OK) plan->slab_seq += static_cast<uint32_t>(n_steps);
+  return rc;
+}
+
+int launch_adjoint_slab(Plan* plan, int32_t n, int64_t k_hi, int64_t k_lo, hipStream_t stream) {
+  const DevProblem* probs = plan->d_problems;
+  const jja_adjoint_run* runs = plan->d_adj;
+  const WorkItem* work = plan->d_work;
+  const SlabDev* slabs = plan->d_slab;
+  const uint32_t seq = plan->slab_seq;
+  const int rc = launch_cooperative(plan, slab_adjoint_kernel(plan->slab_pairs), plan->block_size, n, plan->slab_lds,
+                                    stream, probs, runs, work, slabs, k_hi, k_lo, seq, plan->d_err, plan->wait_limit);
+  if (rc == JJA_OK) plan->slab_seq += static_cast<uint32_t>(k_hi - k_lo + 1);
+  return rc;
+}
+
 template <int BS>
 int launch_adjoint_split_bs(Plan* plan, int32_t n, int64_t k_hi, int64_t k_lo, hipStream_t stream) {
   const DevProblem* probs = plan->d_problems;
@@ -811,7 +900,7 @@ int launch_adjoint_split_bs(Plan* plan, int32_t n, int64_t k_hi, int64_t k_lo, h
   const WorkItem* work = plan->d_work;
   const void* kern = plan->pairs ? reinterpret_cast<const void*>(adjoint_split_kernel<BS, BS <= 512>)
                                  : reinterpret_cast<const void*>(adjoint_split_kernel<BS, false>);
-  return launch_cooperative(plan, kern, BS, n, stream, probs, runs, work, k_hi, k_lo, plan->d_ctrs,
+  return launch_cooperative(plan, kern, BS, n, plan->split_lds, stream, probs, runs, work, k_hi, k_lo, plan->d_ctrs,
                             plan->d_err, plan->wait_limit);
 }
 
@@ -959,8 +1048,8 @@ int jja_plan_create(int32_t n_problems, const jja_problem_desc* descs, jja_plan*
         if ((rc = upload(plan, split.data(), n, &dp.lat_sine_p))) break;
       }
       if ((rc = upload(plan, d.lattice_inv, static_cast<size_t>(R) * dp.lat_cp, &dp.lat_inv))) break;
-      // padded LDS form: the table steps and their mirrors stay inside sides of 8
-      // a side; rows of 32 k + 4 doubles put the 16 rows of a tile on all banks
+      // padded LDS form: the table's steps and their mirrors stay inside a side of
+      // 8 elements or more; rows of 32 k + 4 doubles put the 16 rows of a tile on all banks
       const DstShape dc(C), dr(R);
       const int32_t ld = dc.padded() + 4;
       const int64_t buf = static_cast<int64_t>(dr.padded()) * ld;
@@ -1089,6 +1178,7 @@ int jja_plan_create(int32_t n_problems, const jja_problem_desc* descs, jja_plan*
     alloc(2 * sizeof(uint32_t) * items, reinterpret_cast<void**>(&plan->d_ctrs));
     plan->ctr_cap = 2 * items;
   }
+  if (rc == JJA_OK && n_problems == 1) rc = create_slabs(plan, descs[0]);
   if (rc == JJA_OK && hipEventCreateWithFlags(&plan->done, hipEventDisableTiming) != hipSuccess)
     rc = fail(JJA_EHIP, "jja_plan_create: hipEventCreateWithFlags failed");
   if (rc == JJA_OK && plan->parts > 1) {
@@ -1197,9 +1287,14 @@ int jja_evolve(jja_plan* p, const jja_problem_run* runs, int32_t n_steps, int64_
     // circuit without faces has none and needs none): all columns, one launch
     work.insert(work.end(), work_g.begin(), work_g.end());
     const std::vector<WorkItem> split = split_work(plan, work);
-    if ((rc = reset_counters(plan, work.size(), stream))) return rc;
     if ((rc = upload_work(plan, split, stream))) return rc;
-    rc = launch_evolve_split(plan, static_cast<int32_t>(split.size()), n_steps, step0, stream);
+    const bool slab = slab_run(plan, runs[0]);
+    if (slab)
+      rc = launch_evolve_slab(plan, static_cast<int32_t>(split.size()), n_steps, step0, stream);
+    else if ((rc = reset_counters(plan, work.size(), stream)))
+      return rc;
+    else
+      rc = launch_evolve_split(plan, static_cast<int32_t>(split.size()), n_steps, step0, stream);
   } else {
     // one launch: a kernel for one kind of face store, or one that takes either
     const int32_t n_lds = static_cast<int32_t>(work.size()), n_g = static_cast<int32_t>(work_g.size());
@@ -1209,9 +1304,9 @@ int jja_evolve(jja_plan* p, const jja_problem_run* runs, int32_t n_steps, int64_
     if (lds < 8) lds = 8;
     const int32_t n = n_lds + n_g;
     int64_t resident_lds = 0;
-    const int form = n_g == 0 ? resident_form(plan, runs, &resident_lds) : -1;
+    const int form = n_g == 0 && resident_runs(plan, runs) ? resident_layout(plan, &resident_lds) : -1;
     if (form >= 0)
-      rc = launch_resident(plan, n, form, resident_lds, n_steps, step0, stream);
+      rc = launch_resident_evolve(plan, n, form, resident_lds, n_steps, step0, stream);
     else if (n_g == 0)
       rc = launch_evolve_bs<0>(plan, plan->d_work, n, lds, n_steps, step0, stream);
     else if (n_lds == 0)
@@ -1257,9 +1352,13 @@ int jja_adjoint(jja_plan* p, const jja_adjoint_run* runs, int64_t k_hi, int64_t 
   if (plan->parts > 1) {
     work.insert(work.end(), work_g.begin(), work_g.end());
     const std::vector<WorkItem> split = split_work(plan, work);
-    if ((rc = reset_counters(plan, work.size(), stream))) return rc;
     if ((rc = upload_work(plan, split, stream))) return rc;
-    rc = launch_adjoint_split(plan, static_cast<int32_t>(split.size()), k_hi, k_lo, stream);
+    if (plan->d_slab)
+      rc = launch_adjoint_slab(plan, static_cast<int32_t>(split.size()), k_hi, k_lo, stream);
+    else if ((rc = reset_counters(plan, work.size(), stream)))
+      return rc;
+    else
+      rc = launch_adjoint_split(plan, static_cast<int32_t>(split.size()), k_hi, k_lo, stream);
   } else {
     const int32_t n_lds = static_cast<int32_t>(work.size()), n_g = static_cast<int32_t>(work_g.size());
     order_work(plan, work);
@@ -1267,7 +1366,12 @@ int jja_adjoint(jja_plan* p, const jja_adjoint_run* runs, int64_t k_hi, int64_t 
     work.insert(work.end(), work_g.begin(), work_g.end());
     if ((rc = upload_work(plan, work, stream))) return rc;
     if (lds < 8) lds = 8;
-    if (n_lds) rc = launch_adjoint_bs<false>(plan, plan->d_work, n_lds, lds, k_hi, k_lo, stream);
+    int64_t resident_lds = 0;
+    const int form = n_lds && !n_g ? resident_layout(plan, &resident_lds) : -1;
+    if (form >= 0)
+      rc = launch_resident_adjoint(plan, n_lds, form, resident_lds, k_hi, k_lo, stream);
+    else if (n_lds)
+      rc = launch_adjoint_bs<false>(plan, plan->d_work, n_lds, lds, k_hi, k_lo, stream);
     if (!rc && n_g) rc = launch_adjoint_bs<true>(plan, plan->d_work + n_lds, n_g, 8, k_hi, k_lo, stream);
   }
   if (rc) return rc;

@@ -15,16 +15,6 @@
 
 namespace {
 
-// +-v by the sign bit of an incidence code; 0 for an empty slot
-__device__ __forceinline__ double signed_value(double v, uint32_t code) {
-  const long long b = __builtin_bit_cast(long long, v) ^ (static_cast<long long>(code & 1u) << 63);
-  return code == 0xffffu ? 0.0 : __builtin_bit_cast(double, b);
-}
-__device__ __forceinline__ uint32_t code_address(uint32_t code) { return code == 0xffffu ? 0u : code >> 1; }
-__device__ __forceinline__ uint32_t pack_codes(int32_t a, int32_t b) {
-  return static_cast<uint32_t>(a & 0xffff) | (static_cast<uint32_t>(b & 0xffff) << 16);
-}
-
 // NP > 0: every thread keeps NP junction pairs in registers. NP 0: phases and
 // right-hand sides lie in LDS and the threads loop over the pairs.
 template <int BS, int NP>
@@ -36,11 +26,11 @@ __global__ __launch_bounds__(BS) void evolve_resident_kernel(const DevProblem* _
   constexpr bool REG = NP > 0;
   constexpr int N = REG ? NP : 1;
   constexpr int NF = REG ? kResidentFaces * NP : kResidentRecords;
-  const WorkItem wi = work[blockIdx.x];
-  const DevProblem& P = probs[wi.problem];
-  const jja_problem_run& R = runs[wi.problem];
-  const int64_t w = wi.column;
-  const int tid = threadIdx.x;
+  const int32_t problem = __builtin_amdgcn_readfirstlane(work[blockIdx.x].problem);
+  const int64_t w = __builtin_amdgcn_readfirstlane(work[blockIdx.x].column);
+  const DevProblem& P = probs[problem];
+  const jja_problem_run& R = runs[problem];
+  const int32_t tid0 = threadIdx.x, tid = tid0;
   const int32_t Nj = P.Nj, Nf = P.Nf, pairs = (Nj + 1) >> 1;
   FaceStore<false> zs;
   zs.p = lds;
@@ -154,6 +144,11 @@ __global__ __launch_bounds__(BS) void evolve_resident_kernel(const DevProblem* _
   }
   for (int32_t n = 0; n < n_steps; ++n) {
     const int64_t t = step0 + n;
+    const int32_t again = problem + opaque_zero();
+    const DevProblem& P = probs[again];
+    const jja_problem_run& R = runs[again];
+    const int32_t tid = opaque(tid0);
+    zs.vt = tid;
     if (Nf > 0) {
       const TermView fv = term_view(R.f, !R.f.zero, P.zero, w, t);
       double fq[NF];
@@ -260,12 +255,228 @@ __global__ __launch_bounds__(BS) void evolve_resident_kernel(const DevProblem* _
   }
 }
 
+// The adjoint sweep (adjoint_steps) of a column. NP > 0: lambda_k, the partial sum
+// of lambda_{k-1}, both gradients and the phases of two steps stay in registers for
+// the whole launch; NP 0: both lambdas lie in LDS.
+template <int BS, int NP>
+__global__ __launch_bounds__(BS) void adjoint_resident_kernel(const DevProblem* __restrict__ probs,
+                                                              const jja_adjoint_run* __restrict__ runs,
+                                                              const WorkItem* __restrict__ work, int64_t k_hi,
+                                                              int64_t k_lo) {
+  extern __shared__ double lds[];
+  constexpr bool REG = NP > 0;
+  constexpr int N = REG ? NP : 1;
+  constexpr int NF = REG ? kResidentFaces * NP : kResidentRecords;
+  const int32_t problem = __builtin_amdgcn_readfirstlane(work[blockIdx.x].problem);
+  const int64_t w = __builtin_amdgcn_readfirstlane(work[blockIdx.x].column);
+  const DevProblem& P = probs[problem];
+  const jja_adjoint_run& A = runs[problem];
+  const int32_t tid0 = threadIdx.x, tid = tid0;
+  const int32_t Nj = P.Nj, Nf = P.Nf, pairs = (Nj + 1) >> 1;
+  FaceStore<false> zs;
+  zs.p = lds;
+  zs.vt = tid;
+  zs.vbs = BS;
+  init_store(P, lds, tid, BS);
+  const bool uni = P.coef_si == 0;
+  LAS double* const X = (LAS double*)lds + P.store_doubles;   // lambda_k, then the partial sum
+  LAS double* const B = X + 2 * pairs;
+  LAS double* const U = REG || uni ? X : B + 2 * pairs;
+  const AdjCol C = adjoint_column(P, A, w);
+  GAS double* const gIc = gblw(A.grad_Ic) + static_cast<size_t>(w) * Nj;
+  GAS double* const gIs = gblw(A.grad_Is) + static_cast<size_t>(w) * Nj;
+  GAS double* const gf = gblw(A.grad_f) + static_cast<size_t>(w) * Nf;
+  double rc0 = 0.0, c1 = 0.0, c2 = 0.0;
+  if (uni) {
+    rc0 = rc0_at(P, 0);
+    c1 = coef_at(P, 1, 0);
+    c2 = coef_at(P, 2, 0);
+  }
+  auto history = [&](int64_t m, int32_t j) { return C.hist[static_cast<size_t>(m - C.hist_m0) * C.stride + j]; };
+  const GAS double* const lam_k = C.lam + (k_hi & 1) * C.stride;
+  const GAS double* const lam_p = C.lam + ((k_hi - 1) & 1) * C.stride;
+  double la[N][2], lb[N][2], ic[N][2], ai[N][2], as[N][2], h1[N][2], h2[N][2];
+  uint32_t jc[N][2];
+  auto begin = [&](int k, int32_t q) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      const int32_t j = 2 * q + m;
+      if (j >= Nj) break;
+      double l = lam_k[j];
+      if (A.prime) l = l + adj_g(A, C, k_hi, j);
+      const double u = l * (uni ? rc0 : rc0_at(P, j));
+      if constexpr (REG) {
+        const vint2 c = gbl(reinterpret_cast<const vint2*>(P.junc_code))[j];
+        jc[k][m] = pack_codes(c.x, c.y);
+        la[k][m] = l;
+        lb[k][m] = lam_p[j];
+        ic[k][m] = C.Ic[j];
+        ai[k][m] = gIc[j];
+        as[k][m] = gIs[j];
+        h1[k][m] = history(k_hi - 1, j);
+        h2[k][m] = history(k_hi - 2, j);
+        U[j] = u;
+      } else {
+        X[j] = l;
+        B[j] = lam_p[j];
+        if (!uni) U[j] = u;
+      }
+    }
+  };
+  if constexpr (REG) {
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      if (k * BS + tid < pairs) begin(k, k * BS + tid);
+  } else {
+    for (int32_t q = tid; q < pairs; q += BS) begin(0, q);
+  }
+  uint32_t fc[NF][2], fpos[NF], finish = 0;
+  const int32_t nrec = P.n_face_slices;
+#pragma unroll
+  for (int k = 0; k < NF; ++k) {
+    FaceRec r{{-1, -1, -1, -1}, -1, -1, false};
+    if (k < nrec) face_rec_load(P, k, true, tid, BS, r);
+    fc[k][0] = pack_codes(r.cd[0], r.cd[1]);
+    fc[k][1] = pack_codes(r.cd[2], r.cd[3]);
+    fpos[k] = r.pos < 0 ? 0xffffffffu : static_cast<uint32_t>(r.pos);
+    finish |= r.finish ? 1u << k : 0u;
+  }
+  for (int64_t t = k_hi; t >= k_lo; --t) {
+    const int32_t again = problem + opaque_zero();
+    const DevProblem& P = probs[again];
+    const jja_adjoint_run& A = runs[again];
+    const int32_t tid = opaque(tid0);
+    zs.vt = tid;
+    if (Nf > 0) {
+      lds_barrier();
+      double acc = 0.0;
+#pragma unroll
+      for (int k = 0; k < NF; ++k) {
+        if (k >= nrec) break;
+        double uv[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) uv[i] = U[code_address((fc[k][i >> 1] >> (16 * (i & 1))) & 0xffffu)];
+        if (!REG && uni) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) uv[i] = uv[i] * rc0;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc = acc + signed_value(uv[i], (fc[k][i >> 1] >> (16 * (i & 1))) & 0xffffu);
+        if (finish >> k & 1u) {
+          if (fpos[k] != 0xffffffffu) {
+            const int32_t pos = static_cast<int32_t>(fpos[k]);
+            zs.wr(pos, acc);
+            if (pos < P.copy_rows) zs.wr(Nf + pos, acc);
+          }
+          acc = 0.0;
+        }
+      }
+      lds_barrier();
+      solve_face_system(P, zs);
+      for (int32_t p = tid; p < Nf; p += BS) gf[p] = gf[p] - kTwoPi * zs.rd(store_address(P, p));
+    }
+    auto sweep = [&](int k, int32_t q) {
+      double t1[2], t2[2], nh[2] = {0.0, 0.0}, icj[2], gi[2], gs[2], lk[2], lp[2];
+      uint32_t code[2];
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        const int32_t j = min(2 * q + m, Nj - 1);
+        if constexpr (REG) {
+          code[m] = jc[k][m];
+          t1[m] = h1[k][m];
+          t2[m] = h2[k][m];
+          icj[m] = ic[k][m];
+          gi[m] = ai[k][m];
+          gs[m] = as[k][m];
+          lk[m] = la[k][m];
+          lp[m] = lb[k][m];
+          if (t > k_lo) nh[m] = history(t - 3, j);
+        } else {
+          const vint2 c = gbl(reinterpret_cast<const vint2*>(P.junc_code))[j];
+          code[m] = pack_codes(c.x, c.y);
+          t1[m] = history(t - 1, j);
+          t2[m] = history(t - 2, j);
+          icj[m] = C.Ic[j];
+          gi[m] = gIc[j];
+          gs[m] = gIs[j];
+          lk[m] = X[j];
+          lp[m] = B[j];
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        const int32_t j = 2 * q + m;
+        if (j >= Nj) break;
+        double r0 = rc0, k1 = c1, k2 = c2;
+        if (!uni) {
+          r0 = rc0_at(P, j);
+          k1 = coef_at(P, 1, j);
+          k2 = coef_at(P, 2, j);
+        }
+        const double gj = adj_g(A, C, t - 1, j);
+        const uint32_t ca = code[m] & 0xffffu, cb = code[m] >> 16;
+        const double za = zs.gather(code_address(ca)), zb = zs.gather(code_address(cb));
+        const double y = signed_value(za, ca) + signed_value(zb, cb);
+        const double mu = (y - lk[m]) * r0;
+        double sn, cs;
+        jja_sincos(2.0 * t1[m] - t2[m], &sn, &cs);
+        const double av = 2.0 * icj[m] * cs + k1, bv = k2 - icj[m] * cs;
+        const double gn = gi[m] + sn * mu, sm = gs[m] - mu, part = bv * mu;
+        const double l1 = (lp[m] + av * mu) + gj;
+        if constexpr (REG) {
+          la[k][m] = l1;
+          lb[k][m] = part;
+          ai[k][m] = gn;
+          as[k][m] = sm;
+          h1[k][m] = t2[m];
+          h2[k][m] = nh[m];
+          U[j] = l1 * r0;
+        } else {
+          X[j] = l1;
+          B[j] = part;
+          if (!uni) U[j] = l1 * r0;
+        }
+        if (!REG || t == k_lo) {
+          gIc[j] = gn;
+          gIs[j] = sm;
+        }
+        if (t == k_lo) {
+          // lambda_{k_lo - 1} complete, the partial sum of lambda_{k_lo - 2}
+          (C.lam + ((k_lo - 1) & 1) * C.stride)[j] = l1;
+          (C.lam + (k_lo & 1) * C.stride)[j] = part;
+          C.u[j] = l1 * r0;
+        }
+      }
+    };
+    if constexpr (REG) {
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        if (k * BS + tid < pairs) sweep(k, k * BS + tid);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      for (int32_t q = tid; q < pairs; q += BS) sweep(0, q);
+    }
+  }
+}
+
 template <int BS>
-const void* kernel_of(int pairs) {
+const void* evolve_of(int pairs) {
   switch (pairs) {
     case 1: return reinterpret_cast<const void*>(evolve_resident_kernel<BS, 1>);
     case 2: return reinterpret_cast<const void*>(evolve_resident_kernel<BS, 2>);
+    case 3: return reinterpret_cast<const void*>(evolve_resident_kernel<BS, 3>);
     default: return reinterpret_cast<const void*>(evolve_resident_kernel<BS, 0>);
+  }
+}
+
+template <int BS>
+const void* adjoint_of(int pairs) {
+  switch (pairs) {
+    case 1: return reinterpret_cast<const void*>(adjoint_resident_kernel<BS, 1>);
+    case 2: return reinterpret_cast<const void*>(adjoint_resident_kernel<BS, 2>);
+    case 3: return reinterpret_cast<const void*>(adjoint_resident_kernel<BS, 3>);
+    default: return reinterpret_cast<const void*>(adjoint_resident_kernel<BS, 0>);
   }
 }
 
@@ -273,11 +484,20 @@ const void* kernel_of(int pairs) {
 
 const void* resident_evolve_kernel(int block_size, int pairs) {
   switch (block_size) {
-    case 64: return kernel_of<64>(pairs);
-    case 128: return kernel_of<128>(pairs);
-    case 256: return kernel_of<256>(pairs);
-    case 512: return kernel_of<512>(pairs);
-    case 1024: return pairs ? nullptr : kernel_of<1024>(0);
+    case 64: return evolve_of<64>(pairs);
+    case 128: return evolve_of<128>(pairs);
+    case 256: return evolve_of<256>(pairs);
+    case 512: return evolve_of<512>(pairs);
+    default: return nullptr;
+  }
+}
+
+const void* resident_adjoint_kernel(int block_size, int pairs) {
+  switch (block_size) {
+    case 64: return adjoint_of<64>(pairs);
+    case 128: return adjoint_of<128>(pairs);
+    case 256: return adjoint_of<256>(pairs);
+    case 512: return adjoint_of<512>(pairs);
     default: return nullptr;
   }
 }

@@ -155,6 +155,42 @@ def auto_parts(host, columns, stencil_width, max_parts=16, junctions_per_part=24
     return parts
 
 
+# a slab (jja_slab.hip) holds at most this many junctions and at least these rows
+SLAB_BLOCK = 512
+SLAB_JUNCTIONS = 9 * 2 * SLAB_BLOCK
+SLAB_MIN_ROWS = 4
+SLAB_MIN_JUNCTIONS = 3000
+
+
+def slab_parts(host, columns, n_cu, max_parts=16):
+    """Row slabs per column of a lattice plan: the most whose workgroups, one per
+    compute unit, all fit on the device, or 1 when that leaves slabs too large."""
+    if not host.uses_lattice or not 8 <= host.lattice.C <= SLAB_BLOCK // 2 or host.Nj < SLAB_MIN_JUNCTIONS:
+        return 1
+    lat, parts = host.lattice, 1
+    while parts < max_parts and 2 * parts * columns <= n_cu and lat.R >= 2 * parts * SLAB_MIN_ROWS:
+        parts *= 2
+    rows = -(-lat.R // parts)
+    if parts == 1 or (2 * rows + 1) * (lat.C + 1) > SLAB_JUNCTIONS:
+        return 1
+    # two slabs pay only where one workgroup cannot hold the column's state
+    return 1 if parts == 2 and host.Nj <= RESIDENT_JUNCTIONS else parts
+
+
+def takes_slabs(problem):
+    """Whether a problem leaves its layout open and its runs are ones the slab
+    kernels take (the usual step: stencil 3, no voltage sources, noise from Philox
+    at a constant temperature or none)."""
+    def open_to(name, default):
+        return getattr(problem, name, default) in (None, default)
+    T, Vs = problem.temperature, problem.voltage_sources
+    return (problem.stencil_width == 3 and problem.block_size is None and open_to("face_store", "auto")
+            and getattr(problem, "parts", None) is None and not getattr(problem, "column_pairs", False)
+            and not callable(T) and not callable(Vs) and not problem._T_is_timedep and not problem._Vs_is_timedep
+            and (problem.noise == "philox" or bool(np.allclose(T[:, :, 0], 0)))
+            and bool(np.allclose(Vs[:, :, 0], 0)))
+
+
 class Engine:
     """Device state and launches of one problem. With ``shared = (handle, index,
     host)`` the problem is problem ``index`` of a plan that a BatchEngine owns."""
@@ -181,7 +217,12 @@ class Engine:
                                     local_stages=getattr(problem, "local_stages", "auto"),
                                     solver=getattr(problem, "solver", "auto"))
             parts = getattr(problem, "parts", None)
-            if parts is None:
+            slabs = slab_parts(self.host, W, device_compute_units()) if takes_slabs(problem) else 1
+            if slabs > 1:
+                self.block_size = SLAB_BLOCK
+                self.host = self.host.relayout(SLAB_BLOCK, slabs, slabs=True)
+                parts = 1
+            elif parts is None:
                 parts = auto_parts(self.host, W, sw)
             if parts > 1:
                 self.host = self.host.relayout(self.block_size, parts)

@@ -375,6 +375,7 @@ class CircuitPlan:
         self.local_option = local_stages
         self.solver = solver
         self.column_pairs = False
+        self.slabs = False
         if stencil_width not in STENCILS:
             raise ValueError(f"stencil width must be 3, 4 or 5 (equals {stencil_width})")
         self.Nj, self.Nf = circuit._Nj(), circuit._Nf()
@@ -403,13 +404,15 @@ class CircuitPlan:
         self.target_iter = target_iter
         self._build_layouts(target_iter)
 
-    def relayout(self, block_size, parts=None, face_store=None, local_stages=None, solver=None):
+    def relayout(self, block_size, parts=None, face_store=None, local_stages=None, solver=None, slabs=False):
         """The same circuit, factor and schedule laid out for another workgroup
         size, part count, face store, wave-local stage count or solver (the
-        factorisation depends on none of them)."""
+        factorisation depends on none of them). ``slabs``: a split lattice column
+        may run as row slabs."""
         other = copy.copy(self)
         other.block_size = block_size
         other.column_pairs = False
+        other.slabs = slabs
         if solver is not None:
             if solver not in SOLVERS:
                 raise ValueError("solver must be 'auto', 'lattice' or 'cholesky'")
@@ -1093,6 +1096,7 @@ class CircuitPlan:
         d.index_bytes = self.index_bytes
         if self.uses_lattice:
             self.lattice.set_desc(d)
+            d.lattice_slabs = int(self.slabs)
         return d
 
     def lds_bytes(self):
