@@ -135,6 +135,47 @@ typedef struct jja_slice {
   int32_t flags;   /* G | JJA_SLICE_* | rows << 16 */
 } jja_slice;
 
+/*
+ * Subdomains of a circuit's face system (HOST arrays, copied by plan creation): a
+ * column of `parts` workgroups of 512 threads that exchange values of separator
+ * faces once a step (pyjjasim_amd/domain_plan.py derives the scheme and builds the
+ * arrays). Part p holds `pairs` slots of junction pairs and `faces` slots of faces;
+ * its LDS holds, in doubles, the face sums (0 ..), the solution (faces ..), and the
+ * separator faces' right-hand sides (2 faces ..).
+ *   pair[parts][pairs]            q * 16 + m + 4 m for the junctions 2q (m bit 0) and
+ *                                 2q + 1 (m bit 1) the part holds, or -1
+ *   pair_code[parts][pairs][2][2] 2 * face slot + sign of each member's faces, or 0xffff
+ *   face_code[parts][faces][8]    2 * (2 * pair slot + member) + sign, or 0xffff
+ *   face_id[parts][faces]         the face (circuit order) whose flux and gradient the
+ *                                 part adds, or -1
+ *   face_used[parts][faces]       1 where the slot holds a face
+ *   pub_ptr[parts + 1], pub_at[n_published]  face slots a part publishes
+ *   source[n_gamma][sources]      published values of a separator face, or -1
+ *   records: as the solve records of a problem with 2-byte indices, two programs a
+ *   part (before and after the exchange) for the 8 waves of a workgroup, program
+ *   2p + i's wave w at wave_ptr[(2p + i) * 9 + w]; rows and indices are addresses in
+ *   the part's LDS, r0 is 0 and an off-block record subtracts its sum from its row.
+ */
+typedef struct jja_domains {
+  int32_t parts, pairs, faces, n_gamma, sources, n_published, n_records, pad_;
+  const int32_t* pair;
+  const uint16_t* pair_code;
+  const uint16_t* face_code;
+  const int32_t* face_id;
+  const int32_t* face_used;
+  const int32_t* pub_ptr;
+  const int32_t* pub_at;
+  const int32_t* source;
+  const jja_slice* records;
+  const int32_t* wave_ptr;
+  int64_t n_slice_rows;
+  const int32_t* slice_rows;
+  int64_t n_entries;
+  const double* ent_val;
+  int64_t n_index;
+  const uint16_t* ent_off;
+} jja_domains;
+
 typedef struct jja_problem_desc {
   int32_t n_junctions;
   int32_t n_faces;
@@ -224,6 +265,13 @@ typedef struct jja_problem_desc {
   const double* lattice_inv;
   double lattice_g;            /* g */
   double lattice_gc;           /* g_c */
+  /* NULL, or the subdomains that solve the face system of a plan of this problem
+   * alone (parts >= 2 equal to theirs, block_size 512 * parts, index_bytes 4,
+   * lattice_rows 0, solve positions in circuit order). There are then no solve
+   * records, and only runs of the usual step are taken (no voltage sources, no
+   * given normals, noise amplitude given; JJA_EUNSUPPORTED otherwise); jja_solve
+   * refuses the plan. */
+  const struct jja_domains* domains;
 } jja_problem_desc;
 
 /*

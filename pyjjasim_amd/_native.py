@@ -55,7 +55,17 @@ class ProblemDesc(C.Structure):
         ("cpr_terms", C.c_int32), ("lattice_slabs", C.c_int32), ("cpr_coef", C.c_double * 8),
         ("lattice_rows", C.c_int32), ("lattice_cols", C.c_int32),
         ("lattice_sine", f64p), ("lattice_inv", f64p), ("lattice_g", C.c_double), ("lattice_gc", C.c_double),
+        ("domains", C.c_void_p),
     ]
+
+
+class Domains(C.Structure):
+    _fields_ = [(n, C.c_int32) for n in ("parts", "pairs", "faces", "n_gamma", "sources", "n_published",
+                                         "n_records", "pad_")] + \
+        [(n, C.c_void_p) for n in ("pair", "pair_code", "face_code", "face_id", "face_used", "pub_ptr", "pub_at",
+                                   "source", "records", "wave_ptr")] + \
+        [("n_slice_rows", C.c_int64), ("slice_rows", C.c_void_p), ("n_entries", C.c_int64),
+         ("ent_val", C.c_void_p), ("n_index", C.c_int64), ("ent_off", C.c_void_p)]
 
 
 class Source(C.Structure):

@@ -432,12 +432,13 @@ __device__ __forceinline__ uint32_t record_index(const SliceRegs<GLOBAL>& r, int
 // or past the record's iteration count is read at an offset beyond the
 // resource's range, which returns zeros without a memory access, so a short
 // record moves only the bytes it uses and every record issues the same loads.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t value_resource(const DevProblem& P) {
+template <class D>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t value_resource(const D& P) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(P.ent_val), 0, P.val_bytes, kBufferWord3);
 }
 
-template <bool GLOBAL>
-__device__ __forceinline__ void load_slice(const DevProblem& P, __amdgpu_buffer_rsrc_t vres,
+template <bool GLOBAL, class D>
+__device__ __forceinline__ void load_slice(const D& P, __amdgpu_buffer_rsrc_t vres,
                                            const jja_slice& m, int lane, SliceRegs<GLOBAL>& r) {
   const int lg = __builtin_ctz(static_cast<unsigned>(m.flags & 0xff));
   const uint32_t voff = static_cast<uint32_t>(m.base) * 8u + static_cast<uint32_t>(lane) * 16u;
@@ -521,9 +522,33 @@ __device__ __forceinline__ void process_slice(const Z& zs, int32_t Nf, int lane,
 // and descriptors are read ahead. A wave's executed record count is a multiple
 // of three and four never-executed records follow it, so the loop has a single
 // exit and every lookahead load stays inside the program. Waves meet only at
-// BARRIER records (one per phase, the same number in every wave).
-template <class Z>
-__device__ __forceinline__ void solve(const DevProblem& P, const Z& zs) {
+// BARRIER records (one per phase, the same number in every wave). D: a problem, or
+// anything with its program's arrays.
+// solve_head issues the loads of a program's first two records, which a caller may do
+// early (before a barrier or a wait) to hide their latency.
+template <bool GLOBAL>
+struct SolveHead {
+  SliceRegs<GLOBAL> A, B;
+};
+
+template <class D>
+__device__ __forceinline__ int32_t program_start(const D& P, int32_t vt) {
+  const CAS int32_t* wp = (const CAS int32_t*)(P.wave_ptr) + __builtin_amdgcn_readfirstlane(vt / kWave);
+  return __builtin_amdgcn_readfirstlane(wp[0]);
+}
+
+template <class D, bool GLOBAL>
+__device__ __forceinline__ void solve_head(const D& P, int32_t vt, SolveHead<GLOBAL>& h) {
+  const int lane = vt & (kWave - 1);
+  const jja_slice* __restrict__ prog = P.solve_slices + program_start(P, vt);
+  const __amdgpu_buffer_rsrc_t vres = value_resource(P);
+  load_slice(P, vres, load_rec(prog, 0), lane, h.A);
+  load_slice(P, vres, load_rec(prog, 1), lane, h.B);
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+template <class D, class Z>
+__device__ __forceinline__ void solve_tail(const D& P, const Z& zs, SolveHead<Z::kGlobal>& h) {
   constexpr bool GLOBAL = Z::kGlobal;
   const int lane = zs.vt & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(zs.vt / kWave);
@@ -533,9 +558,8 @@ __device__ __forceinline__ void solve(const DevProblem& P, const Z& zs) {
   const jja_slice* __restrict__ prog = P.solve_slices + k0;
   jja_slice m0 = load_rec(prog, 0), m1 = load_rec(prog, 1), m2 = load_rec(prog, 2);
   const __amdgpu_buffer_rsrc_t vres = value_resource(P);
-  SliceRegs<GLOBAL> A, B, C;
-  load_slice(P, vres, m0, lane, A);
-  load_slice(P, vres, m1, lane, B);
+  SliceRegs<GLOBAL>&A = h.A, &B = h.B;
+  SliceRegs<GLOBAL> C;
   double acc = 0.0;
   for (int32_t k = 0; k < nk; k += 3) {
     const jja_slice m3 = load_rec(prog, k + 3);
@@ -554,6 +578,13 @@ __device__ __forceinline__ void solve(const DevProblem& P, const Z& zs) {
     m1 = m4;
     m2 = m5;
   }
+}
+
+template <class D, class Z>
+__device__ __forceinline__ void solve(const D& P, const Z& zs) {
+  SolveHead<Z::kGlobal> h;
+  solve_head(P, zs.vt, h);
+  solve_tail(P, zs, h);
 }
 
 // ------------------------------------------------------------ lattice solve

@@ -37,6 +37,7 @@
 
 #include "../../include/jja.h"
 #include "jja_device.h"
+#include "jja_domain.h"
 #include "jja_resident.h"
 #include "jja_slab.h"
 
@@ -256,13 +257,15 @@ struct Plan {
                                      // [1] workgroups whose column ran on one XCD
   int32_t n_cu = 0;                  // compute units of the device
   uint32_t wait_limit = kWaitLimit;  // split launches: polls before a column barrier gives up
-  // a lattice column as row slabs (one problem): the device descriptor, dynamic LDS
-  // doubles, pairs a thread holds and the sequence number of the last step
-  SlabDev slab{};
-  SlabDev* d_slab = nullptr;
-  int64_t slab_lds = 0;
-  int32_t slab_pairs = 0;
-  uint32_t slab_seq = 0;
+  // columns in parts that keep their junctions on chip (one problem; row slabs or
+  // subdomains): the device tables and kernels, dynamic LDS doubles and the
+  // sequence number of the last step
+  const void* d_parts = nullptr;
+  const void* parts_evolve = nullptr;
+  const void* parts_adjoint = nullptr;
+  int64_t parts_lds = 0;
+  bool parts_only = false;           // subdomains: there is no other way to solve
+  uint32_t parts_seq = 0;
   int64_t split_lds = 0;             // split launches: dynamic LDS bytes (part-local lattice solves)
   // what the device copies of the launch descriptors hold: a launch uploads
   // only what changed since the previous one
@@ -321,11 +324,11 @@ int upload(Plan* plan, const T* host, size_t n, const T** out) {
 
 // The slab form of a split lattice problem, where it asks for it and fits.
 int create_slabs(Plan* plan, const jja_problem_desc& d) {
-  if (!d.lattice_slabs || !d.lattice_rows || plan->parts < 2 || plan->block_size != kSlabBlock) return JJA_OK;
+  if (!d.lattice_slabs || !d.lattice_rows || plan->parts < 2 || plan->block_size != kPartBlock) return JJA_OK;
   SlabHost h;
   if (!build_slabs(d, plan->parts, kSplitLdsMax, &h)) return JJA_OK;
-  plan->slab_pairs = (h.d.pairs + plan->block_size - 1) / plan->block_size;
-  if (plan->slab_pairs > kSlabPairs) return JJA_OK;
+  const int32_t per = (std::max(h.d.pairs, h.d.faces) + kPartBlock - 1) / kPartBlock;
+  if (per > kSlabPairs) return JJA_OK;
   const std::vector<double> table = dst_table(d.lattice_cols);
   int rc;
   if ((rc = upload(plan, h.pair.data(), h.pair.size(), &h.d.pair))) return rc;
@@ -333,6 +336,7 @@ int create_slabs(Plan* plan, const jja_problem_desc& d) {
   if ((rc = upload(plan, h.face_code.data(), h.face_code.size(), &h.d.face_code))) return rc;
   if ((rc = upload(plan, h.face_id.data(), h.face_id.size(), &h.d.face_id))) return rc;
   if ((rc = upload(plan, h.face_at.data(), h.face_at.size(), &h.d.face_at))) return rc;
+  if ((rc = upload(plan, h.face_pos.data(), h.face_pos.size(), &h.d.face_pos))) return rc;
   if ((rc = upload(plan, table.data(), table.size(), &h.d.table))) return rc;
   if ((rc = upload(plan, h.inv.data(), h.inv.size(), &h.d.inv))) return rc;
   if ((rc = upload(plan, h.spike.data(), h.spike.size(), &h.d.spike))) return rc;
@@ -345,11 +349,65 @@ int create_slabs(Plan* plan, const jja_problem_desc& d) {
   if ((rc = upload(plan, flags.data(), flags.size(), &f))) return rc;
   h.d.ends = const_cast<double*>(e);
   h.d.flags = const_cast<uint32_t*>(f);
-  plan->slab = h.d;
-  plan->slab_lds = 8 * slab_lds_doubles(h.d, d.lattice_cols);
   const SlabDev* dev = nullptr;
-  if ((rc = upload(plan, &plan->slab, 1, &dev))) return rc;
-  plan->d_slab = const_cast<SlabDev*>(dev);
+  if ((rc = upload(plan, &h.d, 1, &dev))) return rc;
+  plan->d_parts = dev;
+  plan->parts_evolve = slab_evolve_kernel(per);
+  plan->parts_adjoint = slab_adjoint_kernel(per);
+  plan->parts_lds = 8 * slab_lds_doubles(h.d, d.lattice_cols);
+  return JJA_OK;
+}
+
+// The subdomains of a problem that has them (validated).
+int create_domains(Plan* plan, const jja_problem_desc& d) {
+  if (!d.domains) return JJA_OK;
+  const jja_domains& s = *d.domains;
+  const size_t G = s.parts, np = G * s.pairs, nf = G * s.faces;
+  DomainDev v{};
+  v.parts = s.parts;
+  v.pairs = s.pairs;
+  v.faces = s.faces;
+  v.n_gamma = s.n_gamma;
+  v.sources = s.sources;
+  v.n_published = s.n_published;
+  v.val_bytes = static_cast<int32_t>(s.n_entries * static_cast<int64_t>(sizeof(double)));
+  std::vector<uint32_t> pc(2 * np), fc(4 * nf), at(nf);
+  for (size_t i = 0; i < pc.size(); ++i) pc[i] = s.pair_code[2 * i] | static_cast<uint32_t>(s.pair_code[2 * i + 1]) << 16;
+  for (size_t i = 0; i < fc.size(); ++i) fc[i] = s.face_code[2 * i] | static_cast<uint32_t>(s.face_code[2 * i + 1]) << 16;
+  for (size_t i = 0; i < nf; ++i) at[i] = s.face_used[i] ? static_cast<uint32_t>(i % s.faces) : 0xffffffffu;
+  int rc;
+  if ((rc = upload(plan, s.pair, np, &v.pair))) return rc;
+  if ((rc = upload(plan, pc.data(), pc.size(), &v.pair_code))) return rc;
+  if ((rc = upload(plan, fc.data(), fc.size(), &v.face_code))) return rc;
+  if ((rc = upload(plan, at.data(), at.size(), &v.face_at))) return rc;
+  if ((rc = upload(plan, s.face_id, nf, &v.face_id))) return rc;
+  v.face_pos = v.face_id;  // solve positions are in circuit order
+  if ((rc = upload(plan, s.pub_ptr, G + 1, &v.pub_ptr))) return rc;
+  if ((rc = upload(plan, s.pub_at, static_cast<size_t>(s.n_published), &v.pub_at))) return rc;
+  if ((rc = upload(plan, s.source, static_cast<size_t>(s.n_gamma) * s.sources, &v.source))) return rc;
+  if ((rc = upload(plan, s.records, static_cast<size_t>(s.n_records), &v.solve_slices))) return rc;
+  if ((rc = upload(plan, s.wave_ptr, 2 * G * (kPartBlock / kWave + 1), &v.wave_ptr))) return rc;
+  if ((rc = upload(plan, s.slice_rows, static_cast<size_t>(s.n_slice_rows), &v.slice_rows))) return rc;
+  if ((rc = upload(plan, s.ent_val, static_cast<size_t>(s.n_entries), &v.ent_val))) return rc;
+  const uint16_t* off = nullptr;
+  if ((rc = upload(plan, s.ent_off, static_cast<size_t>(s.n_index), &off))) return rc;
+  v.ent_off = off;
+  const std::vector<double> pub(static_cast<size_t>(d.max_columns) * 2 * s.n_published, 0.0);
+  const std::vector<uint32_t> flags(static_cast<size_t>(d.max_columns) * G * (kPartBlock / kWave), 0u);
+  const double* e = nullptr;
+  const uint32_t* f = nullptr;
+  if ((rc = upload(plan, pub.data(), pub.size(), &e))) return rc;
+  if ((rc = upload(plan, flags.data(), flags.size(), &f))) return rc;
+  v.pub = const_cast<double*>(e);
+  v.flags = const_cast<uint32_t*>(f);
+  const DomainDev* dev = nullptr;
+  if ((rc = upload(plan, &v, 1, &dev))) return rc;
+  const int32_t per = (std::max(v.pairs, v.faces) + kPartBlock - 1) / kPartBlock;
+  plan->d_parts = dev;
+  plan->parts_evolve = domain_evolve_kernel(per);
+  plan->parts_adjoint = domain_adjoint_kernel(per);
+  plan->parts_lds = 8 * domain_lds_doubles(v);
+  plan->parts_only = true;
   return JJA_OK;
 }
 
@@ -458,6 +516,76 @@ int check_plan_shapes(int32_t n, const jja_problem_desc* descs) {
   return JJA_OK;
 }
 
+// Every index of a problem's subdomains.
+int validate_domains(const jja_problem_desc& d) {
+  const jja_domains& s = *d.domains;
+  auto bad = [](const char* what) { return fail(JJA_EINVAL, std::string("jja_plan_create: subdomains: ") + what); };
+  const int32_t G = s.parts, waves = kPartBlock / kWave;
+  if (G < 2 || G != parts_of(d) || d.block_size != G * kPartBlock || d.index_bytes != 4 || d.column_pairs ||
+      d.n_solve_slices || d.face_copy_rows || d.stencil_width != 3)
+    return bad("layout of the problem");
+  if (s.pairs < 1 || s.faces < 1 || s.n_gamma < 1 || s.sources < 1 || s.n_published < 1 || s.n_records < 1 ||
+      s.pairs > kDomainPairs * kPartBlock || s.faces > kDomainPairs * kPartBlock)
+    return bad("sizes");
+  const int64_t addresses = 2 * static_cast<int64_t>(s.faces) + s.n_gamma;
+  if (8 * (addresses + 2 * static_cast<int64_t>(s.pairs) + 1) > kSplitLdsMax) return bad("LDS");
+  if (!s.pair || !s.pair_code || !s.face_code || !s.face_id || !s.face_used || !s.pub_ptr || !s.pub_at || !s.source ||
+      !s.records || !s.wave_ptr || !s.slice_rows || !s.ent_val || !s.ent_off)
+    return bad("missing array");
+  for (int32_t q = 0; q < d.n_faces; ++q)
+    if (d.face_of_pos[q] != q) return bad("solve positions must be in circuit order");
+  for (int64_t i = 0; i < static_cast<int64_t>(G) * s.pairs; ++i) {
+    const int32_t e = s.pair[i];
+    if (e == -1) continue;
+    const int32_t q = e >> 4, m = e & 3;
+    if (e < 0 || m == 0 || 2 * q >= d.n_junctions || ((m & 2) && 2 * q + 1 >= d.n_junctions)) return bad("pair");
+    for (int32_t c = 0; c < 4; ++c)
+      if (s.pair_code[4 * i + c] != 0xffff && (s.pair_code[4 * i + c] >> 1) >= s.faces) return bad("pair code");
+  }
+  for (int64_t i = 0; i < static_cast<int64_t>(G) * s.faces; ++i) {
+    if (s.face_id[i] < -1 || s.face_id[i] >= d.n_faces || (s.face_id[i] >= 0 && !s.face_used[i])) return bad("face");
+    for (int32_t c = 0; c < 8; ++c)
+      if (s.face_code[8 * i + c] != 0xffff && (s.face_code[8 * i + c] >> 1) >= 2 * s.pairs) return bad("face code");
+  }
+  if (s.pub_ptr[0] != 0 || s.pub_ptr[G] != s.n_published) return bad("published ranges");
+  for (int32_t p = 0; p < G; ++p)
+    if (s.pub_ptr[p + 1] < s.pub_ptr[p]) return bad("published ranges");
+  for (int32_t i = 0; i < s.n_published; ++i)
+    if (s.pub_at[i] < 0 || s.pub_at[i] >= s.faces) return bad("published face");
+  for (int64_t i = 0; i < static_cast<int64_t>(s.n_gamma) * s.sources; ++i)
+    if (s.source[i] < -1 || s.source[i] >= s.n_published) return bad("source");
+  if (s.n_entries < kMaxIter * kWave || s.n_entries * 8 >= (int64_t{1} << 31) || s.n_index < kMaxIter * kWave)
+    return bad("record arrays");
+  for (int32_t pr = 0; pr < 2 * G; ++pr) {
+    const int32_t* wp = s.wave_ptr + static_cast<int64_t>(pr) * (waves + 1);
+    int32_t barriers = -1;
+    for (int32_t w = 0; w < waves; ++w) {
+      if (wp[w] < 0 || wp[w + 1] > s.n_records || wp[w + 1] - wp[w] < 4 || (wp[w + 1] - wp[w] - 4) % 3)
+        return bad("wave program");
+      int32_t nb = 0;
+      for (int32_t k = wp[w]; k < wp[w + 1]; ++k) {
+        const jja_slice& m = s.records[k];
+        const int32_t g = m.flags & 0xff, rows = m.flags >> 16;
+        if (!pow2_le(g, kWave) || m.n_iter < 0 || m.n_iter > kMaxIter || rows < 0 || rows > kWave / g || m.r0 != 0 ||
+            (m.flags & (0xe000 | JJA_SLICE_NARROW | JJA_SLICE_WG_BARRIER)))
+          return bad("record fields");
+        if (m.base < 0 || (m.base % 2) || m.base + kMaxIter * kWave > s.n_entries || m.ibase < 0 || (m.ibase % 8) ||
+            m.ibase + kMaxIter * kWave > s.n_index || m.rowbase < 0 || m.rowbase + kWave / g > s.n_slice_rows)
+          return bad("record data");
+        if (k >= wp[w + 1] - 4) continue;  // loaded ahead, never executed
+        nb += (m.flags & JJA_SLICE_BARRIER) != 0;
+        for (int32_t i = 0; i < rows; ++i)
+          if (s.slice_rows[m.rowbase + i] < -1 || s.slice_rows[m.rowbase + i] >= addresses) return bad("record row");
+        for (int64_t e = m.ibase; e < m.ibase + kMaxIter * kWave; ++e)
+          if (s.ent_off[e] >= addresses) return bad("record index");
+      }
+      if (barriers < 0) barriers = nb;
+      if (nb != barriers) return bad("wave programs disagree on their barriers");
+    }
+  }
+  return JJA_OK;
+}
+
 // Every index the kernels follow is checked here, once, on the host.
 int validate(const jja_problem_desc& d) {
   const int32_t Nj = d.n_junctions, Nf = d.n_faces, BS = d.block_size, ms = d.max_stage_rows;
@@ -540,6 +668,7 @@ int validate(const jja_problem_desc& d) {
       return fail(JJA_EINVAL, "lattice_gc must be finite and > 0");
     return JJA_OK;
   }
+  if (d.domains) return validate_domains(d);
   // solve programs: one per wave of 64 lanes; each runs a multiple of three
   // records and loads four more ahead, all of which must be in range
   const int32_t NW = BS / kWave;
@@ -862,34 +991,34 @@ int launch_evolve_split(Plan* plan, int32_t n, int32_t n_steps, int64_t step0, h
   }
 }
 
-// Whether a run can go to the slab kernels: the usual step (stencil 3, no voltage
-// sources, noise from Philox with a given amplitude or none).
-bool slab_run(const Plan* plan, const jja_problem_run& r) {
-  return plan->d_slab && plan->stencil_width == 3 && r.Vs.zero && !r.noise && (r.T.zero || r.sigma.base);
+// Whether a run can go to the kernels that keep each part's junctions on chip: the
+// usual step (stencil 3, no voltage sources, noise from Philox with a given
+// amplitude or none).
+bool parts_run(const Plan* plan, const jja_problem_run& r) {
+  return plan->d_parts && plan->stencil_width == 3 && r.Vs.zero && !r.noise && (r.T.zero || r.sigma.base);
 }
 
-int launch_evolve_slab(Plan* plan, int32_t n, int32_t n_steps, int64_t step0, hipStream_t stream) {
+int launch_evolve_parts(Plan* plan, int32_t n, int32_t n_steps, int64_t step0, hipStream_t stream) {
   const DevProblem* probs = plan->d_problems;
   const jja_problem_run* runs = plan->d_runs;
   const WorkItem* work = plan->d_work;
-  const SlabDev* slabs = plan->d_slab;
-  const uint32_t seq = plan->slab_seq;
-  const int rc = launch_cooperative(plan, slab_evolve_kernel(plan->slab_pairs), plan->block_size, n,
-                                    plan->slab_lds, stream, probs, runs, work, slabs, n_steps, step0, seq, plan->d_err,
-                                    plan->wait_limit);
-  if (rc == JJA_OK) plan->slab_seq += static_cast<uint32_t>(n_steps);
+  const void* tables = plan->d_parts;
+  const uint32_t seq = plan->parts_seq;
+  const int rc = launch_cooperative(plan, plan->parts_evolve, plan->block_size, n, plan->parts_lds, stream, probs, runs,
+                                    work, tables, n_steps, step0, seq, plan->d_err, plan->wait_limit);
+  if (rc == JJA_OK) plan->parts_seq += static_cast<uint32_t>(n_steps);
   return rc;
 }
 
-int launch_adjoint_slab(Plan* plan, int32_t n, int64_t k_hi, int64_t k_lo, hipStream_t stream) {
+int launch_adjoint_parts(Plan* plan, int32_t n, int64_t k_hi, int64_t k_lo, hipStream_t stream) {
   const DevProblem* probs = plan->d_problems;
   const jja_adjoint_run* runs = plan->d_adj;
   const WorkItem* work = plan->d_work;
-  const SlabDev* slabs = plan->d_slab;
-  const uint32_t seq = plan->slab_seq;
-  const int rc = launch_cooperative(plan, slab_adjoint_kernel(plan->slab_pairs), plan->block_size, n, plan->slab_lds,
-                                    stream, probs, runs, work, slabs, k_hi, k_lo, seq, plan->d_err, plan->wait_limit);
-  if (rc == JJA_OK) plan->slab_seq += static_cast<uint32_t>(k_hi - k_lo + 1);
+  const void* tables = plan->d_parts;
+  const uint32_t seq = plan->parts_seq;
+  const int rc = launch_cooperative(plan, plan->parts_adjoint, plan->block_size, n, plan->parts_lds, stream, probs, runs,
+                                    work, tables, k_hi, k_lo, seq, plan->d_err, plan->wait_limit);
+  if (rc == JJA_OK) plan->parts_seq += static_cast<uint32_t>(k_hi - k_lo + 1);
   return rc;
 }
 
@@ -1178,7 +1307,7 @@ int jja_plan_create(int32_t n_problems, const jja_problem_desc* descs, jja_plan*
     alloc(2 * sizeof(uint32_t) * items, reinterpret_cast<void**>(&plan->d_ctrs));
     plan->ctr_cap = 2 * items;
   }
-  if (rc == JJA_OK && n_problems == 1) rc = create_slabs(plan, descs[0]);
+  if (rc == JJA_OK && n_problems == 1) rc = descs[0].domains ? create_domains(plan, descs[0]) : create_slabs(plan, descs[0]);
   if (rc == JJA_OK && hipEventCreateWithFlags(&plan->done, hipEventDisableTiming) != hipSuccess)
     rc = fail(JJA_EHIP, "jja_plan_create: hipEventCreateWithFlags failed");
   if (rc == JJA_OK && plan->parts > 1) {
@@ -1260,6 +1389,8 @@ int jja_evolve(jja_plan* p, const jja_problem_run* runs, int32_t n_steps, int64_
     if (r.W > plan->max_cols[i])
       return fail(JJA_EINVAL, "jja_evolve: problem " + std::to_string(i) + " has more columns than its max_columns");
     if (r.dt <= 0) return fail(JJA_EINVAL, "jja_evolve: dt must be positive");
+    if (plan->parts_only && !parts_run(plan, r))
+      return fail(JJA_EUNSUPPORTED, "jja_evolve: subdomains take no voltage sources, given normals or varying temperature");
     if (!r.Is.base || !r.Vs.base || !r.f.base || !r.T.base)
       return fail(JJA_EINVAL, "jja_evolve: every source needs a base array");
     if (!r.Vs.zero && !r.theta_s) return fail(JJA_EINVAL, "jja_evolve: non-zero Vs needs theta_s");
@@ -1288,9 +1419,8 @@ int jja_evolve(jja_plan* p, const jja_problem_run* runs, int32_t n_steps, int64_
     work.insert(work.end(), work_g.begin(), work_g.end());
     const std::vector<WorkItem> split = split_work(plan, work);
     if ((rc = upload_work(plan, split, stream))) return rc;
-    const bool slab = slab_run(plan, runs[0]);
-    if (slab)
-      rc = launch_evolve_slab(plan, static_cast<int32_t>(split.size()), n_steps, step0, stream);
+    if (parts_run(plan, runs[0]))
+      rc = launch_evolve_parts(plan, static_cast<int32_t>(split.size()), n_steps, step0, stream);
     else if ((rc = reset_counters(plan, work.size(), stream)))
       return rc;
     else
@@ -1353,8 +1483,8 @@ int jja_adjoint(jja_plan* p, const jja_adjoint_run* runs, int64_t k_hi, int64_t 
     work.insert(work.end(), work_g.begin(), work_g.end());
     const std::vector<WorkItem> split = split_work(plan, work);
     if ((rc = upload_work(plan, split, stream))) return rc;
-    if (plan->d_slab)
-      rc = launch_adjoint_slab(plan, static_cast<int32_t>(split.size()), k_hi, k_lo, stream);
+    if (plan->d_parts)
+      rc = launch_adjoint_parts(plan, static_cast<int32_t>(split.size()), k_hi, k_lo, stream);
     else if ((rc = reset_counters(plan, work.size(), stream)))
       return rc;
     else

@@ -8,29 +8,21 @@
 #include <vector>
 
 #include "../../include/jja.h"
+#include "jja_parts.h"
 
-// Threads of a workgroup, junction pairs a thread may hold, and faces it sums per pair it holds.
-constexpr int kSlabBlock = 512;
+// Most junction pairs a thread holds.
 constexpr int kSlabPairs = 9;
-constexpr int kSlabFacesPerPair = 1;
 
 // One problem's slabs as the kernels see them (device pointers). Part p works on
 // the face rows r0 = p * base + min(p, extra) .. r0 + s - 1, s = base + (p < extra),
 // and on every junction one of them touches; its local rows are 0 (the row below),
 // 1 .. s and s + 1 (the row above), each of ld doubles.
-struct SlabDev {
-  int32_t parts, base, extra, rows;      // rows: the most rows a part has
+struct SlabDev : PartTables {
+  int32_t base, extra, rows;             // rows: the most rows a part has
   int32_t ld, buf;                       // doubles per local row, doubles of one local face array
-  int32_t pairs, faces;                  // slots per part: junction pairs, faces
   int32_t table_lds;                     // the sine table lies in LDS (else it is read from memory)
   int32_t mode_waves;                    // waves that hold the modes (two lanes each)
   int32_t inv_lds;                       // the pivots lie in LDS
-  int32_t pad_;
-  const int32_t* pair;                   // [parts][pairs]: pair * 16 + present bits + 4 * owner bits, or -1
-  const uint32_t* pair_code;             // [parts][pairs][2]: two incidence codes of each member
-  const uint32_t* face_code;             // [parts][faces][2]: four codes of local junction values
-  const int32_t* face_id;                // [parts][faces]: face index, or -1
-  const uint32_t* face_at;               // [parts][faces]: address among the local rows
   const double* table;                   // sine table of C modes (DstShape)
   const double* inv;                     // [rows][C] inverse pivots of a part's own block
   const double* spike;                   // [2][rows][C]: response to the row below, parts of base and base + 1 rows
@@ -42,7 +34,7 @@ struct SlabDev {
 // Host arrays of the same, built from a descriptor.
 struct SlabHost {
   SlabDev d{};
-  std::vector<int32_t> pair, face_id;
+  std::vector<int32_t> pair, face_id, face_pos;
   std::vector<uint32_t> pair_code, face_code, face_at;
   std::vector<double> inv, spike, reduced;
 };
@@ -55,7 +47,7 @@ int64_t slab_lds_doubles(const SlabDev& d, int32_t cols);
 // junctions, or a local index does not fit.
 bool build_slabs(const jja_problem_desc& desc, int32_t parts, int64_t lds_bytes, SlabHost* out);
 
-// Kernels (workgroups of kSlabBlock threads) whose threads hold at most `pairs`
+// Kernels (workgroups of kPartBlock threads) whose threads hold at most `pairs`
 // junction pairs each, or NULL.
 const void* slab_evolve_kernel(int pairs);
 const void* slab_adjoint_kernel(int pairs);

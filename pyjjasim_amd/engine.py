@@ -177,9 +177,24 @@ def slab_parts(host, columns, n_cu, max_parts=16):
     return 1 if parts == 2 and host.Nj <= RESIDENT_JUNCTIONS else parts
 
 
-def takes_slabs(problem):
-    """Whether a problem leaves its layout open and its runs are ones the slab
-    kernels take (the usual step: stencil 3, no voltage sources, noise from Philox
+# subdomains of any other circuit (jja_domain.hip): the fewest faces a part has, and
+# the most faces of a circuit that two parts take
+DOMAIN_MIN_FACES = 100
+DOMAIN_PAIR_FACES = 2000
+
+
+def domain_parts(Nf, columns, n_cu, max_parts=32):
+    """Subdomains per column: the most whose workgroups, one per compute unit, all
+    fit on the device and keep enough faces each."""
+    parts = 1
+    while parts < max_parts and 2 * parts * columns <= n_cu and Nf >= 2 * parts * DOMAIN_MIN_FACES:
+        parts *= 2
+    return 1 if parts == 2 and Nf > DOMAIN_PAIR_FACES else parts
+
+
+def takes_parts(problem):
+    """Whether a problem leaves its layout open and its runs are ones the kernels
+    of slabs and subdomains take (the usual step: stencil 3, no voltage sources, noise from Philox
     at a constant temperature or none)."""
     def open_to(name, default):
         return getattr(problem, name, default) in (None, default)
@@ -211,16 +226,23 @@ class Engine:
         self.lib = lib = _native.lib()
         if shared is None:
             self.block_size = problem.block_size or default_block_size(Nj, Nf)
+            parts_open = takes_parts(problem)
+            domains = domain_parts(Nf, W, device_compute_units()) \
+                if parts_open and getattr(problem, "solver", "auto") == "auto" \
+                and getattr(problem, "local_stages", "auto") == "auto" else 1
             self.host = CircuitPlan(circuit, dt, sw, leaf_size=problem.leaf_size,
                                     block_size=self.block_size,
                                     face_store=getattr(problem, "face_store", "auto"),
                                     local_stages=getattr(problem, "local_stages", "auto"),
-                                    solver=getattr(problem, "solver", "auto"))
+                                    solver=getattr(problem, "solver", "auto"), domains=domains)
+            self.block_size = self.host.block_size
             parts = getattr(problem, "parts", None)
-            slabs = slab_parts(self.host, W, device_compute_units()) if takes_slabs(problem) else 1
+            slabs = slab_parts(self.host, W, device_compute_units()) if parts_open else 1
             if slabs > 1:
                 self.block_size = SLAB_BLOCK
                 self.host = self.host.relayout(SLAB_BLOCK, slabs, slabs=True)
+                parts = 1
+            elif self.host.domains is not None:
                 parts = 1
             elif parts is None:
                 parts = auto_parts(self.host, W, sw)

@@ -359,7 +359,7 @@ class CircuitPlan:
     on the row."""
 
     def __init__(self, circuit, dt, stencil_width=3, leaf_size=16, block_size=1024, target_iter=8,
-                 face_store="auto", parts=1, local_stages="auto", solver="auto"):
+                 face_store="auto", parts=1, local_stages="auto", solver="auto", domains=1):
         if face_store not in ("auto", "lds", "global"):
             raise ValueError("face_store must be 'auto', 'lds' or 'global'")
         if solver not in SOLVERS:
@@ -399,10 +399,25 @@ class CircuitPlan:
         else:
             self.circuit_xy = None
             xy = np.zeros((0, 2))
-        self.solve_plan = SolvePlan(self.K, xy, leaf_size=leaf_size)
+        self._factor = {"K": self.K, "xy": xy, "leaf_size": leaf_size}
         self.lattice = lattice_solve(self.K, xy) if self.Nf and solver != "cholesky" else None
         self.target_iter = target_iter
+        self.domains = None
+        if domains > 1 and self.Nf and self.lattice is None and stencil_width == 3:
+            from .domain_plan import BLOCK, DomainPlan
+            plan = DomainPlan(self.K, xy, self.junc_code, domains)
+            if plan.ok:
+                self.domains, self.parts, self.block_size = plan, domains, BLOCK
         self._build_layouts(target_iter)
+
+    @property
+    def solve_plan(self):
+        """The staged factor of K, made when a layout first needs it (a lattice solve
+        and subdomains do not) and shared by the relayouts."""
+        f = self._factor
+        if "plan" not in f:
+            f["plan"] = SolvePlan(f["K"], f["xy"], leaf_size=f["leaf_size"])
+        return f["plan"]
 
     def relayout(self, block_size, parts=None, face_store=None, local_stages=None, solver=None, slabs=False):
         """The same circuit, factor and schedule laid out for another workgroup
@@ -413,6 +428,7 @@ class CircuitPlan:
         other.block_size = block_size
         other.column_pairs = False
         other.slabs = slabs
+        other.domains = None
         if solver is not None:
             if solver not in SOLVERS:
                 raise ValueError("solver must be 'auto', 'lattice' or 'cholesky'")
@@ -585,10 +601,13 @@ class CircuitPlan:
         return wave_of_grp[label1], part_of
 
     def _build_layouts(self, target_iter=8):
-        BS, sp, Nf, Nj = self.column_threads, self.solve_plan, self.Nf, self.Nj
+        BS, Nf, Nj = self.column_threads, self.Nf, self.Nj
         self._lattice_layout = False
         if Nf == 0:
             self._build_faceless()
+            return
+        if getattr(self, "domains", None) is not None:
+            self._build_domain_layout()
             return
         lattice_ok = self.lattice is not None and self.solver != "cholesky"
         if self.solver == "lattice" and not lattice_ok:
@@ -597,6 +616,7 @@ class CircuitPlan:
         if lattice_ok:
             self._build_lattice_layout()
             return
+        sp = self.solve_plan
         # the face vector and stage scratch of a column: in the workgroup's LDS
         # when they fit (16-bit indices), else in a global per-column array.
         # Wave-local stages keep every scratch row of those stages at once.
@@ -738,7 +758,7 @@ class CircuitPlan:
     def _build_lattice_layout(self):
         """Face records by lattice position (r*C + c) and no solve program: the
         kernel solves K by the lattice solve (lattice_solve.py)."""
-        lat, Nf, Nj, BS = self.lattice, self.Nf, self.Nj, self.column_threads
+        lat, Nf, Nj = self.lattice, self.Nf, self.Nj
         scratch = lat.scratch_rows(Nf, self.parts)
         fits = Nf + scratch <= min(LDS_BYTES // 8, 65536)
         if self.face_store == "lds" and not fits:
@@ -753,6 +773,21 @@ class CircuitPlan:
         jpos = np.where(jc >= 0, 2 * pos[np.maximum(jc, 0) >> 1] + (jc & 1), -1)
         self.junc_pos_code = jpos.astype(np.int32).ravel()
         self.face_of_pos = lat.face_of_pos.astype(np.int32)
+        self._face_records_only(pos)
+        self._lattice_layout = True
+
+    def _build_domain_layout(self):
+        """Face records in circuit order and no solve program: the subdomains hold
+        the solve (domain_plan.py)."""
+        self.global_store, self.index_bytes = True, 4
+        self.local_stages = self.part_stages = self.scratch_rows = 0
+        self.junc_pos_code = np.ascontiguousarray(self.junc_code, dtype=np.int32)
+        self.face_of_pos = np.arange(self.Nf, dtype=np.int32)
+        self._face_records_only(np.arange(self.Nf))
+
+    def _face_records_only(self, pos):
+        """Face records by solve position ``pos`` and an empty solve program."""
+        BS = self.column_threads
         fp = self.face_ptr.astype(np.int64)
         F = sliced(fp, self.face_code.astype(np.int64), np.ones(int(fp[-1])), BS, pos, fixed_group=1,
                    target_iter=FACE_ITER)
@@ -778,7 +813,6 @@ class CircuitPlan:
         self._face_rec = self._slice_array(self.face_slices)
         self._solve_rec = self._slice_array([])
         self._wave_ptr = np.ascontiguousarray(self.wave_ptr, dtype=np.int32)
-        self._lattice_layout = True
 
     def _build_faceless(self):
         """A circuit without faces (a tree): K is 0 x 0 and the step is
@@ -1065,7 +1099,6 @@ class CircuitPlan:
     def desc(self, max_columns=1):
         """ctypes ProblemDesc pointing at this object's arrays (keep self alive),
         for runs of at most ``max_columns`` columns."""
-        sp = self.solve_plan
         P = _native.ptr
         d = _native.ProblemDesc()
         d.n_junctions, d.n_faces = self.Nj, self.Nf
@@ -1097,6 +1130,9 @@ class CircuitPlan:
         if self.uses_lattice:
             self.lattice.set_desc(d)
             d.lattice_slabs = int(self.slabs)
+        if getattr(self, "domains", None) is not None:
+            self._domain_desc = self.domains.desc()
+            d.domains = C.addressof(self._domain_desc)
         return d
 
     def lds_bytes(self):
@@ -1291,6 +1327,6 @@ class MatrixPlan(CircuitPlan):
         self.Rv = np.zeros(0)
         self.Ic = np.zeros(0)
         self.K = K
-        self.solve_plan = SolvePlan(K, np.asarray(xy, dtype=np.float64), leaf_size=leaf_size)
+        self._factor = {"K": K, "xy": np.asarray(xy, dtype=np.float64), "leaf_size": leaf_size}
         self.target_iter = 8
         self._build_layouts(self.target_iter)

@@ -1,0 +1,91 @@
+"""Subdomains of a circuit's face system (domain_plan.py): the kernel's steps,
+emulated on the host from the rows it streams, against a direct sparse solve; every
+junction in one part; what does not fit or is not positive definite is left to the
+factor."""
+import numpy as np
+import pytest
+import scipy.sparse
+import scipy.sparse.linalg
+
+import pyjjasim_amd as pa
+from pyjjasim_amd.domain_plan import DomainPlan
+from pyjjasim_amd.solver_plan import CircuitPlan, cycle_codes, face_system_matrix
+
+
+def _system(c):
+    cx, cy = c.get_face_centroids()
+    jc = cycle_codes(c.get_cycle_matrix(), c._Nf(), c._Nj())[2]
+    return face_system_matrix(c, 0.05), np.stack([cx, cy], axis=1), jc
+
+
+def _disordered():
+    c = pa.SquareArray(21, 17)
+    rng = np.random.default_rng(2)
+    c.set_resistance(np.exp(0.3 * rng.standard_normal(c.junction_count())))
+    c.set_capacitance(rng.random(c.junction_count()))
+    return c
+
+
+def _mutual():
+    c = pa.SquareArray(14, 13)
+    n = c.junction_count()
+    c.set_inductance(scipy.sparse.diags([0.1, 1.0, 0.1], [-1, 0, 1], shape=(n, n)).tocsc())
+    return c
+
+
+CIRCUITS = {"honeycomb": (lambda: pa.HoneycombArray(11, 9), 4), "triangular": (lambda: pa.TriangularArray(9, 8), 8),
+            "triangular_16": (lambda: pa.TriangularArray(20, 21), 16), "square_R": (_disordered, 2),
+            "square_R_32": (_disordered, 32), "mutual": (_mutual, 4)}
+
+
+@pytest.mark.parametrize("name", sorted(CIRCUITS))
+def test_domain_solve_matches_direct(name):
+    make, parts = CIRCUITS[name]
+    K, xy, jc = _system(make())
+    d = DomainPlan(K, xy, jc, parts)
+    assert d.ok
+    b = np.random.default_rng(1).standard_normal(K.shape[0])
+    x = scipy.sparse.linalg.spsolve(K.tocsc(), b)
+    assert np.abs(d.emulate(b) - x).max() <= 1e-11 * np.abs(x).max()
+    # every junction is present and owned once
+    e = d.pair[d.pair >= 0]
+    held = np.concatenate([2 * (e[(e >> m) & 1 == 1] >> 4) + m for m in range(2)])
+    assert np.array_equal(np.sort(held), np.arange(len(jc) // 2))
+    assert np.array_equal((e & 3) << 2, e & 12)
+    # every face's flux and gradient belong to one part
+    assert np.array_equal(np.sort(d.face_id[d.face_id >= 0]), np.arange(K.shape[0]))
+
+
+def test_domain_plan_validates():
+    """The descriptor of a plan with subdomains passes the library's checks, and a
+    changed index does not."""
+    import ctypes as C
+    from pyjjasim_amd import _native
+    c = pa.HoneycombArray(11, 9)
+    plan = CircuitPlan(c, 0.05, domains=4)
+    assert plan.domains is not None and plan.parts == 4
+    lib = _native.lib()
+    assert lib.jja_plan_validate(1, C.byref(plan.desc(max_columns=2))) == 0
+    for name, value in (("ent_off", 60000), ("pub_at", plan.domains.n_local), ("slice_rows", 1 << 20),
+                        ("source", 1 << 20), ("face_code", 4 * plan.domains.pairs), ("pair", 1 << 26)):
+        a = getattr(plan.domains, name)
+        a = a.reshape(-1)
+        at = int(np.flatnonzero(a != a[0])[0]) if name in ("ent_off", "slice_rows") else 0
+        old = a[at]
+        a[at] = value
+        assert lib.jja_plan_validate(1, C.byref(plan.desc(max_columns=2))) != 0, name
+        a[at] = old
+    assert lib.jja_plan_validate(1, C.byref(plan.desc(max_columns=2))) == 0
+
+
+def test_domain_plan_leaves_the_rest_to_the_factor():
+    K, xy, jc = _system(pa.HoneycombArray(11, 9))
+    assert not DomainPlan(-K, xy, jc, 4).ok                    # not positive definite
+    K2 = K.copy()
+    K2.data[:] = np.nan
+    assert not DomainPlan(K2, xy, jc, 4).ok
+    assert not DomainPlan(*_system(pa.HoneycombArray(3, 2)), 16).ok    # parts without faces of their own
+    # lattices keep the lattice solve, other stencils the factor
+    assert CircuitPlan(pa.SquareArray(12, 12), 0.05, domains=4).uses_lattice
+    p = CircuitPlan(pa.HoneycombArray(11, 9), 0.05, 4, domains=4)
+    assert p.domains is None and p.parts == 1
