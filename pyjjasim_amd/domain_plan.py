@@ -41,10 +41,10 @@ LDS_DOUBLES = 163840 // 8 - 32
 CELLS = (1, 2, 4, 8, 16, 32)
 
 
-def bisect(faces, xy, adj, levels):
+def bisect(faces, xy, touched, levels):
     """``faces`` cut into 2^levels parts and the separators between them: halves by
-    the longer side's coordinate, the faces of the second half that touch the
-    first taken out."""
+    the longer side's coordinate, the faces of the second half that the first half
+    touches (``touched``: index array -> mask over all faces) taken out."""
     none = np.zeros(0, dtype=np.int64)
     if levels == 0:
         return [faces], none
@@ -55,13 +55,10 @@ def bisect(faces, xy, adj, levels):
     order = faces[np.argsort(p[:, axis], kind="stable")]
     half = (len(order) + 1) // 2
     a, b = order[:half], order[half:]
-    touched = np.zeros(adj.shape[0], dtype=bool)
-    touched[adj[a].indices] = True
-    cut = touched[b]
-    sep, rest = b[cut], b[~cut]
-    pa, sa = bisect(a, xy, adj, levels - 1)
-    pb, sb = bisect(rest, xy, adj, levels - 1)
-    return pa + pb, np.concatenate((sep, sa, sb))
+    cut = touched(a)[b]
+    pa, sa = bisect(a, xy, touched, levels - 1)
+    pb, sb = bisect(b[~cut], xy, touched, levels - 1)
+    return pa + pb, np.concatenate((b[cut], sa, sb))
 
 
 def spd_inverse(M):
@@ -85,22 +82,14 @@ class _Programs(CircuitPlan):
 
 
 def _phase(rows, blocks, kind):
-    """A phase for the builder: row i sums blocks (matrix, column addresses) in turn."""
+    """A phase for the builder: row i sums dense blocks (row numbers, column
+    addresses, matrix) in turn."""
     n = len(rows)
-    lens = np.zeros(n, dtype=np.int64)
-    idx, val, who = [], [], []
-    for M, cols in blocks:
-        r, c = np.nonzero(M)
-        idx.append(np.asarray(cols, dtype=np.int64)[c])
-        val.append(M[r, c])
-        who.append(r)
-    if idx:
-        who = np.concatenate(who)
-        order = np.argsort(who, kind="stable")
-        idx, val = np.concatenate(idx)[order], np.concatenate(val)[order]
-        lens = np.bincount(who, minlength=n)
-    else:
-        idx, val = np.zeros(0, dtype=np.int64), np.zeros(0)
+    who = np.concatenate([np.repeat(r, len(c)) for r, c, _ in blocks])
+    order = np.argsort(who, kind="stable")
+    idx = np.concatenate([np.tile(c, len(r)) for r, c, _ in blocks])[order]
+    val = np.concatenate([M.ravel() for _, _, M in blocks])[order]
+    lens = np.bincount(who, minlength=n)
     ptr = np.concatenate(([0], np.cumsum(lens)))
     return (0, np.asarray(rows, dtype=np.int64), ptr, idx, val, kind, None, "col", "col")
 
@@ -116,9 +105,12 @@ class DomainPlan:
         K = scipy.sparse.csr_matrix(K)
         Nf, Nj = K.shape[0], len(junc_code) // 2
         self.Nf, self.Nj = Nf, Nj
-        adj = K.copy()
-        adj.data = np.ones_like(adj.data)
-        interiors, gamma = bisect(np.arange(Nf), xy, adj, parts.bit_length() - 1)
+
+        def touched(a):
+            mask = np.zeros(Nf, dtype=bool)
+            mask[K[a].indices] = True
+            return mask
+        interiors, gamma = bisect(np.arange(Nf), xy, touched, parts.bit_length() - 1)
         if min(len(i) for i in interiors) < 1 or len(gamma) > MAX_GAMMA or len(gamma) == 0:
             return
         gamma = np.sort(gamma)
@@ -134,7 +126,7 @@ class DomainPlan:
         if clash.any():
             return                         # interiors joined by a junction of weight zero in K
         # separator faces that border each interior, then those of the junctions it is given
-        border = [set(gamma[np.asarray(adj[gamma][:, f].sum(axis=1)).ravel() > 0].tolist()) for f in interiors]
+        border = [set(gamma[touched(f)[gamma]].tolist()) for f in interiors]
         load = np.bincount(owner[owner >= 0], minlength=parts)
         for j in np.flatnonzero(owner < 0):
             mine = [int(f) for f in face[j] if f >= 0]
@@ -155,7 +147,7 @@ class DomainPlan:
             return
         self.n_local = n_loc
         try:
-            if not self._choose_cells(K, xy, adj):
+            if not self._choose_cells(K, xy):
                 return
         except np.linalg.LinAlgError:
             return                         # not positive definite: left to the factor to refuse
@@ -165,17 +157,17 @@ class DomainPlan:
         self.ok = 2 * n_loc + len(gamma) + 2 * self.pairs + 2 <= LDS_DOUBLES
 
     # ------------------------------------------------------------- elimination
-    def _eliminate(self, K, f, border, cells, seps):
-        """Dense operators of one interior: per cell (faces, inverse, border rows,
-        E); separators' Schur inverse and E onto the border; the border's update."""
+    def _eliminate(self, K, cells, seps, border):
+        """Dense operators of one interior from its dense matrix K (local indices):
+        per cell (faces, inverse, border rows, E); the separators' Schur inverse and
+        E onto the border; the border's update."""
         rows = np.concatenate((seps, border))
         ns = len(seps)
         Krr = np.zeros((len(rows), len(rows)))   # minus what the cells add
         ops = []
         for c in cells:
-            Kc = K[c][:, c].toarray()
-            inv = spd_inverse(Kc)
-            Krc = K[rows][:, c].toarray()
+            inv = spd_inverse(K[np.ix_(c, c)])
+            Krc = K[np.ix_(rows, c)]
             hit = np.flatnonzero(np.abs(Krc).sum(axis=1))
             E = Krc[hit] @ inv
             Krr[np.ix_(hit, hit)] -= E @ Krc[hit].T
@@ -183,52 +175,56 @@ class DomainPlan:
         Sl = Eb = None
         up = Krr[ns:, ns:].copy()
         if ns:
-            S = K[seps][:, seps].toarray() + Krr[:ns, :ns]
-            Sl = spd_inverse(S)
-            Kbs = K[border][:, seps].toarray() + Krr[ns:, :ns]
+            Sl = spd_inverse(K[np.ix_(seps, seps)] + Krr[:ns, :ns])
+            Kbs = K[np.ix_(border, seps)] + Krr[ns:, :ns]
             Eb = Kbs @ Sl
             up -= Eb @ Kbs.T
         return ops, Sl, Eb, up
 
-    def _choose_cells(self, K, xy, adj):
+    def _choose_cells(self, K, xy):
         """Cells per interior: the count whose operators have the fewest entries,
-        each phase counted as the entries a workgroup streams meanwhile."""
+        each phase counted as the entries a workgroup streams meanwhile. Then every
+        part's operators and the separators' Schur inverse."""
+        def local(p):
+            f = np.concatenate((self.interiors[p], self.border[p]))
+            return f, K[f][:, f].toarray(), len(self.interiors[p])
+
+        def cut(D, at, n, levels):
+            near = D[:n, :n] != 0
+            return bisect(np.arange(n), at, lambda a: near[a].any(axis=0), levels)
         best = None
-        p = int(np.argmax([len(i) for i in self.interiors]))
-        f, b = self.interiors[p], len(self.border[p])
-        for n in CELLS:
-            if len(f) < 4 * n:
+        f, D, n = local(int(np.argmax([len(i) for i in self.interiors])))
+        for count in CELLS:
+            if n < 4 * count:
                 break
-            cells, seps = bisect(f, xy, adj, n.bit_length() - 1)
+            cells, seps = cut(D, xy[f], n, count.bit_length() - 1)
             if min(len(c) for c in cells) < 1:
                 break
-            rows = np.concatenate((seps, self.border[p]))
-            work = 0
-            for c in cells:
-                hit = int((np.asarray(adj[rows][:, c].sum(axis=1)).ravel() > 0).sum())
-                work += len(c) * (len(c) + 2 * hit)
+            rows = np.concatenate((seps, np.arange(n, len(f))))
+            work = sum(len(c) * (len(c) + 2 * int((D[np.ix_(rows, c)] != 0).any(axis=1).sum())) for c in cells)
             ns = len(seps)
-            work += ns * (ns + 2 * b) + (2 * 3000 if ns else 0)
+            work += ns * (ns + 2 * (len(f) - n)) + (2 * 3000 if ns else 0)
             if best is None or work < best[0]:
-                best = (work, n)
+                best = (work, count)
         if best is None:
             return False
         self.cells = best[1]
-        G = len(self.gamma)
         gpos = -np.ones(self.Nf, dtype=np.int64)
-        gpos[self.gamma] = np.arange(G)
+        gpos[self.gamma] = np.arange(len(self.gamma))
         S = K[self.gamma][:, self.gamma].toarray()
         self.local = []
-        for f, b in zip(self.interiors, self.border):
-            n = self.cells
+        for p in range(self.parts):
+            f, D, n = local(p)
+            count = self.cells
             while True:
-                cells, seps = bisect(f, xy, adj, n.bit_length() - 1)
-                if min(len(c) for c in cells) >= 1 or n == 1:
+                cells, seps = cut(D, xy[f], n, count.bit_length() - 1)
+                if count == 1 or min(len(c) for c in cells) >= 1:
                     break
-                n //= 2
-            ops, Sl, Eb, up = self._eliminate(K, f, b, cells, seps)
-            S[np.ix_(gpos[b], gpos[b])] += up
-            self.local.append((ops, seps, Sl, Eb))
+                count //= 2
+            ops, Sl, Eb, up = self._eliminate(D, cells, seps, np.arange(n, len(f)))
+            g = gpos[self.border[p]]
+            S[np.ix_(g, g)] += up
+            self.local.append(([(f[c], inv, hit, E) for c, inv, hit, E in ops], f[seps], Sl, Eb))
         self.gpos = gpos
         self.Sinv = spd_inverse(S)
         return True
@@ -298,31 +294,20 @@ class DomainPlan:
         order, at = self.addr[p]
         b, n = self.border[p], self.n_local
         rows = np.concatenate((seps, b))
-        G0 = 2 * n + self.gpos
-        blocks = []
-        for c, _, hit, E in ops:
-            M = np.zeros((len(rows), len(c)))
-            M[hit] = E
-            blocks.append((M, at[c]))
-        before = [_phase(at[rows], blocks, 0)]
+        before = [_phase(at[rows], [(hit, at[c], E) for c, _, hit, E in ops], 0)]
         if len(seps):
-            before.append(_phase(at[b], [(Eb, at[seps])], 0))
+            before.append(_phase(at[b], [(np.arange(len(b)), at[seps], Eb)], 0))
         B = _native.SLICE_BLOCK
-        g = self.gpos[b]
-        after = [_phase(n + at[b], [(self.Sinv[g], G0[self.gamma])], B)]
+        after = [_phase(n + at[b], [(np.arange(len(b)), 2 * n + np.arange(len(self.gamma)), self.Sinv[self.gpos[b]])], B)]
         if len(seps):
-            after.append(_phase(n + at[seps], [(Sl, at[seps]), (-Eb.T, n + at[b])], B))
-        cell_rows, row0 = np.concatenate([c for c, _, _, _ in ops]), 0
-        cb = []
+            i = np.arange(len(seps))
+            after.append(_phase(n + at[seps], [(i, at[seps], Sl), (i, n + at[b], -Eb.T)], B))
+        cell_rows, row0, blocks = np.concatenate([c for c, _, _, _ in ops]), 0, []
         for c, inv, hit, E in ops:
-            M = np.zeros((len(cell_rows), len(c)))
-            M[row0:row0 + len(c)] = inv
-            cb.append((M, at[c]))
-            M = np.zeros((len(cell_rows), len(hit)))
-            M[row0:row0 + len(c)] = -E.T
-            cb.append((M, n + at[rows[hit]]))
+            i = row0 + np.arange(len(c))
+            blocks += [(i, at[c], inv), (i, n + at[rows[hit]], -E.T)]
             row0 += len(c)
-        after.append(_phase(n + at[cell_rows], cb, B))
+        after.append(_phase(n + at[cell_rows], blocks, B))
         return before, after
 
     def _programs(self):
