@@ -20,6 +20,7 @@ import numpy as np
 import scipy.sparse
 
 from .device_linalg import cut_solver, cycle_solver, _torch
+from .time_evolution import _steps
 
 # device memory one chunk of selected steps may take (bytes)
 CHUNK_BYTES = 1 << 30
@@ -112,13 +113,15 @@ class DeviceQueries:
         (N, W, S) device tensor)."""
         tps = np.flatnonzero(self.problem._to_time_point_mask(select_time_points))
         W = self.problem.get_problem_count()
-        out = np.zeros((N, W, len(tps)))
         if len(tps) == 0:
-            return out
+            return np.zeros((N, W, 0))
         idx = self.res._time_point_index(tps)
         c = self.circuit
         per_step = 8 * W * (4 * max(c._Nn(), c._Nj(), c._Nf()) + 2 * c._Nj())
         step = max(1, int(CHUNK_BYTES // max(per_step, 1)))
+        if step >= len(tps):
+            return func(tps, idx).contiguous().cpu().numpy()
+        out = np.empty((N, W, len(tps)))
         for s0 in range(0, len(tps), step):
             sl = slice(s0, s0 + step)
             out[:, :, sl] = func(tps[sl], idx[sl]).cpu().numpy()
@@ -133,7 +136,7 @@ class DeviceQueries:
     # ------------------------------------------------------------ queries
     def phase(self, theta, tps, idx):
         Nj, W, S = theta.shape[0], theta.shape[1], len(idx)
-        th = self._dev(theta[:, :, idx]).reshape(Nj, W * S)
+        th = self._dev(_steps(theta, idx)).reshape(Nj, W * S)
         return self._msq(self.M()(th)).reshape(-1, W, S)
 
     def potential(self, voltage, tps, idx):
@@ -152,7 +155,7 @@ class DeviceQueries:
         """The relation's integral Ic sum_k a_k (1 - cos(k theta)) / k, in the
         operation order of FourierCPR (Ic (1 - cos theta) for the default)."""
         torch = self.torch
-        th = self._dev(theta[:, :, idx])
+        th = self._dev(_steps(theta, idx))
         Ic = self._dev(self.circuit._Ic())[:, None, None]
         n, a = self._series()
         if n == 0:
@@ -164,7 +167,7 @@ class DeviceQueries:
 
     def supercurrent(self, theta, tps, idx):
         torch = self.torch
-        th = self._dev(theta[:, :, idx])
+        th = self._dev(_steps(theta, idx))
         Ic = self._dev(self.circuit._Ic())[:, None, None]
         n, a = self._series()
         if n == 0:
@@ -177,21 +180,21 @@ class DeviceQueries:
     def cycle_current(self, current, tps, idx):
         Nj, W, S = current.shape[0], current.shape[1], len(idx)
         Is = self._dev(_input_at(self.problem.current_sources, Nj, W, tps))
-        d = (self._dev(current[:, :, idx]) - Is).reshape(Nj, W * S)
+        d = (self._dev(_steps(current, idx)) - Is).reshape(Nj, W * S)
         return self.cycle().solve(self.A()(d)).reshape(-1, W, S)
 
     def flux(self, current, tps, idx):
         Nj, W, S = current.shape[0], current.shape[1], len(idx)
         f = self._dev(_input_at(self.problem.external_flux, self.circuit._Nf(), W, tps))
-        LI = self.L()(self._dev(current[:, :, idx]).reshape(Nj, W * S))
+        LI = self.L()(self._dev(_steps(current, idx)).reshape(Nj, W * S))
         return f + (self.A()(LI) / (2 * np.pi)).reshape(-1, W, S)
 
     def magnetic_energy(self, current, tps, idx):
         Nj, W, S = current.shape[0], current.shape[1], len(idx)
-        I2 = self._dev(current[:, :, idx]).reshape(Nj, W * S) ** 2
+        I2 = self._dev(_steps(current, idx)).reshape(Nj, W * S) ** 2
         return self.L(0.5)(I2).reshape(Nj, W, S)
 
     def capacitive_energy(self, voltage, tps, idx):
-        V = self._dev(voltage[:, :, idx])
+        V = self._dev(_steps(voltage, idx))
         Ch = self._dev(0.5 * self.circuit._C())[:, None, None]
         return Ch * V ** 2
