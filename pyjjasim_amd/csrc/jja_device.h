@@ -205,23 +205,30 @@ __device__ __forceinline__ void normal_pair(uint64_t seed, uint32_t j, uint32_t 
   for (int r = 0; r < 10; ++r) {
     const uint64_t p0 = static_cast<uint64_t>(0xD2511F53u) * c0;
     const uint64_t p1 = static_cast<uint64_t>(0xCD9E8D57u) * c2;
-    const uint32_t n0 = static_cast<uint32_t>(p1 >> 32) ^ c1 ^ k0;
-    const uint32_t n2 = static_cast<uint32_t>(p0 >> 32) ^ c3 ^ k1;
+    // a ^ b ^ c in one instruction
+    c0 = __builtin_amdgcn_bitop3_b32(static_cast<uint32_t>(p1 >> 32), c1, k0, 0x96);
+    c2 = __builtin_amdgcn_bitop3_b32(static_cast<uint32_t>(p0 >> 32), c3, k1, 0x96);
     c1 = static_cast<uint32_t>(p1);
     c3 = static_cast<uint32_t>(p0);
-    c0 = n0;
-    c2 = n2;
     k0 += 0x9E3779B9u;
     k1 += 0xBB67AE85u;
   }
-  const uint64_t a = ((static_cast<uint64_t>(c1) << 32) | c0) >> 11;
-  const uint64_t b = ((static_cast<uint64_t>(c3) << 32) | c2) >> 11;
-  const double u1 = static_cast<double>(a + 1) * 0x1.0p-53;
-  const double u2 = static_cast<double>(b) * 0x1.0p-53;
-  const double rho = sqrt(-2.0 * log(u1));
-  const double ang = kTwoPi * u2;
+  // u1 = (a + 1) 2^-53 and u2 = b 2^-53, a and b the upper 53 bits of (c1, c0) and
+  // (c3, c2): all sums below are exact
+  const double k53 = JJA_K(0x1.0p-53), k32 = JJA_K(0x1.0p-32);
+  const double u1 = fma(static_cast<double>(c1), k32, fma(static_cast<double>(c0 >> 11), k53, k53));
+  const double u2 = fma(static_cast<double>(c3), k32, static_cast<double>(c2 >> 11) * k53);
+  // sqrt(-2 log u1) by Goldschmidt's iteration from the estimate of its reciprocal
+  // root; u1 = 1 gives 1e-150 for 0
+  const double x = fmax(2.0 * jja_neg_log(u1), 1e-300);
+  const double e = __builtin_amdgcn_rsq(x);
+  double g = x * e, h = 0.5 * e;
+  const double c = fma(-h, g, 0.5);
+  g = fma(g, c, g);
+  h = fma(h, c, h);
+  const double rho = fma(fma(-g, g, x), h, g);
   double sn, cs;
-  jja_sincos(ang, &sn, &cs);  // one argument reduction for both
+  jja_sincos_turn(u2, &sn, &cs);
   *z0 = rho * cs;
   *z1 = rho * sn;
 }
