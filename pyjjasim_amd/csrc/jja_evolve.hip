@@ -39,6 +39,7 @@
 #include "jja_device.h"
 #include "jja_domain.h"
 #include "jja_resident.h"
+#include "jja_wide.h"
 #include "jja_slab.h"
 
 // Device scratch of jja_solve_noalloc (a global face store for its columns):
@@ -266,6 +267,10 @@ struct Plan {
   int64_t parts_lds = 0;
   bool parts_only = false;           // subdomains: there is no other way to solve
   uint32_t parts_seq = 0;
+  // every problem's tables for the kernel that holds a large lattice column in the
+  // registers of one workgroup, or NULL; its dynamic LDS bytes
+  const WideDev* d_wide = nullptr;
+  int64_t wide_lds = 0;
   int64_t split_lds = 0;             // split launches: dynamic LDS bytes (part-local lattice solves)
   // what the device copies of the launch descriptors hold: a launch uploads
   // only what changed since the previous one
@@ -356,6 +361,38 @@ int create_slabs(Plan* plan, const jja_problem_desc& d) {
   plan->parts_adjoint = slab_adjoint_kernel(per);
   plan->parts_lds = 8 * slab_lds_doubles(h.d, d.lattice_cols);
   return JJA_OK;
+}
+
+// The tables of jja_wide.hip, where every problem of the plan takes that form: lattices
+// whose padded four-product solve does not fit in LDS. Where that fits, the kernel with
+// its phases in memory is the faster one (one column a CU, 200 columns with noise: 57x57
+// 26.2 us a step against 30.2, 64x64 30.8 against 32.1); where it does not, this one
+// (72x72 39.1 against 50.8, 100x100 62.9 against 83.8).
+int create_wide(Plan* plan, const jja_problem_desc* descs, int32_t n) {
+  if (plan->parts != 1 || plan->stencil_width != 3 || plan->block_size <= kResidentBlock) return JJA_OK;
+  std::vector<WideHost> h(n);
+  int64_t lds = 0;
+  for (int32_t i = 0; i < n; ++i) {
+    if (!descs[i].lattice_rows || plan->problems[i].lat_ld || plan->problems[i].index_bytes != 2 ||
+        !build_wide(descs[i], plan->lds_limit, &h[i]))
+      return JJA_OK;
+    lds = std::max(lds, 8 * wide_lds_doubles(h[i].d, descs[i].n_junctions));
+  }
+  std::vector<WideDev> dev(n);
+  for (int32_t i = 0; i < n; ++i) {
+    WideHost& v = h[i];
+    const std::vector<double> table = dst_table(descs[i].lattice_cols);
+    int rc;
+    if ((rc = upload(plan, v.junc_code.data(), v.junc_code.size(), &v.d.junc_code))) return rc;
+    if ((rc = upload(plan, v.face_code.data(), v.face_code.size(), &v.d.face_code))) return rc;
+    if ((rc = upload(plan, table.data(), table.size(), &v.d.table))) return rc;
+    if ((rc = upload(plan, v.inv.data(), v.inv.size(), &v.d.inv))) return rc;
+    if ((rc = upload(plan, v.spike.data(), v.spike.size(), &v.d.spike))) return rc;
+    if ((rc = upload(plan, v.reduced.data(), v.reduced.size(), &v.d.reduced))) return rc;
+    dev[i] = v.d;
+  }
+  plan->wide_lds = lds;
+  return upload(plan, dev.data(), dev.size(), &plan->d_wide);
 }
 
 // The subdomains of a problem that has them (validated).
@@ -861,6 +898,35 @@ int launch_resident_adjoint(Plan* plan, int32_t n, int form, int64_t lds, int64_
                          k_lo);
 }
 
+// Those also take the default current-phase relation alone, and inputs that are one
+// value for all junctions or lie one after the other.
+bool wide_runs(const Plan* plan, const jja_problem_run* runs) {
+  if (!plan->d_wide || !resident_runs(plan, runs)) return false;
+  auto plain = [](const jja_source& s) { return s.zero || s.s_i == 0 || s.s_i == 1; };
+  for (size_t p = 0; p < plan->problems.size(); ++p)
+    if (plan->problems[p].cpr_terms || !plain(runs[p].Is) || !plain(runs[p].f) || (!runs[p].T.zero && !plain(runs[p].sigma))) return false;
+  return true;
+}
+
+int launch_wide(Plan* plan, const jja_problem_run* host_runs, int32_t n, int32_t n_steps, int64_t step0,
+                hipStream_t stream) {
+  bool gauss = false, uniform = true;
+  for (size_t p = 0; p < plan->problems.size(); ++p) {
+    const bool noisy = !host_runs[p].T.zero;
+    gauss = gauss || noisy;
+    uniform = uniform && plan->problems[p].coef_si == 0 && (!noisy || host_runs[p].sigma.s_i == 0);
+  }
+  const void* kern = wide_evolve_kernel(gauss, uniform);
+  if (int rc = set_lds_limit(plan, kern, static_cast<int>(plan->wide_lds))) return rc;
+  const DevProblem* probs = plan->d_problems;
+  const jja_problem_run* runs = plan->d_runs;
+  const WorkItem* work = plan->d_work;
+  const WideDev* tables = plan->d_wide;
+  void* argv[] = {&probs, &runs, &work, &tables, &n_steps, &step0};
+  JJA_HIP(hipLaunchKernel(kern, dim3(n), dim3(kWideBlock), argv, static_cast<size_t>(plan->wide_lds), stream));
+  return JJA_OK;
+}
+
 template <int STORE>
 int launch_evolve_bs(Plan* plan, const WorkItem* work, int32_t n, int64_t lds, int32_t n_steps,
                      int64_t step0, hipStream_t stream) {
@@ -1308,6 +1374,7 @@ int jja_plan_create(int32_t n_problems, const jja_problem_desc* descs, jja_plan*
     plan->ctr_cap = 2 * items;
   }
   if (rc == JJA_OK && n_problems == 1) rc = descs[0].domains ? create_domains(plan, descs[0]) : create_slabs(plan, descs[0]);
+  if (rc == JJA_OK) rc = create_wide(plan, descs, n_problems);
   if (rc == JJA_OK && hipEventCreateWithFlags(&plan->done, hipEventDisableTiming) != hipSuccess)
     rc = fail(JJA_EHIP, "jja_plan_create: hipEventCreateWithFlags failed");
   if (rc == JJA_OK && plan->parts > 1) {
@@ -1437,6 +1504,8 @@ int jja_evolve(jja_plan* p, const jja_problem_run* runs, int32_t n_steps, int64_
     const int form = n_g == 0 && resident_runs(plan, runs) ? resident_layout(plan, &resident_lds) : -1;
     if (form >= 0)
       rc = launch_resident_evolve(plan, n, form, resident_lds, n_steps, step0, stream);
+    else if (n_g == 0 && wide_runs(plan, runs))
+      rc = launch_wide(plan, runs, n, n_steps, step0, stream);
     else if (n_g == 0)
       rc = launch_evolve_bs<0>(plan, plan->d_work, n, lds, n_steps, step0, stream);
     else if (n_lds == 0)

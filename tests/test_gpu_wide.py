@@ -1,0 +1,46 @@
+"""Large lattice columns held in the registers of one workgroup (taken for the usual
+step of lattices that leave no room in LDS for the padded solve) against the kernel of
+512 threads, at 1e-9 of the phase scale with identical vortex counts."""
+import numpy as np
+import pytest
+
+import pyjjasim_amd as pa
+
+pytestmark = pytest.mark.gpu
+
+# the smallest; an odd count of junctions in the first round (a pair across both), both
+# ways; an odd junction count; long sides both ways (15 row parts a mode); the largest
+SIZES = [(66, 66), (70, 71), (71, 70), (72, 72), (34, 261), (261, 34), (120, 70), (60, 128), (99, 100), (100, 100)]
+
+
+def _run(c, block_size, W, Nt, T, beta_time, **kw):
+    t = 0.05 * np.arange(Nt)
+    drive = pa.SeparableSource(c.current_base(0.0)[:, None] * np.linspace(0.5, 1.3, W), 1.0 + 0.3 * np.sin(t))
+    f = 0.1 + 0.02 * np.arange(c.face_count())[:, None, None] / c.face_count() + 0.01 * np.sin(t)[None, None, :]
+    if beta_time:
+        T = T * (1.0 + 0.5 * np.cos(t))[None, None, :] * np.ones((c.junction_count(), 1, 1))
+    return pa.TimeEvolutionProblem(c, solver="lattice", parts=1, block_size=block_size, time_step=0.05,
+                                   time_step_count=Nt, external_flux=f, current_sources=drive, temperature=T, seed=3,
+                                   store_time_steps=[0, 5, 17, Nt - 1], steps_per_launch=13, **kw).compute()
+
+
+def _compare(a, b):
+    for get in ("get_theta", "get_current", "get_voltage"):
+        u, v = getattr(a, get)(), getattr(b, get)()
+        assert np.abs(u - v).max() <= 1e-9 * np.abs(u).max(), get
+    np.testing.assert_array_equal(a.get_vortex_configuration(), b.get_vortex_configuration())
+
+
+@pytest.mark.parametrize("n,m", SIZES)
+@pytest.mark.parametrize("aniso,beta_l,T,beta_time", [(False, 0.0, 0.02, False), (True, 0.5, 0.0, False),
+                                                      (True, 0.0, 0.02, True)])
+def test_gpu_wide_matches(n, m, aniso, beta_l, T, beta_time):
+    c = pa.SquareArray(n, m)
+    x1, y1, x2, y2 = c.get_junction_coordinates()
+    c.set_capacitance(np.where(y1 == y2, 1.0, 2.0) if aniso else 1.0)
+    if beta_l:
+        c.set_inductance(beta_l)
+    rng = np.random.default_rng(n + m)
+    c.set_critical_current(np.exp(0.1 * rng.standard_normal(c.junction_count())))
+    print(f"[wide] {n}x{m} T={T}", flush=True)
+    _compare(_run(c, 512, 2, 36, T, beta_time), _run(c, 1024, 2, 36, T, beta_time))
