@@ -165,6 +165,12 @@ __device__ __forceinline__ int32_t opaque_zero() {
   return z;
 }
 
+// A value at a byte offset from a wave-uniform base.
+template <class T>
+__device__ __forceinline__ T at_offset(const GAS T* base, uint32_t bytes) {
+  return *reinterpret_cast<const GAS T*>(reinterpret_cast<const GAS char*>(base) + bytes);
+}
+
 // 16-bit incidence codes (2 * address + sign, 0xffff empty) of the kernels that
 // keep them in registers, two to a word: +-v by the sign bit, 0 for an empty slot
 __device__ __forceinline__ double signed_value(double v, uint32_t code) {

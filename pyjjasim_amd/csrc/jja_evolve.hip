@@ -346,7 +346,7 @@ int create_slabs(Plan* plan, const jja_problem_desc& d) {
   if ((rc = upload(plan, h.inv.data(), h.inv.size(), &h.d.inv))) return rc;
   if ((rc = upload(plan, h.spike.data(), h.spike.size(), &h.d.spike))) return rc;
   if ((rc = upload(plan, h.reduced.data(), h.reduced.size(), &h.d.reduced))) return rc;
-  const std::vector<double> ends(static_cast<size_t>(d.max_columns) * 4 * plan->parts * d.lattice_cols, 0.0);
+  const std::vector<double> ends(static_cast<size_t>(d.max_columns) * 2 * h.d.ends_rows * d.lattice_cols, 0.0);
   const std::vector<uint32_t> flags(static_cast<size_t>(d.max_columns) * plan->parts * h.d.mode_waves, 0u);
   const double* e = nullptr;
   const uint32_t* f = nullptr;

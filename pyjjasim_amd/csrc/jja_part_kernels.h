@@ -24,21 +24,21 @@ struct PartFace {
 
 template <int W>
 __device__ __forceinline__ PartFace<W> part_face(const PartTables& T, int32_t part, int32_t slot) {
+  // loaded without a branch (a slot past the last reads the last), so that the loads of
+  // all slots are in flight together
   PartFace<W> f;
+  const int64_t at = static_cast<int64_t>(part) * T.faces + min(slot, T.faces - 1);
 #pragma unroll
-  for (int i = 0; i < W; ++i) f.code[i] = 0xffffffffu;
-  f.at = 0xffffffffu;
-  f.id = -1;
-  if (slot < T.faces) {
-    const int64_t at = static_cast<int64_t>(part) * T.faces + slot;
-#pragma unroll
-    for (int i = 0; i < W; i += 2) {
-      const vuint2 c = gbl(reinterpret_cast<const vuint2*>(T.face_code + W * at + i))[0];
-      f.code[i] = c.x;
-      f.code[i + 1] = c.y;
-    }
-    f.at = gbl(T.face_at)[at];
-    f.id = gbl(T.face_id)[at];
+  for (int i = 0; i < W; i += 2) {
+    const vuint2 c = gbl(reinterpret_cast<const vuint2*>(T.face_code + W * at + i))[0];
+    f.code[i] = c.x;
+    f.code[i + 1] = c.y;
+  }
+  f.at = gbl(T.face_at)[at];
+  f.id = gbl(T.face_id)[at];
+  if (slot >= T.faces) {
+    f.at = 0xffffffffu;
+    f.id = -1;
   }
   return f;
 }
@@ -175,14 +175,15 @@ __global__ __launch_bounds__(kPartBlock) void evolve_parts_kernel(const DevProbl
       for (int k = 0; k < NF; ++k) {
         if constexpr (!KEEP) face[k] = part_face<FW>(S, part, k * BS + tid);
         fq[k] = KEEP ? fx[k] * fv.amp : 0.0;
-        if (!keep_f) fq[k] = face[k].id >= 0 ? term_at(fv, face[k].id) : 0.0;
+        if (!keep_f) fq[k] = term_at(fv, max(face[k].id, 0));  // used by faces that have one
       }
       typename Solver::Head head;
       solver.head(S, tid, head);
       lds_barrier();
 #pragma unroll
       for (int k = 0; k < NF; ++k)
-        if (face[k].at != 0xffffffffu) face_in[face[k].at] = face_sum(face[k], U) - kTwoPi * fq[k];
+        if (face[k].at != 0xffffffffu)
+          face_in[face[k].at] = face_sum(face[k], U) - (face[k].id >= 0 ? kTwoPi * fq[k] : 0.0);
       lds_barrier();
       solver.solve(P, S, seq0 + 1u + static_cast<uint32_t>(n), tid, BS, head);
     }

@@ -23,11 +23,12 @@ struct SlabDev : PartTables {
   int32_t table_lds;                     // the sine table lies in LDS (else it is read from memory)
   int32_t mode_waves;                    // waves that hold the modes (two lanes each)
   int32_t inv_lds;                       // the pivots lie in LDS
+  int32_t ends_rows;                     // 2 parts rounded up to a multiple of four
   const double* table;                   // sine table of C modes (DstShape)
   const double* inv;                     // [rows][C] inverse pivots of a part's own block
   const double* spike;                   // [2][rows][C]: response to the row below, parts of base and base + 1 rows
-  const double* reduced;                 // [2 parts][2 parts][C]: first and last rows of the parts from their own blocks'
-  double* ends;                          // [columns][2][parts][2][C] end rows of a step
+  const double* reduced;                 // [2 parts][ends_rows][C]: first and last rows of the parts from their own blocks'
+  double* ends;                          // [columns][2][ends_rows][C] end rows of a step, two of a part
   uint32_t* flags;                       // [columns][parts][mode_waves] sequence number of the last end rows
 };
 

@@ -28,6 +28,7 @@
 #include <algorithm>
 
 #include "jja_part_kernels.h"
+#include "jja_rowdst.h"
 #include "jja_rowparts.h"
 
 namespace {
@@ -105,6 +106,23 @@ __device__ __forceinline__ void slab_transform(const LAS double* src, LAS double
   }
 }
 
+// An end row's value as another part published it.
+__device__ __forceinline__ double end_row(const GAS double* at) {
+  return __builtin_bit_cast(
+      double, __hip_atomic_load(reinterpret_cast<unsigned long long*>(const_cast<double*>((const double*)at)),
+                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+
+// AHEAD: the reduced system's first coefficients and the responses are loaded before the
+// wait for the other parts, and eight end rows at once after it. With nine pairs a thread
+// (large lattices, 255 modes: four rows of 32 coefficients a mode) that shortens wait and
+// reduced system from 48,000 to 33,000 cycles; with few modes the loads only delay the
+// polls (one 100x100 column in 16 parts: 16.5 us a step against 17.6), and four end rows
+// at a time with their coefficients are enough. A table in memory then also takes
+// row_transform, which reads it once for a slab's 16 rows and the border rows (both
+// transforms together 57,000 cycles before, 40,000 now); the kernels with few pairs keep
+// their inputs in the registers that it needs.
+template <bool AHEAD>
 struct SlabSolver {
   using Dev = SlabDev;
   static constexpr int kFaceWords = 2;
@@ -112,7 +130,7 @@ struct SlabSolver {
   LAS double *in, *out, *u;       // face rows Z (both); junction values in the rows' transform Y
   LAS double* inv;                // pivots
   const LAS double* table;
-  GAS double* ends;               // this column's [2][parts][2][C]
+  GAS double* ends;               // this column's [2][ends_rows][C]
   uint32_t* flags;                // this column's [parts][mode_waves]
   uint32_t wait_limit;
   int32_t* err;
@@ -130,7 +148,7 @@ struct SlabSolver {
     table = next;
     const int32_t entries = S.table_lds ? DstShape(C).entries() : 0;
     stopped = (volatile LAS int32_t*)(next + entries);
-    ends = gblw(S.ends) + column * (4 * parts * static_cast<int64_t>(C));
+    ends = gblw(S.ends) + column * (2 * S.ends_rows * static_cast<int64_t>(C));
     flags = S.flags + column * (parts * S.mode_waves);
     for (int32_t i = tid; i < S.buf + max(S.buf, 2 * S.pairs); i += nt) in[i] = 0.0;
     if (S.inv_lds)
@@ -149,15 +167,19 @@ struct SlabSolver {
 // K^-1 of the column's face sums: in rows 1 .. s on entry, the solution in rows
 // 0 .. s + 1 on exit (a neighbour's row below the first or above the last face row
 // is zero). seq: the step's sequence number.
-__device__ __forceinline__ void SlabSolver::solve(const DevProblem& P, const SlabDev& S, uint32_t seq, int32_t tid,
+template <bool AHEAD>
+__device__ __forceinline__ void SlabSolver<AHEAD>::solve(const DevProblem& P, const SlabDev& S, uint32_t seq, int32_t tid,
                                                   int32_t nt, Head&) const {
-  constexpr int TB = 8;  // rows or terms loaded together
+  constexpr int TB = 8;                // rows loaded together
+  constexpr int RB = 4;                // end rows whose coefficients are loaded together
   const int32_t G = parts;
   LAS double *const Z = in, *const Y = u;
   if (S.table_lds)
-    slab_transform<const LAS double*>(Z, Y, table, C, s + 2, ld, tid, nt);
+    slab_transform<const LAS double*>(Z + ld, Y + ld, table, C, s, ld, tid, nt);
+  else if constexpr (AHEAD)
+    row_transform<false>(Z + ld, Y + ld, gbl(S.table), C, s, ld, tid, nt);
   else
-    slab_transform<const GAS double*>(Z, Y, gbl(S.table), C, s + 2, ld, tid, nt);
+    slab_transform<const GAS double*>(Z + ld, Y + ld, gbl(S.table), C, s, ld, tid, nt);
   lds_barrier();
   const int32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid & (kWave - 1);
   if (wave < S.mode_waves) {
@@ -203,7 +225,7 @@ __device__ __forceinline__ void SlabSolver::solve(const DevProblem& P, const Sla
         }
     }
     // publish the end rows, wait for the other parts'
-    const int64_t step = (seq & 1u) ? 2 * static_cast<int64_t>(G) * C : 0;
+    const int64_t step = (seq & 1u) ? static_cast<int64_t>(S.ends_rows) * C : 0;
     GAS double* e = ends + step + k;
     if (live)
       __hip_atomic_store(reinterpret_cast<unsigned long long*>((double*)(e + (2 * part + side) * C)),
@@ -214,6 +236,38 @@ __device__ __forceinline__ void SlabSolver::solve(const DevProblem& P, const Sla
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     if (lane == 0)
       __hip_atomic_store(flags + part * S.mode_waves + wave, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // the reduced system's coefficients (zero past the last end row) and the responses
+    const int32_t outer = side ? 2 * part + 2 : 2 * part - 1, own = 2 * part + side;
+    const bool edge = outer < 0 || outer >= 2 * G;  // beyond the lattice: zero
+    const int32_t E = S.ends_rows;
+    const uint32_t at_outer = 8u * static_cast<uint32_t>((edge ? own : outer) * E * C + k);
+    const uint32_t at_own = 8u * static_cast<uint32_t>(own * E * C + k), at_mode = 8u * static_cast<uint32_t>(k);
+    struct Chunk {
+      double outer[RB], own[RB];
+    } c[2];
+    auto coefficients = [&](Chunk& to, int32_t i0) __attribute__((always_inline)) {
+      i0 = min(i0, E - RB);
+#pragma unroll
+      for (int q = 0; q < RB; ++q) {
+        to.outer[q] = at_offset(gbl(S.reduced) + (i0 + q) * C, at_outer);
+        to.own[q] = at_offset(gbl(S.reduced) + (i0 + q) * C, at_own);
+      }
+    };
+    const GAS double* V = gbl(S.spike) + (s > S.base ? static_cast<int64_t>(S.rows) * C : 0);
+    double va[TB], vb[TB];
+    auto responses = [&](int32_t l0) __attribute__((always_inline)) {
+#pragma unroll
+      for (int q = 0; q < TB; ++q) {
+        const int32_t l = min(l0 + side + 2 * q, s - 1);
+        va[q] = V[l * C + k];
+        vb[q] = V[(s - 1 - l) * C + k];
+      }
+    };
+    if constexpr (AHEAD) {
+      coefficients(c[0], 0);
+      coefficients(c[1], RB);
+      responses(1);
+    }
     if (!*stopped) {
       const uint32_t* f = flags + min(lane, G - 1) * S.mode_waves + wave;
       uint32_t spins = 0;
@@ -235,52 +289,69 @@ __device__ __forceinline__ void SlabSolver::solve(const DevProblem& P, const Sla
     // first of the part above. Both neighbours form a row by the same sum, so the
     // junctions between two parts, which both keep, see the same bits in both (with
     // bits of their own the copies would drift apart like two separate junctions).
-    const int32_t outer = side ? 2 * part + 2 : 2 * part - 1, own = 2 * part + side;
-    const bool edge = outer < 0 || outer >= 2 * G;  // beyond the lattice: zero
-    const GAS double* ro = gbl(S.reduced) + static_cast<int64_t>(edge ? own : outer) * 2 * G * C + k;
-    const GAS double* rw = gbl(S.reduced) + static_cast<int64_t>(own) * 2 * G * C + k;
     double no = 0.0, nw = 0.0;
-    for (int32_t i0 = 0; i0 < 2 * G; i0 += 4) {
-      double ev[4], co[4], cw[4];
+    if constexpr (AHEAD) {
+      for (int32_t i0 = 0; i0 < E; i0 += 2 * RB) {
+        double ev[2 * RB];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        ev[q] = __builtin_bit_cast(
-            double, __hip_atomic_load(reinterpret_cast<unsigned long long*>((double*)(e + (i0 + q) * C)), __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT));
-        co[q] = ro[(i0 + q) * C];
-        cw[q] = rw[(i0 + q) * C];
-      }
+        for (int q = 0; q < 2 * RB; ++q) ev[q] = end_row(e + min(i0 + q, E - 1) * C);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        no = __builtin_fma(co[q], ev[q], no);
-        nw = __builtin_fma(cw[q], ev[q], nw);
+        for (int h = 0; h < 2; ++h) {
+          if (i0 + h * RB < E) {
+#pragma unroll
+            for (int q = 0; q < RB; ++q) {
+              no = __builtin_fma(c[h].outer[q], ev[h * RB + q], no);
+              nw = __builtin_fma(c[h].own[q], ev[h * RB + q], nw);
+            }
+            coefficients(c[h], i0 + (h + 2) * RB);
+          }
+        }
       }
+    } else {
+      const GAS double* ro = gbl(S.reduced) + static_cast<int64_t>(edge ? own : outer) * E * C + k;
+      const GAS double* rw = gbl(S.reduced) + static_cast<int64_t>(own) * E * C + k;
+      for (int32_t i0 = 0; i0 < E; i0 += RB) {
+        double ev[RB], co[RB], cw[RB];
+#pragma unroll
+        for (int q = 0; q < RB; ++q) {
+          ev[q] = end_row(e + (i0 + q) * C);
+          co[q] = ro[(i0 + q) * C];
+          cw[q] = rw[(i0 + q) * C];
+        }
+#pragma unroll
+        for (int q = 0; q < RB; ++q) {
+          no = __builtin_fma(co[q], ev[q], no);
+          nw = __builtin_fma(cw[q], ev[q], nw);
+        }
+      }
+      responses(1);
     }
     if (edge) no = 0.0;
     const double swapped = dpp_f64<0xB1, 0xf>(no);  // quad_perm [1, 0, 3, 2]: the mode's other lane
     const double below = side ? swapped : no, above = side ? no : swapped;
-    const GAS double* V = gbl(S.spike) + (s > S.base ? static_cast<int64_t>(S.rows) * C : 0) + k;
-    for (int32_t l0 = 1 + side; l0 < s - 1; l0 += 2 * TB) {
-      double v[TB], va[TB], vb[TB];
+    for (int32_t l0 = 1; l0 + side < s - 1; l0 += 2 * TB) {
+      double v[TB];
+#pragma unroll
+      for (int q = 0; q < TB; ++q) v[q] = y[min(l0 + side + 2 * q, s - 1) * ld];
 #pragma unroll
       for (int q = 0; q < TB; ++q) {
-        const int32_t l = min(l0 + 2 * q, s - 1);
-        v[q] = y[l * ld];
-        va[q] = V[l * C];
-        vb[q] = V[(s - 1 - l) * C];
+        const int32_t l = l0 + side + 2 * q;
+        if (l < s - 1) y[l * ld] = __builtin_fma(va[q], below, __builtin_fma(vb[q], above, v[q]));
       }
-#pragma unroll
-      for (int q = 0; q < TB; ++q)
-        if (l0 + 2 * q < s - 1) y[(l0 + 2 * q) * ld] = __builtin_fma(va[q], below, __builtin_fma(vb[q], above, v[q]));
+      if (l0 + 2 * TB < s - 1) responses(l0 + 2 * TB);
     }
     y[(side ? s - 1 : 0) * ld] = nw;
     Y[(side ? s + 1 : 0) * ld + k] = no;
   }
-  lds_barrier();
-  if (S.table_lds)
-    slab_transform<const LAS double*>(Y, Z, table, C, s + 2, ld, tid, nt);
-  else
-    slab_transform<const GAS double*>(Y, Z, gbl(S.table), C, s + 2, ld, tid, nt);
+  if (AHEAD && !S.table_lds) {
+    row_transform<true>(Y, Z, gbl(S.table), C, s + 2, ld, tid, nt);
+  } else {
+    lds_barrier();
+    if (S.table_lds)
+      slab_transform<const LAS double*>(Y, Z, table, C, s + 2, ld, tid, nt);
+    else if constexpr (!AHEAD)
+      slab_transform<const GAS double*>(Y, Z, gbl(S.table), C, s + 2, ld, tid, nt);
+  }
   lds_barrier();
 }
 
@@ -381,7 +452,13 @@ bool build_slabs(const jja_problem_desc& desc, int32_t parts, int64_t lds_bytes,
                                      static_cast<uint32_t>(fcode[4 * static_cast<size_t>(e) + 2 * i + 1]) << 16;
     }
   }
-  row_part_tables(R, C, G, desc.lattice_g, desc.lattice_gc, &out->inv, &out->spike, &out->reduced);
+  std::vector<double> reduced;
+  row_part_tables(R, C, G, desc.lattice_g, desc.lattice_gc, &out->inv, &out->spike, &reduced);
+  d.ends_rows = (2 * G + 3) / 4 * 4;
+  out->reduced.assign(2 * static_cast<size_t>(G) * d.ends_rows * C, 0.0);
+  for (int32_t r = 0; r < 2 * G; ++r)
+    std::copy_n(&reduced[2 * static_cast<size_t>(r) * G * C], 2 * static_cast<size_t>(G) * C,
+                &out->reduced[static_cast<size_t>(r) * d.ends_rows * C]);
   // LDS: the pivots, then the sine table, where there is room
   d.inv_lds = d.table_lds = 0;
   if (8 * slab_lds_doubles(d, C) > lds_bytes) return false;
@@ -393,17 +470,17 @@ bool build_slabs(const jja_problem_desc& desc, int32_t parts, int64_t lds_bytes,
 }
 
 const void* slab_evolve_kernel(int pairs) {
-  if (pairs <= 1) return reinterpret_cast<const void*>(evolve_parts_kernel<SlabSolver, 1>);
-  if (pairs <= 2) return reinterpret_cast<const void*>(evolve_parts_kernel<SlabSolver, 2>);
-  if (pairs <= 3) return reinterpret_cast<const void*>(evolve_parts_kernel<SlabSolver, 3>);
-  if (pairs <= 5) return reinterpret_cast<const void*>(evolve_parts_kernel<SlabSolver, 5>);
-  return pairs <= kSlabPairs ? reinterpret_cast<const void*>(evolve_parts_kernel<SlabSolver, kSlabPairs>) : nullptr;
+  if (pairs <= 1) return reinterpret_cast<const void*>(evolve_parts_kernel<SlabSolver<false>, 1>);
+  if (pairs <= 2) return reinterpret_cast<const void*>(evolve_parts_kernel<SlabSolver<false>, 2>);
+  if (pairs <= 3) return reinterpret_cast<const void*>(evolve_parts_kernel<SlabSolver<false>, 3>);
+  if (pairs <= 5) return reinterpret_cast<const void*>(evolve_parts_kernel<SlabSolver<false>, 5>);
+  return pairs <= kSlabPairs ? reinterpret_cast<const void*>(evolve_parts_kernel<SlabSolver<true>, kSlabPairs>) : nullptr;
 }
 
 const void* slab_adjoint_kernel(int pairs) {
-  if (pairs <= 1) return reinterpret_cast<const void*>(adjoint_parts_kernel<SlabSolver, 1>);
-  if (pairs <= 2) return reinterpret_cast<const void*>(adjoint_parts_kernel<SlabSolver, 2>);
-  if (pairs <= 3) return reinterpret_cast<const void*>(adjoint_parts_kernel<SlabSolver, 3>);
-  if (pairs <= 5) return reinterpret_cast<const void*>(adjoint_parts_kernel<SlabSolver, 5>);
-  return pairs <= kSlabPairs ? reinterpret_cast<const void*>(adjoint_parts_kernel<SlabSolver, kSlabPairs>) : nullptr;
+  if (pairs <= 1) return reinterpret_cast<const void*>(adjoint_parts_kernel<SlabSolver<false>, 1>);
+  if (pairs <= 2) return reinterpret_cast<const void*>(adjoint_parts_kernel<SlabSolver<false>, 2>);
+  if (pairs <= 3) return reinterpret_cast<const void*>(adjoint_parts_kernel<SlabSolver<false>, 3>);
+  if (pairs <= 5) return reinterpret_cast<const void*>(adjoint_parts_kernel<SlabSolver<false>, 5>);
+  return pairs <= kSlabPairs ? reinterpret_cast<const void*>(adjoint_parts_kernel<SlabSolver<false>, kSlabPairs>) : nullptr;
 }

@@ -22,13 +22,7 @@ namespace {
 
 typedef double vdouble16 __attribute__((ext_vector_type(16)));
 
-// A value at a byte offset from a wave-uniform base.
-template <class T>
-__device__ __forceinline__ T at_offset(const GAS T* base, uint32_t bytes) {
-  return *reinterpret_cast<const GAS T*>(reinterpret_cast<const GAS char*>(base) + bytes);
-}
-
-// The same for data that no other column reads: it does not displace the tables that
+// at_offset for data that no other column reads: it does not displace the tables that
 // all columns share from the L2.
 template <class T>
 __device__ __forceinline__ T stream_offset(const GAS T* base, uint32_t bytes) {
