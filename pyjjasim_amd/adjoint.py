@@ -112,6 +112,8 @@ class DifferentiableEvolution:
         results are invalid); waits for the launches of a split plan."""
         eng = self.eng
         if eng.host.parts > 1:
+            if self.torch.cuda.is_current_stream_capturing():
+                return  # a replay reports nothing; the next call outside the graph does
             self.torch.cuda.current_stream().synchronize()
         _native.check(eng.lib.jja_plan_status(eng.handle))
 

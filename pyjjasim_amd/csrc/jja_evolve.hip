@@ -259,14 +259,15 @@ struct Plan {
   int32_t n_cu = 0;                  // compute units of the device
   uint32_t wait_limit = kWaitLimit;  // split launches: polls before a column barrier gives up
   // columns in parts that keep their junctions on chip (one problem; row slabs or
-  // subdomains): the device tables and kernels, dynamic LDS doubles and the
-  // sequence number of the last step
+  // subdomains): the device tables and kernels, dynamic LDS doubles, and each
+  // part's sequence number of its last step [max_columns][parts], kept on the device
+  // so that a launch replayed from a graph counts on
   const void* d_parts = nullptr;
   const void* parts_evolve = nullptr;
   const void* parts_adjoint = nullptr;
   int64_t parts_lds = 0;
   bool parts_only = false;           // subdomains: there is no other way to solve
-  uint32_t parts_seq = 0;
+  uint32_t* d_parts_seq = nullptr;
   // every problem's tables for the kernel that holds a large lattice column in the
   // registers of one workgroup, or NULL; its dynamic LDS bytes
   const WideDev* d_wide = nullptr;
@@ -1032,6 +1033,13 @@ int launch_cooperative(Plan* plan, const void* kern, int BS, int32_t n, int64_t 
     return fail(JJA_EUNSUPPORTED, "split launch of " + std::to_string(n) + " workgroups; the device holds " +
                                       std::to_string(static_cast<int64_t>(per_cu) * plan->n_cu) + " at once");
   void* argv[] = {static_cast<void*>(&args)...};
+  // a graph takes the plain launch: its workgroups fit on the device together (above)
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  JJA_HIP(hipStreamIsCapturing(stream, &capture));
+  if (capture != hipStreamCaptureStatusNone) {
+    JJA_HIP(hipLaunchKernel(kern, dim3(n), dim3(BS), argv, static_cast<size_t>(lds), stream));
+    return JJA_OK;
+  }
   JJA_HIP(hipLaunchCooperativeKernel(kern, dim3(n), dim3(BS), argv, static_cast<size_t>(lds), stream));
   return JJA_OK;
 }
@@ -1069,11 +1077,8 @@ int launch_evolve_parts(Plan* plan, int32_t n, int32_t n_steps, int64_t step0, h
   const jja_problem_run* runs = plan->d_runs;
   const WorkItem* work = plan->d_work;
   const void* tables = plan->d_parts;
-  const uint32_t seq = plan->parts_seq;
-  const int rc = launch_cooperative(plan, plan->parts_evolve, plan->block_size, n, plan->parts_lds, stream, probs, runs,
-                                    work, tables, n_steps, step0, seq, plan->d_err, plan->wait_limit);
-  if (rc == JJA_OK) plan->parts_seq += static_cast<uint32_t>(n_steps);
-  return rc;
+  return launch_cooperative(plan, plan->parts_evolve, plan->block_size, n, plan->parts_lds, stream, probs, runs, work,
+                            tables, n_steps, step0, plan->d_parts_seq, plan->d_err, plan->wait_limit);
 }
 
 int launch_adjoint_parts(Plan* plan, int32_t n, int64_t k_hi, int64_t k_lo, hipStream_t stream) {
@@ -1081,11 +1086,8 @@ int launch_adjoint_parts(Plan* plan, int32_t n, int64_t k_hi, int64_t k_lo, hipS
   const jja_adjoint_run* runs = plan->d_adj;
   const WorkItem* work = plan->d_work;
   const void* tables = plan->d_parts;
-  const uint32_t seq = plan->parts_seq;
-  const int rc = launch_cooperative(plan, plan->parts_adjoint, plan->block_size, n, plan->parts_lds, stream, probs, runs,
-                                    work, tables, k_hi, k_lo, seq, plan->d_err, plan->wait_limit);
-  if (rc == JJA_OK) plan->parts_seq += static_cast<uint32_t>(k_hi - k_lo + 1);
-  return rc;
+  return launch_cooperative(plan, plan->parts_adjoint, plan->block_size, n, plan->parts_lds, stream, probs, runs, work,
+                            tables, k_hi, k_lo, plan->d_parts_seq, plan->d_err, plan->wait_limit);
 }
 
 template <int BS>
@@ -1374,6 +1376,12 @@ int jja_plan_create(int32_t n_problems, const jja_problem_desc* descs, jja_plan*
     plan->ctr_cap = 2 * items;
   }
   if (rc == JJA_OK && n_problems == 1) rc = descs[0].domains ? create_domains(plan, descs[0]) : create_slabs(plan, descs[0]);
+  if (rc == JJA_OK && plan->d_parts) {
+    const std::vector<uint32_t> seq(static_cast<size_t>(descs[0].max_columns) * plan->parts, 0u);
+    const uint32_t* d = nullptr;
+    rc = upload(plan, seq.data(), seq.size(), &d);
+    plan->d_parts_seq = const_cast<uint32_t*>(d);
+  }
   if (rc == JJA_OK) rc = create_wide(plan, descs, n_problems);
   if (rc == JJA_OK && hipEventCreateWithFlags(&plan->done, hipEventDisableTiming) != hipSuccess)
     rc = fail(JJA_EHIP, "jja_plan_create: hipEventCreateWithFlags failed");

@@ -5,7 +5,9 @@
 //   u    junction values the face sums read, by pair slot: 2 * slot + member
 //   in   face sums, written at the faces' addresses
 //   out  the solution, read at the junctions' codes and the faces' addresses
-// head() issues loads that solve() needs before the face sums.
+// head() issues loads that solve() needs before the face sums. seqs: every part's
+// sequence number of its last step; all parts of a column run the same steps, so they
+// agree, and each advances its own at the end of a launch.
 #ifndef JJA_PART_KERNELS_H
 #define JJA_PART_KERNELS_H
 
@@ -60,7 +62,7 @@ __global__ __launch_bounds__(kPartBlock) void evolve_parts_kernel(const DevProbl
                                                          const jja_problem_run* __restrict__ runs,
                                                          const WorkItem* __restrict__ work,
                                                          const typename Solver::Dev* __restrict__ tables, int32_t n_steps,
-                                                         int64_t step0, uint32_t seq0, int32_t* err,
+                                                         int64_t step0, uint32_t* seqs, int32_t* err,
                                                          uint32_t wait_limit) {
   extern __shared__ double lds[];
   constexpr int BS = kPartBlock, FW = Solver::kFaceWords;
@@ -75,6 +77,7 @@ __global__ __launch_bounds__(kPartBlock) void evolve_parts_kernel(const DevProbl
   const int64_t w = wi.column / S.parts;
   const int32_t tid0 = threadIdx.x, tid = tid0;
   const int32_t part = wi.column % S.parts;
+  const uint32_t seq0 = __builtin_amdgcn_readfirstlane(gbl(seqs)[wi.column]);  // before the solver's barrier
   const Solver solver(P, S, w, part, lds, err, wait_limit, tid, BS);
   LAS double *const U = solver.u, *const face_in = solver.in, *const face_out = solver.out;
   const int32_t Nj = P.Nj;
@@ -241,6 +244,7 @@ __global__ __launch_bounds__(kPartBlock) void evolve_parts_kernel(const DevProbl
       __builtin_amdgcn_sched_barrier(0);
     }
   }
+  if (threadIdx.x == 0) gblw(seqs)[wi.column] = seq0 + static_cast<uint32_t>(n_steps);
 }
 
 // The adjoint sweep (adjoint_steps) of a part: with few pairs a thread keeps
@@ -251,7 +255,7 @@ __global__ __launch_bounds__(kPartBlock) void adjoint_parts_kernel(const DevProb
                                                           const jja_adjoint_run* __restrict__ runs,
                                                           const WorkItem* __restrict__ work,
                                                           const typename Solver::Dev* __restrict__ tables, int64_t k_hi, int64_t k_lo,
-                                                          uint32_t seq0, int32_t* err, uint32_t wait_limit) {
+                                                          uint32_t* seqs, int32_t* err, uint32_t wait_limit) {
   extern __shared__ double lds[];
   constexpr int BS = kPartBlock, FW = Solver::kFaceWords;
   constexpr bool KEEP = NP <= 2;
@@ -265,6 +269,7 @@ __global__ __launch_bounds__(kPartBlock) void adjoint_parts_kernel(const DevProb
   const int64_t w = wi.column / S.parts;
   const int32_t tid0 = threadIdx.x, tid = tid0;
   const int32_t part = wi.column % S.parts;
+  const uint32_t seq0 = __builtin_amdgcn_readfirstlane(gbl(seqs)[wi.column]);  // before the solver's barrier
   const Solver solver(P, S, w, part, lds, err, wait_limit, tid, BS);
   LAS double *const U = solver.u, *const face_in = solver.in, *const face_out = solver.out;
   const int32_t Nj = P.Nj;
@@ -422,6 +427,7 @@ __global__ __launch_bounds__(kPartBlock) void adjoint_parts_kernel(const DevProb
     for (int k = 0; k < NF; ++k)
       if (fp[k] >= 0) gf[fp[k]] = af[k];
   }
+  if (threadIdx.x == 0) gblw(seqs)[wi.column] = seq0 + static_cast<uint32_t>(k_hi - k_lo + 1);
 }
 
 }  // namespace
