@@ -93,7 +93,7 @@ struct DevProblem {
   int32_t lat_ef;              // folded rows stored per row: ES (LDS store), ES rounded up to 4 (global)
   int32_t lat_mp, lat_bp;      // split column: modes per part and blocks per mode of the part-local
                                // tridiagonal solve in LDS (lat_mp 0: the column-wide one)
-  int32_t lat_pad_;
+  int32_t lat_tile;            // both sides at most 16: one wave solves (solve_lattice_tile)
   int64_t lat_t0;              // store offset of the folded rows (even: 16-byte loads)
   const double* lat_sine;      // [ES][CP]
   const double* lat_sine_p;    // [ES][2][CP/2]: the same table, even and odd modes apart (matrix-core B operands)
@@ -104,7 +104,7 @@ struct DevProblem {
   // lat_buf, then the sine tables of both sides at lat_tab (DstShape)
   int32_t lat_ld, lat_buf, lat_tab;
   int32_t store_doubles;       // LDS store: doubles a column's store takes
-  const double* lat_table;     // the sine tables (C's, then R's unless R == C)
+  const double* lat_table;     // the sine tables (C's, then R's unless R == C); lat_tile: TileShape's
   const double* lat_lam;       // [padded rows][lat_ld] inverse eigenvalues, 0 in the padding
   const int32_t* face_addr;    // [n_slice_rows]: store address of a face record's row slot
 };
@@ -121,6 +121,14 @@ struct DstShape {
   __host__ __device__ __forceinline__ int32_t entries() const { return pairs * steps * 2 * 64; }
   // rows or columns that outputs of all blocks take
   __host__ __device__ __forceinline__ int32_t padded() const { return 32 * pairs; }
+};
+
+// Tables of a lattice of at most 16 by 16 faces in LDS: the sine matrices of C and R
+// modes as operands of four steps, lane l of step s S[4 s + l / 16][l % 16], and the
+// inverse eigenvalues as results, register r of lane l row l / 16 + 4 r, column l % 16;
+// zero past the lattice. Rows of 20 doubles put the 16 rows of an operand on all banks.
+struct TileShape {
+  static constexpr int32_t kSide = 16, kLd = 20, kTable = 256;
 };
 
 // Store address of solve position q (an LDS store; the global one is linear).
@@ -815,7 +823,55 @@ __device__ __forceinline__ void dst_product(const LAS double* src, LAS double* d
   }
 }
 
+// K^-1 for a lattice of at most 16 by 16 faces: Z <- S_R (lam o (S_R Z S_C)) S_C by one
+// wave, without barriers between the four products. The result of a product lies in the
+// lanes as the operand B of the next (register r of the result is step r's operand), so
+// the three products that sum over rows follow each other in registers, and only the
+// last, over columns, takes its operand through LDS. The chain of 16 matrix
+// instructions is 1200 cycles; four products shared by the workgroup's waves, halved by
+// parity, spend longer at their barriers (64 columns of 12x9, thermal: 4.67 us a step,
+// now 3.46).
+__device__ __forceinline__ void solve_lattice_tile(const DevProblem& P, const FaceStore<false>& zs) {
+  constexpr int32_t N = TileShape::kSide, LD = TileShape::kLd, T = TileShape::kTable;
+  if (zs.vt < kWave) {
+    const int32_t R = P.lat_rows, C = P.lat_cols;
+    const int32_t lane = zs.vt, lr = lane & 15, lk = lane >> 4;
+    LAS double* z = (LAS double*)zs.p;
+    LAS double* t = z + P.lat_buf;
+    const LAS double* tab = z + P.lat_tab + lane;
+    double x[4], sc[4], sr[4], lam[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      // past the lattice the tables are zero: any finite operand will do
+      x[s] = z[min(lr, R - 1) * LD + min(4 * s + lk, C - 1)];
+      sc[s] = tab[s * kWave];
+      sr[s] = tab[T + s * kWave];
+      lam[s] = tab[2 * T + s * kWave];
+    }
+    vdouble4 a{0.0, 0.0, 0.0, 0.0}, b = a, c = a, d = a;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) a = __builtin_amdgcn_mfma_f64_16x16x4f64(x[s], sc[s], a, 0, 0, 0);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) b = __builtin_amdgcn_mfma_f64_16x16x4f64(sr[s], a[s], b, 0, 0, 0);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) c = __builtin_amdgcn_mfma_f64_16x16x4f64(sr[s], b[s] * lam[s], c, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) t[(lk + 4 * r) * LD + lr] = c[r];
+    // one wave's LDS accesses stay in order
+#pragma unroll
+    for (int s = 0; s < 4; ++s) x[s] = t[lr * LD + 4 * s + lk];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) d = __builtin_amdgcn_mfma_f64_16x16x4f64(x[s], sc[s], d, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (lk + 4 * r < R && lr < C) z[(lk + 4 * r) * LD + lr] = d[r];
+  }
+  static_assert(N * N == T, "a table of four steps of 64 lanes");
+  zs.barrier();
+}
+
 __device__ __forceinline__ void solve_lattice_padded(const DevProblem& P, const FaceStore<false>& zs) {
+  if (P.lat_tile) return solve_lattice_tile(P, zs);
   const int32_t R = P.lat_rows, C = P.lat_cols, ld = P.lat_ld;
   LAS double* z = (LAS double*)zs.p;
   LAS double* t = z + P.lat_buf;

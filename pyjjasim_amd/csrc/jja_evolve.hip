@@ -315,6 +315,24 @@ std::vector<double> dst_eigenvalues(int32_t n) {
   return mu;
 }
 
+// The tables of a lattice of at most 16 by 16 faces (TileShape)
+std::vector<double> tile_table(int32_t R, int32_t C, double g, double gc) {
+  constexpr int32_t T = TileShape::kTable;
+  std::vector<double> t(3 * T, 0.0);
+  const double pi = 3.14159265358979323846;
+  const std::vector<double> mc = dst_eigenvalues(C), mr = dst_eigenvalues(R);
+  for (int32_t e = 0; e < T; ++e) {
+    const int32_t i = 4 * (e / kWave) + e % kWave / 16, j = e % 16;  // row of a step's operand and of a result register
+    for (int32_t side = 0; side < 2; ++side) {
+      const int32_t n = side ? R : C, m = (i + 1) * (j + 1) % (2 * (n + 1));
+      if (i < n && j < n && m % (n + 1) != 0)
+        t[side * T + e] = std::sqrt(2.0 / (n + 1)) * std::sin(pi * static_cast<double>(m) / (n + 1));
+    }
+    if (i < R && j < C) t[2 * T + e] = 1.0 / (g * mr[i] + gc * mc[j]);
+  }
+  return t;
+}
+
 template <typename T>
 int upload(Plan* plan, const T* host, size_t n, const T** out) {
   *out = nullptr;
@@ -1251,7 +1269,15 @@ int jja_plan_create(int32_t n_problems, const jja_problem_desc* descs, jja_plan*
       const int32_t ld = dc.padded() + 4;
       const int64_t buf = static_cast<int64_t>(dr.padded()) * ld;
       const int64_t tables = dc.entries() + (R == C ? 0 : dr.entries());
-      if (d.index_bytes == 2 && R >= 8 && C >= 8 && 8 * (2 * buf + tables) <= plan->lds_limit) {
+      if (d.index_bytes == 2 && R <= TileShape::kSide && C <= TileShape::kSide) {
+        dp.lat_tile = 1;
+        dp.lat_ld = TileShape::kLd;
+        dp.lat_buf = TileShape::kSide * TileShape::kLd;
+        dp.lat_tab = 2 * dp.lat_buf;
+        dp.store_doubles = dp.lat_tab + 3 * TileShape::kTable;
+        const std::vector<double> t = tile_table(R, C, d.lattice_g, d.lattice_gc);
+        if ((rc = upload(plan, t.data(), t.size(), &dp.lat_table))) break;
+      } else if (d.index_bytes == 2 && R >= 8 && C >= 8 && 8 * (2 * buf + tables) <= plan->lds_limit) {
         dp.lat_ld = ld;
         dp.lat_buf = static_cast<int32_t>(buf);
         dp.lat_tab = static_cast<int32_t>(2 * buf);

@@ -241,7 +241,7 @@ __device__ __forceinline__ void SlabSolver<AHEAD>::solve(const DevProblem& P, co
     const bool edge = outer < 0 || outer >= 2 * G;  // beyond the lattice: zero
     const int32_t E = S.ends_rows;
     const uint32_t at_outer = 8u * static_cast<uint32_t>((edge ? own : outer) * E * C + k);
-    const uint32_t at_own = 8u * static_cast<uint32_t>(own * E * C + k), at_mode = 8u * static_cast<uint32_t>(k);
+    const uint32_t at_own = 8u * static_cast<uint32_t>(own * E * C + k);
     struct Chunk {
       double outer[RB], own[RB];
     } c[2];
