@@ -426,11 +426,11 @@ def large_bench(pa, torch, steps, checkpoint, n=512, W=16, full_steps=50000, sol
             "host_setup_s": setup_s}
 
 
-TRAFFIC_PROFILE = os.path.join("profiles", "evolve_kernel_square100_W256_traffic.txt")
+TRAFFIC_PROFILE = os.path.join("profiles", "evolve_wide_kernel_square100_W256_traffic.txt")
 
 
 def measured_traffic():
-    """HBM bytes per step of evolve_kernel from the committed rocprofv3 counter
+    """HBM bytes per step of evolve_wide_kernel from the committed rocprofv3 counter
     summary (FETCH_SIZE + WRITE_SIZE of one dispatch, each scaled by the
     copy-kernel factor, divided by the dispatch's steps), the launch length
     and the face-system solver it was taken with; None when the summary is
@@ -610,7 +610,7 @@ def main():
         if mt is not None and mt[2] == info["solver"]:
             per_step, prof_len, _ = mt
             traffic = per_step * tot_steps / n_launch
-            traffic_note = (f"{TRAFFIC_PROFILE}: {per_step / 1e6:.1f} MB/step measured on a "
+            traffic_note = (f"{TRAFFIC_PROFILE}: {per_step / 1e6:.2f} MB/step measured on a "
                             f"{prof_len}-step dispatch, times {tot_steps / n_launch:g} steps per launch")
     # integrity check at full size: device vortex counts equal the host count
     A = c.get_cycle_matrix()
@@ -640,7 +640,7 @@ def main():
                    "solve_stages": info["n_stages"] if info["solver"] == "cholesky" else None},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "traffic_source": traffic_note,
-                     "kernel": "evolve_kernel", "bytes_per_step": info["bytes_per_step"],
+                     "kernel": "evolve_wide_kernel", "bytes_per_step": info["bytes_per_step"],
                      "bytes_per_launch": bytes_per_launch, "stored_steps_in_window": info["stored_in_window"],
                      "mean_launch_ms": mean_launch_ms, "launches": n_launch},
         "plain": plain,

@@ -10,6 +10,10 @@
 // megabytes streamed from the L2 every step, which bounds large parts; small ones
 // are bound by the phases' latency and the meeting.
 //
+// Measured, us a step in one workgroup before (with the state in memory) and now: honeycomb
+// 30x30, 64 columns 41, 18.4 in 4 parts; triangular 80x80, 4 columns 535, 42 in 32;
+// triangular 20x20, 8 columns 35, 11.4 in 8.
+//
 // The meeting is that of the row slabs (jja_slab.hip): published values and the
 // waves' flags are device-scope accesses, buffered by the step's parity.
 #include "jja_domain.h"

@@ -19,6 +19,12 @@
 // product with the reciprocal 1/c0), so results agree with the CPU scheme to
 // the rounding of sin, of those quotients and of the linear solve.
 //
+// This file holds the general kernels, the plan and the C API. Columns that fit stay on
+// chip for a whole launch in kernels of their own, chosen at launch for the usual step
+// (stencil 3, no voltage sources, noise from Philox at a given amplitude or none):
+// jja_resident.hip (small columns), jja_wide.hip (large lattices, one workgroup),
+// jja_slab.hip (lattices in row slabs) and jja_domain.hip (other circuits in subdomains).
+//
 // The solve is a linear program of slices whose addresses do not depend on any
 // data: each thread prefetches the entries of the next slice (also across the
 // phase barriers, which only order LDS traffic) while it processes the current

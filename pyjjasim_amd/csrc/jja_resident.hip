@@ -8,7 +8,9 @@
 // step waits for a write of u, the face records, their codes, the gathers of u
 // and the junction pass's own loads in turn, five to seven round trips of about
 // a microsecond. Here a step touches LDS only (and global memory for stored
-// steps and for inputs that vary in time).
+// steps and for inputs that vary in time). Measured with the padded lattice solve,
+// us a step: 12x9, 64 columns 9.9 before, 4.7 (with one wave's solve 3.5 now); 37x53, 96
+// columns 23.0 before, 13.4 now.
 #include "jja_resident.h"
 
 #include "jja_device.h"

@@ -126,7 +126,8 @@ TURN_BYTES = 1 << 28
 
 # junctions up to which a column's whole state fits in one workgroup's LDS
 # beside the face vector (or in registers): the kernels for that take at most
-# 512 threads, which then have 256 registers each
+# 512 threads, which then have 256 registers each (1024 threads spilled over 100
+# of their 128). Larger lattices take 1024, or the registers of jja_wide.hip
 RESIDENT_JUNCTIONS = 6144
 
 
@@ -158,7 +159,10 @@ def auto_parts(host, columns, stencil_width, max_parts=16, junctions_per_part=24
     return parts
 
 
-# a slab (jja_slab.hip) holds at most this many junctions and at least these rows
+# a slab (jja_slab.hip) holds at most this many junctions and at least these rows.
+# Fewer junctions than SLAB_MIN_JUNCTIONS stay in one workgroup: the parts' meeting
+# costs 4 to 5 us a step (us a step in 1 / 4 / 8 workgroups: 24x24 7.4 / 8.8 / 9.2,
+# 32x32 8.5 / 9.6 / 10.1, but 48x48 16.0 / 12.2 / 11.0)
 SLAB_BLOCK = 512
 SLAB_JUNCTIONS = 9 * 2 * SLAB_BLOCK
 SLAB_MIN_ROWS = 4
@@ -167,7 +171,9 @@ SLAB_MIN_JUNCTIONS = 3000
 
 def slab_parts(host, columns, n_cu, max_parts=16):
     """Row slabs per column of a lattice plan: the most whose workgroups, one per
-    compute unit, all fit on the device, or 1 when that leaves slabs too large."""
+    compute unit, all fit on the device, or 1 when that leaves slabs too large. One
+    100x100 column takes 57.7 us a step in one workgroup, 25.7 in 4 slabs, 18.5 in 8,
+    16.1 in 16 and 19.9 in 32."""
     if not host.uses_lattice or not 8 <= host.lattice.C <= SLAB_BLOCK // 2 or host.Nj < SLAB_MIN_JUNCTIONS:
         return 1
     lat, parts = host.lattice, 1
@@ -176,19 +182,24 @@ def slab_parts(host, columns, n_cu, max_parts=16):
     rows = -(-lat.R // parts)
     if parts == 1 or (2 * rows + 1) * (lat.C + 1) > SLAB_JUNCTIONS:
         return 1
-    # two slabs pay only where one workgroup cannot hold the column's state
+    # two slabs pay only where one workgroup cannot hold the column's state (us a step
+    # in 1 / 2: 37x53 13.3 / 15.2, 64x64 25.7 / 18.4, 80x80 41.8 / 36.2)
     return 1 if parts == 2 and host.Nj <= RESIDENT_JUNCTIONS else parts
 
 
 # subdomains of any other circuit (jja_domain.hip): the fewest faces a part has, and
-# the most faces of a circuit that two parts take
+# the most faces of a circuit that two parts take (us a step: a 10x10 honeycomb array
+# 14.7 in one workgroup, 11 in 2 to 4; 30x30 with 64 columns 39.3 in one, 33.7 in 2,
+# 18.6 in 4; a 30x30 triangular one 45.7 in one, 64 in 2, 19.3 in 8: two parts of a
+# large circuit keep long elimination chains and gain nothing)
 DOMAIN_MIN_FACES = 100
 DOMAIN_PAIR_FACES = 2000
 
 
 def domain_parts(Nf, columns, n_cu, max_parts=32):
     """Subdomains per column: the most whose workgroups, one per compute unit, all
-    fit on the device and keep enough faces each."""
+    fit on the device and keep enough faces each (an 80x80 triangular column takes
+    535 us a step in one workgroup, 74 in 16 subdomains, 42 in 32)."""
     parts = 1
     while parts < max_parts and 2 * parts * columns <= n_cu and Nf >= 2 * parts * DOMAIN_MIN_FACES:
         parts *= 2

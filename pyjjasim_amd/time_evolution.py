@@ -25,11 +25,17 @@ Extensions (keyword-only, defaults keep reference behaviour):
   face_store       "auto" (default): each column keeps its face vector in LDS when
                    it fits (up to about 10^4 faces) and in global memory otherwise;
                    "lds" or "global" force one.
-  parts            Workgroups per column for circuits with a global face store:
-                   None (default) picks the largest power of two up to 16 that
-                   keeps all columns' workgroups resident on the device; 1 keeps
-                   one workgroup per column. With the factor, results do not
-                   depend on it; the lattice solve's rounding does (1e-12).
+  parts            Workgroups per column: None (default) chooses by the circuit's
+                   size and the number of columns: row slabs of a lattice or
+                   subdomains of another circuit, whose parts keep their junctions
+                   on chip and meet once a step (left open: block_size, face_store,
+                   column_pairs; usual steps only), else, with a global face
+                   store, the largest power of two up to 16 that keeps all
+                   columns' workgroups resident on the device. 1 keeps one
+                   workgroup per column, a larger number splits a global face
+                   store. With the factor, results do not depend on a number given;
+                   the lattice solve's rounding does (1e-12), as do slabs'
+                   and subdomains'.
   local_stages     Lowest stages of the factor schedule solved wave-locally (each
                    wave solves whole independent subtrees, with no barrier between
                    those stages; for a split column, the stages above them are
