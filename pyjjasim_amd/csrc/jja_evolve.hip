@@ -571,7 +571,10 @@ int check_plan_shapes(int32_t n, const jja_problem_desc* descs) {
       return fail(JJA_EINVAL, "jja_plan_create: all problems of a plan need the same block_size/parts");
     if (split && d.index_bytes != 4)
       return fail(JJA_EINVAL, "jja_plan_create: with a split column, every problem needs the global face store");
-
+    // subdomains are built for a plan's only problem, and nothing else solves there
+    if (d.domains && (n != 1 || d.lattice_rows != 0 || d.n_faces <= 0 || d.n_junctions <= 0))
+      return fail(JJA_EINVAL, "jja_plan_create: domains need a plan of one problem with junctions and faces, "
+                              "without a lattice solve");
     if ((d.column_pairs != 0) != (descs[0].column_pairs != 0))
       return fail(JJA_EINVAL, "jja_plan_create: column_pairs must be the same for every problem of a plan");
   }

@@ -89,3 +89,28 @@ def test_domain_plan_leaves_the_rest_to_the_factor():
     assert CircuitPlan(pa.SquareArray(12, 12), 0.05, domains=4).uses_lattice
     p = CircuitPlan(pa.HoneycombArray(11, 9), 0.05, 4, domains=4)
     assert p.domains is None and p.parts == 1
+
+
+def test_domain_plans_stand_alone():
+    """What the header asks of a descriptor with subdomains is checked: a plan of that
+    problem alone, no lattice solve beside them, and faces and junctions to work on."""
+    import ctypes as C
+    from pyjjasim_amd import _native
+    lib = _native.lib()
+    make = lambda: CircuitPlan(pa.HoneycombArray(11, 9), 0.05, domains=4)
+    plans = [make(), make()]
+    both = (_native.ProblemDesc * 2)(*[p.desc(max_columns=2) for p in plans])
+    assert lib.jja_plan_validate(1, both) == 0
+    assert lib.jja_plan_validate(2, both) == -1                    # JJA_EINVAL
+    assert b"domains" in lib.jja_last_error()
+    beside = CircuitPlan(pa.SquareArray(12, 12), 0.05).relayout(512, 4)   # a split lattice
+    d = beside.desc(max_columns=2)
+    assert lib.jja_plan_validate(1, C.byref(d)) == 0
+    d.domains = both[0].domains
+    assert lib.jja_plan_validate(1, C.byref(d)) == -1
+    for name in ("n_junctions", "n_faces"):
+        d = make().desc(max_columns=2)
+        d.domains = both[0].domains
+        setattr(d, name, 0)
+        d.n_face_slices = 0
+        assert lib.jja_plan_validate(1, C.byref(d)) == -1, name
