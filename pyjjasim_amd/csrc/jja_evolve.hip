@@ -491,6 +491,20 @@ int claim_stream(Plan* plan, hipStream_t stream) {
   return JJA_OK;
 }
 
+// Whether `stream` is being captured into a graph.
+int capture_state(hipStream_t stream, bool* capturing) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  JJA_HIP(hipStreamIsCapturing(stream, &status));
+  *capturing = status != hipStreamCaptureStatusNone;
+  return JJA_OK;
+}
+
+// Split launches that meet at column barriers are not captured: their barrier words are
+// cleared by a memset, and they need the cooperative launch.
+int refuse_capture(const char* who) {
+  return fail(JJA_EUNSUPPORTED, std::string(who) + ": a launch with column barriers cannot be captured into a graph");
+}
+
 int mark_launched(Plan* plan, hipStream_t stream) {
   JJA_HIP(hipEventRecord(plan->done, stream));
   plan->last_stream = stream;
@@ -1061,9 +1075,9 @@ int launch_cooperative(Plan* plan, const void* kern, int BS, int32_t n, int64_t 
                                       std::to_string(static_cast<int64_t>(per_cu) * plan->n_cu) + " at once");
   void* argv[] = {static_cast<void*>(&args)...};
   // a graph takes the plain launch: its workgroups fit on the device together (above)
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  JJA_HIP(hipStreamIsCapturing(stream, &capture));
-  if (capture != hipStreamCaptureStatusNone) {
+  bool capturing = false;
+  if (int rc = capture_state(stream, &capturing)) return rc;
+  if (capturing) {
     JJA_HIP(hipLaunchKernel(kern, dim3(n), dim3(BS), argv, static_cast<size_t>(lds), stream));
     return JJA_OK;
   }
@@ -1519,6 +1533,9 @@ int jja_evolve(jja_plan* p, const jja_problem_run* runs, int32_t n_steps, int64_
     for (int32_t w = 0; w < items_of(plan, r.W); ++w) (global ? work_g : work).push_back({i, w});
   }
   hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
+  bool capturing = false;
+  if (int rc = capture_state(stream, &capturing)) return rc;
+  if (capturing && plan->parts > 1 && !parts_run(plan, runs[0])) return refuse_capture("jja_evolve");
   if (int rc = claim_stream(plan, stream)) return rc;
   if (int rc = upload_if_changed(plan->d_runs, runs, static_cast<size_t>(np), plan->h_runs, plan->runs_valid, stream))
     return rc;
@@ -1587,6 +1604,9 @@ int jja_adjoint(jja_plan* p, const jja_adjoint_run* runs, int64_t k_hi, int64_t 
     for (int32_t w = 0; w < items_of(plan, r.W); ++w) (global ? work_g : work).push_back({i, w});
   }
   hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
+  bool capturing = false;
+  if (int rc = capture_state(stream, &capturing)) return rc;
+  if (capturing && plan->parts > 1 && !plan->d_parts) return refuse_capture("jja_adjoint");
   if (int rc = claim_stream(plan, stream)) return rc;
   if (int rc = upload_if_changed(plan->d_adj, runs, static_cast<size_t>(np), plan->h_adj, plan->adj_valid, stream))
     return rc;

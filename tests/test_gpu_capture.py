@@ -40,3 +40,24 @@ def test_forward_replays(make, parts):
                 again = evo(Ic, f, Is)
             side.synchronize()
             assert torch.equal(again, want)
+
+
+def test_column_barriers_refuse_capture():
+    """A pass whose parts meet at column barriers is refused while its stream is captured,
+    before anything is recorded, and runs as before afterwards."""
+    torch = pytest.importorskip("torch")
+    from pyjjasim_amd import _native
+    c, W = pa.SquareArray(30, 30), 2
+    put = lambda a: torch.tensor(a, dtype=torch.float64, device="cuda")
+    Ic, f = put(np.ones(c.junction_count())), put(np.full((c.face_count(), W), 0.1))
+    Is = put(np.outer(c.current_base(0.0), [0.5, 1.1]))
+    with pa.DifferentiableEvolution(c, time_step=0.05, time_step_count=12, problem_count=W, store_time_steps=[11], parts=4,
+                                    face_store="global", block_size=256) as evo, torch.no_grad():
+        print("[capture] column barriers", flush=True)
+        want = evo(Ic, f, Is)
+        torch.cuda.synchronize()
+        with pytest.raises(_native.NativeError, match="captured"):
+            with torch.cuda.graph(torch.cuda.CUDAGraph()):
+                evo(Ic, f, Is)
+        torch.cuda.synchronize()
+        assert torch.equal(evo(Ic, f, Is), want)
