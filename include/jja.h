@@ -367,6 +367,13 @@ typedef struct jja_problem_run {
  * jja_plan_status after its runs. Steps step0 .. step0 + n_steps - 1 must lie
  * within what every run's sources, noise and slot maps cover: those arrays
  * carry no length here, so the caller keeps launches inside the horizon.
+ * On a stream that is being captured into a graph, the launch is recorded with
+ * descriptors and work items of its own, which the plan keeps until it is destroyed
+ * (equal ones once; 64 MiB at most, then JJA_ENOMEM): later calls do not change what a
+ * replay reads. The arrays the descriptors point to are the caller's, and so is the
+ * order of replays and other launches of the plan. Launches whose parts meet at column
+ * barriers (parts > 1 without slabs or subdomains) are refused (JJA_EUNSUPPORTED).
+ * jja_adjoint does the same.
  */
 int jja_evolve(jja_plan* plan, const jja_problem_run* runs, int32_t n_steps, int64_t step0,
                void* stream);

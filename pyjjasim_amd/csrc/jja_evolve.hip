@@ -285,6 +285,20 @@ struct Plan {
   std::vector<jja_adjoint_run> h_adj;
   std::vector<WorkItem> h_work;
   bool runs_valid = false, adj_valid = false, work_valid = false;
+  // what the launch being prepared reads: the arrays above, or a captured launch's own
+  const jja_problem_run* use_runs = nullptr;
+  const jja_adjoint_run* use_adj = nullptr;
+  const WorkItem* use_work = nullptr;
+  // A launch recorded into a graph reads descriptors and work items that never change:
+  // a replay must find those of its capture, whatever eager launches did meanwhile.
+  // Equal contents are kept once; chunks are freed with the plan.
+  struct Kept {
+    std::vector<char> host;
+    void* dev;
+  };
+  std::vector<Kept> kept;
+  char* kept_chunk = nullptr;
+  size_t kept_left = 0, kept_bytes = 0;
   // the stream of the previous launch and an event recorded after it
   hipEvent_t done = nullptr;
   hipStream_t last_stream = nullptr;
@@ -522,6 +536,61 @@ int upload_if_changed(T* dev, const T* host, size_t n, std::vector<T>& shadow, b
   shadow.assign(host, host + n);
   valid = true;
   return JJA_OK;
+}
+
+// This thread may allocate and copy beside a stream that is being captured.
+struct BesideCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  BesideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~BesideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// A device copy of `bytes` of host data that stays as it is until the plan is destroyed,
+// made outside the graph being captured.
+constexpr size_t kKeptChunk = size_t{1} << 16, kKeptLimit = size_t{1} << 26;
+int keep_copy(Plan* plan, const void* host, size_t bytes, const void** out) {
+  for (const Plan::Kept& k : plan->kept)
+    if (k.host.size() == bytes && std::memcmp(k.host.data(), host, bytes) == 0) {
+      *out = k.dev;
+      return JJA_OK;
+    }
+  const size_t room = (bytes + 255) & ~size_t{255};
+  if (plan->kept_bytes + room > kKeptLimit)
+    return fail(JJA_ENOMEM, "the plan's captured launches hold " + std::to_string(plan->kept_bytes) +
+                                " bytes of descriptors; destroy the plan to free them");
+  const BesideCapture beside;
+  if (room > plan->kept_left) {
+    const size_t chunk = std::max(room, kKeptChunk);
+    void* d = nullptr;
+    if (hipMalloc(&d, chunk) != hipSuccess) return fail(JJA_ENOMEM, "captured launch: device allocation failed");
+    plan->allocations.push_back(d);
+    plan->kept_chunk = static_cast<char*>(d);
+    plan->kept_left = chunk;
+  }
+  void* const d = plan->kept_chunk;
+  hipStream_t side = nullptr;
+  JJA_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
+  hipError_t e = hipMemcpyAsync(d, host, bytes, hipMemcpyHostToDevice, side);
+  if (e == hipSuccess) e = hipStreamSynchronize(side);
+  (void)hipStreamDestroy(side);
+  if (e != hipSuccess) return fail(JJA_EHIP, std::string("captured launch: copy of its descriptors: ") + hipGetErrorString(e));
+  const char* bytes0 = static_cast<const char*>(host);
+  plan->kept.push_back({std::vector<char>(bytes0, bytes0 + bytes), d});
+  plan->kept_chunk += room;
+  plan->kept_left -= room;
+  plan->kept_bytes += room;
+  *out = d;
+  return JJA_OK;
+}
+
+// The device array a launch reads n descriptors from: the plan's, brought up to date, or
+// a copy of the launch's own when it is captured.
+template <typename T>
+int stage(Plan* plan, T* dev, const T* host, size_t n, std::vector<T>& shadow, bool& valid, hipStream_t stream,
+          bool capturing, const T** use) {
+  if (capturing) return keep_copy(plan, host, n * sizeof(T), reinterpret_cast<const void**>(use));
+  *use = dev;
+  return upload_if_changed(dev, host, n, shadow, valid, stream);
 }
 
 // Raise a kernel's dynamic LDS limit to at least lds bytes. The limit belongs
@@ -839,7 +908,7 @@ int launch_evolve(Plan* plan, const WorkItem* work, int32_t n_work, int64_t lds,
   auto* kern = evolve_kernel<BS, SW, STORE>;
   if (int rc = set_lds_limit(plan, reinterpret_cast<const void*>(kern), static_cast<int>(lds))) return rc;
   hipLaunchKernelGGL(kern, dim3(n_work), dim3(BS), static_cast<size_t>(lds), stream,
-                     plan->d_problems, plan->d_runs, work, n_steps, step0);
+                     plan->d_problems, plan->use_runs, work, n_steps, step0);
   JJA_HIP(hipGetLastError());
   return JJA_OK;
 }
@@ -850,7 +919,7 @@ int launch_adjoint(Plan* plan, const WorkItem* work, int32_t n_work, int64_t lds
   auto* kern = adjoint_kernel<BS, GLOBAL>;
   if (int rc = set_lds_limit(plan, reinterpret_cast<const void*>(kern), static_cast<int>(lds))) return rc;
   hipLaunchKernelGGL(kern, dim3(n_work), dim3(BS), static_cast<size_t>(lds), stream,
-                     plan->d_problems, plan->d_adj, work, k_hi, k_lo);
+                     plan->d_problems, plan->use_adj, work, k_hi, k_lo);
   JJA_HIP(hipGetLastError());
   return JJA_OK;
 }
@@ -865,10 +934,11 @@ int launch_vortex(Plan* plan, int32_t p, const double* theta, int32_t cols, int3
 }
 
 // Copies the work items of one launch to the plan's array (sized at plan
-// creation) when they differ from what it holds.
-int upload_work(Plan* plan, const std::vector<WorkItem>& work, hipStream_t stream) {
+// creation) when they differ from what it holds, or to a captured launch's own.
+int upload_work(Plan* plan, const std::vector<WorkItem>& work, hipStream_t stream, bool capturing) {
   if (work.size() > plan->work_cap) return fail(JJA_EINVAL, "launch has more work items than the plan was sized for");
-  return upload_if_changed(plan->d_work, work.data(), work.size(), plan->h_work, plan->work_valid, stream);
+  return stage(plan, plan->d_work, work.data(), work.size(), plan->h_work, plan->work_valid, stream, capturing,
+               &plan->use_work);
 }
 
 template <int BS, int STORE>
@@ -925,8 +995,8 @@ int launch_resident(Plan* plan, const void* kern, int32_t n, int64_t lds, hipStr
 int launch_resident_evolve(Plan* plan, int32_t n, int form, int64_t lds, int32_t n_steps, int64_t step0,
                            hipStream_t stream) {
   const DevProblem* probs = plan->d_problems;
-  const jja_problem_run* runs = plan->d_runs;
-  const WorkItem* work = plan->d_work;
+  const jja_problem_run* runs = plan->use_runs;
+  const WorkItem* work = plan->use_work;
   return launch_resident(plan, resident_evolve_kernel(plan->block_size, form), n, lds, stream, probs, runs, work, n_steps,
                          step0);
 }
@@ -934,8 +1004,8 @@ int launch_resident_evolve(Plan* plan, int32_t n, int form, int64_t lds, int32_t
 int launch_resident_adjoint(Plan* plan, int32_t n, int form, int64_t lds, int64_t k_hi, int64_t k_lo,
                             hipStream_t stream) {
   const DevProblem* probs = plan->d_problems;
-  const jja_adjoint_run* runs = plan->d_adj;
-  const WorkItem* work = plan->d_work;
+  const jja_adjoint_run* runs = plan->use_adj;
+  const WorkItem* work = plan->use_work;
   return launch_resident(plan, resident_adjoint_kernel(plan->block_size, form), n, lds, stream, probs, runs, work, k_hi,
                          k_lo);
 }
@@ -961,8 +1031,8 @@ int launch_wide(Plan* plan, const jja_problem_run* host_runs, int32_t n, int32_t
   const void* kern = wide_evolve_kernel(gauss, uniform);
   if (int rc = set_lds_limit(plan, kern, static_cast<int>(plan->wide_lds))) return rc;
   const DevProblem* probs = plan->d_problems;
-  const jja_problem_run* runs = plan->d_runs;
-  const WorkItem* work = plan->d_work;
+  const jja_problem_run* runs = plan->use_runs;
+  const WorkItem* work = plan->use_work;
   const WideDev* tables = plan->d_wide;
   void* argv[] = {&probs, &runs, &work, &tables, &n_steps, &step0};
   JJA_HIP(hipLaunchKernel(kern, dim3(n), dim3(kWideBlock), argv, static_cast<size_t>(plan->wide_lds), stream));
@@ -1088,8 +1158,8 @@ int launch_cooperative(Plan* plan, const void* kern, int BS, int32_t n, int64_t 
 template <int BS>
 int launch_evolve_split_bs(Plan* plan, int32_t n, int32_t n_steps, int64_t step0, hipStream_t stream) {
   const DevProblem* probs = plan->d_problems;
-  const jja_problem_run* runs = plan->d_runs;
-  const WorkItem* work = plan->d_work;
+  const jja_problem_run* runs = plan->use_runs;
+  const WorkItem* work = plan->use_work;
   const void* kern = plan->pairs ? reinterpret_cast<const void*>(evolve_split_kernel<BS, 3, BS <= 512>)
                                  : reinterpret_cast<const void*>(evolve_split_kernel<BS, 3, false>);
   return launch_cooperative(plan, kern, BS, n, plan->split_lds, stream, probs, runs, work, n_steps, step0, plan->d_ctrs,
@@ -1115,8 +1185,8 @@ bool parts_run(const Plan* plan, const jja_problem_run& r) {
 
 int launch_evolve_parts(Plan* plan, int32_t n, int32_t n_steps, int64_t step0, hipStream_t stream) {
   const DevProblem* probs = plan->d_problems;
-  const jja_problem_run* runs = plan->d_runs;
-  const WorkItem* work = plan->d_work;
+  const jja_problem_run* runs = plan->use_runs;
+  const WorkItem* work = plan->use_work;
   const void* tables = plan->d_parts;
   return launch_cooperative(plan, plan->parts_evolve, plan->block_size, n, plan->parts_lds, stream, probs, runs, work,
                             tables, n_steps, step0, plan->d_parts_seq, plan->d_err, plan->wait_limit);
@@ -1124,8 +1194,8 @@ int launch_evolve_parts(Plan* plan, int32_t n, int32_t n_steps, int64_t step0, h
 
 int launch_adjoint_parts(Plan* plan, int32_t n, int64_t k_hi, int64_t k_lo, hipStream_t stream) {
   const DevProblem* probs = plan->d_problems;
-  const jja_adjoint_run* runs = plan->d_adj;
-  const WorkItem* work = plan->d_work;
+  const jja_adjoint_run* runs = plan->use_adj;
+  const WorkItem* work = plan->use_work;
   const void* tables = plan->d_parts;
   return launch_cooperative(plan, plan->parts_adjoint, plan->block_size, n, plan->parts_lds, stream, probs, runs, work,
                             tables, k_hi, k_lo, plan->d_parts_seq, plan->d_err, plan->wait_limit);
@@ -1134,8 +1204,8 @@ int launch_adjoint_parts(Plan* plan, int32_t n, int64_t k_hi, int64_t k_lo, hipS
 template <int BS>
 int launch_adjoint_split_bs(Plan* plan, int32_t n, int64_t k_hi, int64_t k_lo, hipStream_t stream) {
   const DevProblem* probs = plan->d_problems;
-  const jja_adjoint_run* runs = plan->d_adj;
-  const WorkItem* work = plan->d_work;
+  const jja_adjoint_run* runs = plan->use_adj;
+  const WorkItem* work = plan->use_work;
   const void* kern = plan->pairs ? reinterpret_cast<const void*>(adjoint_split_kernel<BS, BS <= 512>)
                                  : reinterpret_cast<const void*>(adjoint_split_kernel<BS, false>);
   return launch_cooperative(plan, kern, BS, n, plan->split_lds, stream, probs, runs, work, k_hi, k_lo, plan->d_ctrs,
@@ -1536,8 +1606,9 @@ int jja_evolve(jja_plan* p, const jja_problem_run* runs, int32_t n_steps, int64_
   bool capturing = false;
   if (int rc = capture_state(stream, &capturing)) return rc;
   if (capturing && plan->parts > 1 && !parts_run(plan, runs[0])) return refuse_capture("jja_evolve");
-  if (int rc = claim_stream(plan, stream)) return rc;
-  if (int rc = upload_if_changed(plan->d_runs, runs, static_cast<size_t>(np), plan->h_runs, plan->runs_valid, stream))
+  if (int rc = capturing ? JJA_OK : claim_stream(plan, stream)) return rc;
+  if (int rc = stage(plan, plan->d_runs, runs, static_cast<size_t>(np), plan->h_runs, plan->runs_valid, stream, capturing,
+                     &plan->use_runs))
     return rc;
   int rc = JJA_OK;
   if (plan->parts > 1) {
@@ -1545,7 +1616,7 @@ int jja_evolve(jja_plan* p, const jja_problem_run* runs, int32_t n_steps, int64_
     // circuit without faces has none and needs none): all columns, one launch
     work.insert(work.end(), work_g.begin(), work_g.end());
     const std::vector<WorkItem> split = split_work(plan, work);
-    if ((rc = upload_work(plan, split, stream))) return rc;
+    if ((rc = upload_work(plan, split, stream, capturing))) return rc;
     if (parts_run(plan, runs[0]))
       rc = launch_evolve_parts(plan, static_cast<int32_t>(split.size()), n_steps, step0, stream);
     else if ((rc = reset_counters(plan, work.size(), stream)))
@@ -1557,7 +1628,7 @@ int jja_evolve(jja_plan* p, const jja_problem_run* runs, int32_t n_steps, int64_
     const int32_t n_lds = static_cast<int32_t>(work.size()), n_g = static_cast<int32_t>(work_g.size());
     work.insert(work.end(), work_g.begin(), work_g.end());
     order_work(plan, work);
-    if ((rc = upload_work(plan, work, stream))) return rc;
+    if ((rc = upload_work(plan, work, stream, capturing))) return rc;
     if (lds < 8) lds = 8;
     const int32_t n = n_lds + n_g;
     int64_t resident_lds = 0;
@@ -1567,14 +1638,14 @@ int jja_evolve(jja_plan* p, const jja_problem_run* runs, int32_t n_steps, int64_
     else if (n_g == 0 && wide_runs(plan, runs))
       rc = launch_wide(plan, runs, n, n_steps, step0, stream);
     else if (n_g == 0)
-      rc = launch_evolve_bs<0>(plan, plan->d_work, n, lds, n_steps, step0, stream);
+      rc = launch_evolve_bs<0>(plan, plan->use_work, n, lds, n_steps, step0, stream);
     else if (n_lds == 0)
-      rc = launch_evolve_bs<1>(plan, plan->d_work, n, 8, n_steps, step0, stream);
+      rc = launch_evolve_bs<1>(plan, plan->use_work, n, 8, n_steps, step0, stream);
     else
-      rc = launch_evolve_bs<2>(plan, plan->d_work, n, lds, n_steps, step0, stream);
+      rc = launch_evolve_bs<2>(plan, plan->use_work, n, lds, n_steps, step0, stream);
   }
   if (rc) return rc;
-  return mark_launched(plan, stream);
+  return capturing ? JJA_OK : mark_launched(plan, stream);  // nothing has been launched yet
 }
 
 int jja_adjoint(jja_plan* p, const jja_adjoint_run* runs, int64_t k_hi, int64_t k_lo, void* stream_ptr) {
@@ -1607,14 +1678,15 @@ int jja_adjoint(jja_plan* p, const jja_adjoint_run* runs, int64_t k_hi, int64_t 
   bool capturing = false;
   if (int rc = capture_state(stream, &capturing)) return rc;
   if (capturing && plan->parts > 1 && !plan->d_parts) return refuse_capture("jja_adjoint");
-  if (int rc = claim_stream(plan, stream)) return rc;
-  if (int rc = upload_if_changed(plan->d_adj, runs, static_cast<size_t>(np), plan->h_adj, plan->adj_valid, stream))
+  if (int rc = capturing ? JJA_OK : claim_stream(plan, stream)) return rc;
+  if (int rc = stage(plan, plan->d_adj, runs, static_cast<size_t>(np), plan->h_adj, plan->adj_valid, stream, capturing,
+                     &plan->use_adj))
     return rc;
   int rc = JJA_OK;
   if (plan->parts > 1) {
     work.insert(work.end(), work_g.begin(), work_g.end());
     const std::vector<WorkItem> split = split_work(plan, work);
-    if ((rc = upload_work(plan, split, stream))) return rc;
+    if ((rc = upload_work(plan, split, stream, capturing))) return rc;
     if (plan->d_parts)
       rc = launch_adjoint_parts(plan, static_cast<int32_t>(split.size()), k_hi, k_lo, stream);
     else if ((rc = reset_counters(plan, work.size(), stream)))
@@ -1626,18 +1698,18 @@ int jja_adjoint(jja_plan* p, const jja_adjoint_run* runs, int64_t k_hi, int64_t 
     order_work(plan, work);
     order_work(plan, work_g);
     work.insert(work.end(), work_g.begin(), work_g.end());
-    if ((rc = upload_work(plan, work, stream))) return rc;
+    if ((rc = upload_work(plan, work, stream, capturing))) return rc;
     if (lds < 8) lds = 8;
     int64_t resident_lds = 0;
     const int form = n_lds && !n_g ? resident_layout(plan, &resident_lds) : -1;
     if (form >= 0)
       rc = launch_resident_adjoint(plan, n_lds, form, resident_lds, k_hi, k_lo, stream);
     else if (n_lds)
-      rc = launch_adjoint_bs<false>(plan, plan->d_work, n_lds, lds, k_hi, k_lo, stream);
-    if (!rc && n_g) rc = launch_adjoint_bs<true>(plan, plan->d_work + n_lds, n_g, 8, k_hi, k_lo, stream);
+      rc = launch_adjoint_bs<false>(plan, plan->use_work, n_lds, lds, k_hi, k_lo, stream);
+    if (!rc && n_g) rc = launch_adjoint_bs<true>(plan, plan->use_work + n_lds, n_g, 8, k_hi, k_lo, stream);
   }
   if (rc) return rc;
-  return mark_launched(plan, stream);
+  return capturing ? JJA_OK : mark_launched(plan, stream);  // nothing has been launched yet
 }
 
 int jja_solve(jja_plan* p, int32_t i, const double* b, int64_t ldb, double* x, int64_t ldx, int32_t cols,

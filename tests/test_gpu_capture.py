@@ -61,3 +61,54 @@ def test_column_barriers_refuse_capture():
                 evo(Ic, f, Is)
         torch.cuda.synchronize()
         assert torch.equal(evo(Ic, f, Is), want)
+
+
+def _inputs(torch, c, W, seed):
+    """Ic, f and Is, the last two without a column axis: the kernels read them in place."""
+    rng = np.random.default_rng(seed)
+    put = lambda a: torch.tensor(a, dtype=torch.float64, device="cuda")
+    return (put(np.exp(0.1 * rng.standard_normal(c.junction_count()))), put(0.1 + 0.05 * rng.random(c.face_count())),
+            put((0.5 + 0.1 * seed) * c.current_base(0.0)))
+
+
+PLANS = [(lambda: pa.SquareArray(12, 12), {}), (lambda: pa.SquareArray(70, 72), {"parts": 1}),
+         (lambda: pa.SquareArray(70, 72), {}), (lambda: pa.HoneycombArray(16, 16), {})]
+
+
+@pytest.mark.parametrize("make,opts", PLANS, ids=["resident", "wide", "slabs", "domains"])
+@pytest.mark.parametrize("grad", [False, True])
+def test_replays_keep_their_inputs(make, opts, grad):
+    """Captured on a stream of its own without a pass before it; between the replays eager
+    passes, forward and backward, with other tensors on other streams. Every replay gives
+    what the captured inputs give (two segments, so the backward pass recomputes phases
+    and runs the adjoint twice), and every eager pass what its own give."""
+    torch = pytest.importorskip("torch")
+    c, W, Nt = make(), 2, 15
+    A, B = _inputs(torch, c, W, 1), _inputs(torch, c, W, 2)
+    G = torch.tensor(np.random.default_rng(3).standard_normal((c.junction_count(), W, 2)), device="cuda")
+    kw = dict(time_step=0.05, time_step_count=Nt, problem_count=W, temperature=0.01, store_time_steps=[3, Nt - 1],
+              checkpoint_every=8, seed=6, **opts)
+
+    def run(evo, leaves):
+        with torch.set_grad_enabled(grad):
+            th = evo(*leaves)
+            return (th.detach(),) + (torch.autograd.grad(th, leaves, G) if grad else ())
+    leaves = [[x.clone().requires_grad_(grad) for x in X] for X in (A, B)]
+    print(f"[capture] {c.junction_count()} junctions, grad={grad}", flush=True)
+    with pa.DifferentiableEvolution(c, **kw) as evo:
+        want = [[x.clone() for x in run(evo, X)] for X in leaves]
+    with pa.DifferentiableEvolution(c, **kw) as evo:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = run(evo, leaves[0])
+        for k in range(4):
+            graph.replay()
+            torch.cuda.synchronize()
+            for a, b in zip(out, want[0]):
+                assert torch.equal(a, b)
+            side = torch.cuda.Stream()
+            with torch.cuda.stream(side):
+                for X, ref in (zip(leaves, want) if k % 2 else [(leaves[1], want[1])]):
+                    for a, b in zip(run(evo, X), ref):
+                        assert torch.equal(a, b)
+            side.synchronize()
