@@ -282,7 +282,8 @@ __device__ __forceinline__ void wide_pass(const DevProblem& P, const jja_problem
   LAS double* const U = Z + S.buf + 2;
   const uint32_t noise_col = static_cast<uint32_t>(R.column_offset + w);
   const GAS double* Icp = gbl(R.Ic ? R.Ic : P.Ic);
-  const TermView isn = term_view(R.Is, prep, P.zero, w, t + 1);
+  // a source marked zero is left out of the step, whatever its values
+  const TermView isn = term_view(R.Is, prep && !R.Is.zero, P.zero, w, t + 1);
   const TermView sgn = term_view(R.sigma, GAUSS && prep && !R.T.zero, P.zero, w, t + 1);
   const double rc0 = rc0_at(P, 0), c1 = coef_at(P, 1, 0), c2 = coef_at(P, 2, 0), sg0 = sgn.p[0] * sgn.amp;
   const size_t stride = static_cast<size_t>(R.W) * Nj, col = static_cast<size_t>(w) * Nj;

@@ -44,3 +44,16 @@ def test_gpu_wide_matches(n, m, aniso, beta_l, T, beta_time):
     c.set_critical_current(np.exp(0.1 * rng.standard_normal(c.junction_count())))
     print(f"[wide] {n}x{m} T={T}", flush=True)
     _compare(_run(c, 512, 2, 36, T, beta_time), _run(c, 1024, 2, 36, T, beta_time))
+
+
+def test_gpu_wide_skips_a_zero_current_source():
+    """A current source that counts as zero (np.allclose) is left out of the step, as in the
+    general kernels, and still added to the stored current."""
+    c = pa.SquareArray(66, 66)
+    Is = 9e-9 * np.cos(np.arange(c.junction_count()))[:, None, None] * np.ones((1, 2, 1))
+    f = 0.1 + 0.1 * np.random.default_rng(0).random(c.face_count())[:, None, None]
+    print("[wide] zero current source", flush=True)
+    a, b = (pa.TimeEvolutionProblem(c, solver="lattice", parts=1, block_size=bs, time_step=0.05, time_step_count=36,
+                                    external_flux=f, current_sources=Is, store_time_steps=[0, 17, 35]).compute()
+            for bs in (512, 1024))
+    _compare(a, b)
