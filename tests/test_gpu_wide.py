@@ -57,3 +57,53 @@ def test_gpu_wide_skips_a_zero_current_source():
                                     external_flux=f, current_sources=Is, store_time_steps=[0, 17, 35]).compute()
             for bs in (512, 1024))
     _compare(a, b)
+
+
+def _lattice(n, m, aniso):
+    c = pa.SquareArray(n, m)
+    x1, y1, x2, y2 = c.get_junction_coordinates()
+    c.set_capacitance(np.where(y1 == y2, 1.0, 2.0) if aniso else 1.0)
+    c.set_critical_current(np.exp(0.1 * np.random.default_rng(n + m).standard_normal(c.junction_count())))
+    return c
+
+
+def _same_bits(a, b):
+    return np.array_equal(a.get_theta(), b.get_theta())
+
+
+# the other combinations of noise and of coefficients that are one value: coefficients of
+# their own with noise, a noise amplitude of their own, neither
+@pytest.mark.parametrize("aniso,T", [(True, 0.02), (False, "junction"), (False, 0.0)])
+def test_gpu_wide_forms_match(aniso, T):
+    """The two workgroup sizes agree, and not bit for bit: the large one's columns lay in
+    registers (fused multiply-adds; the general kernels' results do not depend on the
+    size)."""
+    c = _lattice(71, 70, aniso)
+    if T == "junction":
+        T = 0.01 + 0.02 * np.random.default_rng(5).random((c.junction_count(), 1, 1))
+    print("[wide] forms", flush=True)
+    a, b = (_run(c, bs, 2, 36, T, False) for bs in (512, 1024))
+    _compare(a, b)
+    assert not _same_bits(a, b)
+
+
+def test_gpu_wide_leaves_varying_temperature_to_the_general_kernel():
+    c = _lattice(66, 66, True)
+    assert _same_bits(*(_run(c, bs, 2, 36, 0.02, True) for bs in (512, 1024)))
+
+
+def test_gpu_wide_lattices_share_a_plan():
+    """Two large lattices of different sizes in one launch: each as alone with workgroups of
+    512 threads, and in registers."""
+    print("[wide] batch", flush=True)
+    problems = []
+    for n, m, W, T in ((66, 68, 2, 0.02), (99, 100, 1, 0.0)):
+        c = _lattice(n, m, n == 66)
+        problems.append(dict(circuit=c, time_step=0.05, time_step_count=30, external_flux=0.1, temperature=T, seed=3,
+                             current_sources=c.current_base(0.0)[:, None, None] * np.linspace(0.5, 1.3, W)[None, :, None],
+                             store_time_steps=[0, 11, 29], solver="lattice", parts=1, steps_per_launch=13))
+    both = pa.TimeEvolutionBatch([pa.TimeEvolutionProblem(block_size=1024, **p) for p in problems], block_size=1024).compute()
+    for p, b in zip(problems, both):
+        a = pa.TimeEvolutionProblem(block_size=512, **p).compute()
+        _compare(a, b)
+        assert not _same_bits(a, b)
