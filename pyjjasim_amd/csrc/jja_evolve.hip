@@ -174,6 +174,41 @@ __global__ __launch_bounds__(BS) void adjoint_split_kernel(const DevProblem* __r
   }
 }
 
+// After a launch whose parts keep their junctions on chip: once a wait has given up (err),
+// what the launch left in a column does not look valid, every value becomes NaN. The host
+// is told as well (jja_plan_status), but nobody asks after a replay of a graph. A kernel of
+// its own, one workgroup a column: the same in the step kernels cost them 1 to 3% in
+// spilled scalar registers (256x256, 16 columns), this one some two microseconds a launch.
+constexpr int kVerdictBlock = 256;
+__global__ __launch_bounds__(kVerdictBlock) void evolve_verdict_kernel(const jja_problem_run* __restrict__ runs, int32_t Nj,
+                                                                       const int32_t* __restrict__ err, int32_t n_steps,
+                                                                       int64_t step0) {
+  if (!err[0]) return;
+  const jja_problem_run& R = runs[0];
+  const size_t stride = static_cast<size_t>(R.W) * Nj, col = static_cast<size_t>(blockIdx.x) * Nj;
+  const double bad = __builtin_nan("");
+  for (int32_t j = threadIdx.x; j < Nj; j += kVerdictBlock) R.theta[col + j] = R.theta[stride + col + j] = bad;
+  for (int64_t i = 0; i < n_steps; ++i) {
+    const int64_t at = step0 + i - R.slot_t0;
+    const int32_t tho = R.th_slot ? R.th_slot[at] : -1, Io = R.I_slot ? R.I_slot[at] : -1;
+    for (int32_t j = threadIdx.x; j < Nj; j += kVerdictBlock) {
+      if (tho >= 0) R.th_out[tho * stride + col + j] = bad;
+      if (Io >= 0) R.I_out[Io * stride + col + j] = bad;
+    }
+  }
+}
+
+__global__ __launch_bounds__(kVerdictBlock) void adjoint_verdict_kernel(const jja_adjoint_run* __restrict__ runs, int32_t Nj,
+                                                                        int32_t Nf, const int32_t* __restrict__ err) {
+  if (!err[0]) return;
+  const jja_adjoint_run& A = runs[0];
+  const size_t stride = static_cast<size_t>(A.W) * Nj, w = blockIdx.x;
+  const double bad = __builtin_nan("");
+  for (int32_t j = threadIdx.x; j < Nj; j += kVerdictBlock)
+    A.grad_Ic[w * Nj + j] = A.grad_Is[w * Nj + j] = A.lam[w * Nj + j] = A.lam[stride + w * Nj + j] = bad;
+  for (int32_t f = threadIdx.x; f < Nf; f += kVerdictBlock) A.grad_f[w * Nf + f] = bad;
+}
+
 // n[col][f] = -sum_j A[f,j] rint(theta_j / 2pi) (time_evolution.py:734-755): one
 // workgroup per phase vector, one thread per face position (a workgroup takes
 // the slots of all parts of a split plan in turn).
@@ -1188,8 +1223,13 @@ int launch_evolve_parts(Plan* plan, int32_t n, int32_t n_steps, int64_t step0, h
   const jja_problem_run* runs = plan->use_runs;
   const WorkItem* work = plan->use_work;
   const void* tables = plan->d_parts;
-  return launch_cooperative(plan, plan->parts_evolve, plan->block_size, n, plan->parts_lds, stream, probs, runs, work,
-                            tables, n_steps, step0, plan->d_parts_seq, plan->d_err, plan->wait_limit);
+  if (int rc = launch_cooperative(plan, plan->parts_evolve, plan->block_size, n, plan->parts_lds, stream, probs, runs, work,
+                                  tables, n_steps, step0, plan->d_parts_seq, plan->d_err, plan->wait_limit))
+    return rc;
+  hipLaunchKernelGGL(evolve_verdict_kernel, dim3(n / plan->parts), dim3(kVerdictBlock), 0, stream, runs,
+                     plan->problems[0].Nj, plan->d_err, n_steps, step0);
+  JJA_HIP(hipGetLastError());
+  return JJA_OK;
 }
 
 int launch_adjoint_parts(Plan* plan, int32_t n, int64_t k_hi, int64_t k_lo, hipStream_t stream) {
@@ -1197,8 +1237,13 @@ int launch_adjoint_parts(Plan* plan, int32_t n, int64_t k_hi, int64_t k_lo, hipS
   const jja_adjoint_run* runs = plan->use_adj;
   const WorkItem* work = plan->use_work;
   const void* tables = plan->d_parts;
-  return launch_cooperative(plan, plan->parts_adjoint, plan->block_size, n, plan->parts_lds, stream, probs, runs, work,
-                            tables, k_hi, k_lo, plan->d_parts_seq, plan->d_err, plan->wait_limit);
+  if (int rc = launch_cooperative(plan, plan->parts_adjoint, plan->block_size, n, plan->parts_lds, stream, probs, runs, work,
+                                  tables, k_hi, k_lo, plan->d_parts_seq, plan->d_err, plan->wait_limit))
+    return rc;
+  hipLaunchKernelGGL(adjoint_verdict_kernel, dim3(n / plan->parts), dim3(kVerdictBlock), 0, stream, runs,
+                     plan->problems[0].Nj, plan->problems[0].Nf, plan->d_err);
+  JJA_HIP(hipGetLastError());
+  return JJA_OK;
 }
 
 template <int BS>

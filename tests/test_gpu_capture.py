@@ -112,3 +112,30 @@ def test_replays_keep_their_inputs(make, opts, grad):
                     for a, b in zip(run(evo, X), ref):
                         assert torch.equal(a, b)
             side.synchronize()
+
+
+@pytest.mark.parametrize("make", [lambda: pa.SquareArray(70, 72), lambda: pa.HoneycombArray(16, 16)], ids=["slabs", "domains"])
+def test_a_replay_that_gave_up_shows(make):
+    """Parts that stop waiting for each other (a wait limit of no polls, every kernel still
+    running to its end) leave no phases that look valid: the replay's results hold NaN, the
+    next call outside the graph raises, and the one after that is exact again."""
+    torch = pytest.importorskip("torch")
+    from pyjjasim_amd import _native
+    c, W = make(), 2
+    X = _inputs(torch, c, W, 1)
+    with pa.DifferentiableEvolution(c, time_step=0.05, time_step_count=15, problem_count=W, store_time_steps=[14]) as evo, \
+            torch.no_grad():
+        print(f"[capture] {c.junction_count()} junctions give up", flush=True)
+        want = evo(*X)
+        torch.cuda.synchronize()
+        _native.check(evo.eng.lib.jja_plan_set_wait_limit(evo.eng.handle, 0))
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = evo(*X)
+        _native.check(evo.eng.lib.jja_plan_set_wait_limit(evo.eng.handle, 1 << 21))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.isnan(out).any()
+        with pytest.raises(_native.NativeError, match="gave up"):
+            evo(*X)
+        assert torch.equal(evo(*X), want)
