@@ -290,6 +290,13 @@ int jja_plan_destroy(jja_plan* plan);
  */
 int jja_plan_status(jja_plan* plan);
 /*
+ * The same of the launches that have finished, for a plan whose columns run in slabs or
+ * subdomains, without waiting for the device (it waits only to report a failure; JJA_OK
+ * for other plans). A launch there that gave up leaves NaN in its columns' history,
+ * stored steps and gradients.
+ */
+int jja_plan_poll(jja_plan* plan);
+/*
  * Polls a column barrier of the plan's split launches makes before it gives up
  * (default 2^21, each poll sleeping briefly: far longer than any phase of a
  * step). A small value forces the give-up path, which jja_plan_status then

@@ -107,14 +107,27 @@ class DifferentiableEvolution:
         self.close()
         return False
 
+    def _on_chip(self):
+        """Whether the columns' parts keep their junctions on chip (slabs, subdomains)."""
+        host = self.eng.host
+        return host.slabs or host.domains is not None
+
+    def _check_finished(self):
+        """Raise NativeError if a finished pass in slabs or subdomains gave up waiting
+        between its parts (it left NaN); waits for nothing."""
+        eng = self.eng
+        if self._on_chip() and not self.torch.cuda.is_current_stream_capturing():
+            _native.check(eng.lib.jja_plan_poll(eng.handle))
+
     def _check_status(self):
         """Raise NativeError if a column barrier of a split launch gave up (its
-        results are invalid); waits for the launches of a split plan."""
+        results are invalid); waits for the launches of a plan with column barriers.
+        Passes in slabs or subdomains stay asynchronous, as those of one workgroup:
+        one that gives up leaves NaN, and the next call after it has finished raises."""
         eng = self.eng
-        if eng.host.parts > 1:
-            if self.torch.cuda.is_current_stream_capturing():
-                return  # a replay reports nothing; the next call outside the graph does
-            self.torch.cuda.current_stream().synchronize()
+        if eng.host.parts == 1 or self._on_chip():
+            return
+        self.torch.cuda.current_stream().synchronize()
         _native.check(eng.lib.jja_plan_status(eng.handle))
 
     # ------------------------------------------------------------------ forward
@@ -132,6 +145,7 @@ class DifferentiableEvolution:
     def forward(self, Ic, f, Is):
         """Stored theta (Nj, W, n_stored) and the state the backward needs."""
         eng = self.eng
+        self._check_finished()
         self._set_inputs(Ic, f, Is)
         eng.theta.copy_(self.theta0)
         eng.t = 0
@@ -147,6 +161,7 @@ class DifferentiableEvolution:
     def backward(self, state, g):
         """Gradients (Ic (Nj,), f (W, Nf), Is (W, Nj)) of <g, theta_stored>."""
         torch, eng = self.torch, self.eng
+        self._check_finished()
         ckpt, Ic, f, Is, fsrc, isrc = state
         # the inputs of this graph (another call may have run since)
         self._Ic, self._f, self._Is = Ic, f, Is

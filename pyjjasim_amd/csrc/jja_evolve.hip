@@ -175,15 +175,16 @@ __global__ __launch_bounds__(BS) void adjoint_split_kernel(const DevProblem* __r
 }
 
 // After a launch whose parts keep their junctions on chip: once a wait has given up (err),
-// what the launch left in a column does not look valid, every value becomes NaN. The host
-// is told as well (jja_plan_status), but nobody asks after a replay of a graph. A kernel of
+// what the launch left in a column does not look valid, every value becomes NaN, and the
+// host is told through pinned memory, which it reads without waiting (jja_plan_poll). A kernel of
 // its own, one workgroup a column: the same in the step kernels cost them 1 to 3% in
 // spilled scalar registers (256x256, 16 columns), this one some two microseconds a launch.
 constexpr int kVerdictBlock = 256;
 __global__ __launch_bounds__(kVerdictBlock) void evolve_verdict_kernel(const jja_problem_run* __restrict__ runs, int32_t Nj,
-                                                                       const int32_t* __restrict__ err, int32_t n_steps,
-                                                                       int64_t step0) {
+                                                                       const int32_t* __restrict__ err, int32_t* host_err,
+                                                                       int32_t n_steps, int64_t step0) {
   if (!err[0]) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(host_err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   const jja_problem_run& R = runs[0];
   const size_t stride = static_cast<size_t>(R.W) * Nj, col = static_cast<size_t>(blockIdx.x) * Nj;
   const double bad = __builtin_nan("");
@@ -199,8 +200,10 @@ __global__ __launch_bounds__(kVerdictBlock) void evolve_verdict_kernel(const jja
 }
 
 __global__ __launch_bounds__(kVerdictBlock) void adjoint_verdict_kernel(const jja_adjoint_run* __restrict__ runs, int32_t Nj,
-                                                                        int32_t Nf, const int32_t* __restrict__ err) {
+                                                                        int32_t Nf, const int32_t* __restrict__ err,
+                                                                        int32_t* host_err) {
   if (!err[0]) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(host_err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   const jja_adjoint_run& A = runs[0];
   const size_t stride = static_cast<size_t>(A.W) * Nj, w = blockIdx.x;
   const double bad = __builtin_nan("");
@@ -309,6 +312,8 @@ struct Plan {
   int64_t parts_lds = 0;
   bool parts_only = false;           // subdomains: there is no other way to solve
   uint32_t* d_parts_seq = nullptr;
+  // those launches' report to the host: pinned, 1 once a wait has given up
+  int32_t* host_err = nullptr;
   // every problem's tables for the kernel that holds a large lattice column in the
   // registers of one workgroup, or NULL; its dynamic LDS bytes
   const WideDev* d_wide = nullptr;
@@ -524,6 +529,7 @@ int create_domains(Plan* plan, const jja_problem_desc& d) {
 
 void free_plan(Plan* plan) {
   for (void* p : plan->allocations) (void)hipFree(p);
+  if (plan->host_err) (void)hipHostFree(plan->host_err);
   if (plan->done) (void)hipEventDestroy(plan->done);
   delete plan;
 }
@@ -1227,7 +1233,7 @@ int launch_evolve_parts(Plan* plan, int32_t n, int32_t n_steps, int64_t step0, h
                                   tables, n_steps, step0, plan->d_parts_seq, plan->d_err, plan->wait_limit))
     return rc;
   hipLaunchKernelGGL(evolve_verdict_kernel, dim3(n / plan->parts), dim3(kVerdictBlock), 0, stream, runs,
-                     plan->problems[0].Nj, plan->d_err, n_steps, step0);
+                     plan->problems[0].Nj, plan->d_err, plan->host_err, n_steps, step0);
   JJA_HIP(hipGetLastError());
   return JJA_OK;
 }
@@ -1241,7 +1247,7 @@ int launch_adjoint_parts(Plan* plan, int32_t n, int64_t k_hi, int64_t k_lo, hipS
                                   tables, k_hi, k_lo, plan->d_parts_seq, plan->d_err, plan->wait_limit))
     return rc;
   hipLaunchKernelGGL(adjoint_verdict_kernel, dim3(n / plan->parts), dim3(kVerdictBlock), 0, stream, runs,
-                     plan->problems[0].Nj, plan->problems[0].Nf, plan->d_err);
+                     plan->problems[0].Nj, plan->problems[0].Nf, plan->d_err, plan->host_err);
   JJA_HIP(hipGetLastError());
   return JJA_OK;
 }
@@ -1545,6 +1551,9 @@ int jja_plan_create(int32_t n_problems, const jja_problem_desc* descs, jja_plan*
     const uint32_t* d = nullptr;
     rc = upload(plan, seq.data(), seq.size(), &d);
     plan->d_parts_seq = const_cast<uint32_t*>(d);
+    if (rc == JJA_OK && hipHostMalloc(reinterpret_cast<void**>(&plan->host_err), sizeof(int32_t), hipHostMallocMapped) != hipSuccess)
+      rc = fail(JJA_ENOMEM, "jja_plan_create: pinned host allocation failed");
+    if (rc == JJA_OK) *plan->host_err = 0;
   }
   if (rc == JJA_OK) rc = create_wide(plan, descs, n_problems);
   if (rc == JJA_OK && hipEventCreateWithFlags(&plan->done, hipEventDisableTiming) != hipSuccess)
@@ -1574,7 +1583,15 @@ int jja_plan_status(jja_plan* p) {
   JJA_HIP(hipMemcpy(&e, plan->d_err, sizeof(e), hipMemcpyDeviceToHost));
   if (!e) return JJA_OK;
   JJA_HIP(hipMemset(plan->d_err, 0, sizeof(int32_t)));
+  if (plan->host_err) __atomic_store_n(plan->host_err, 0, __ATOMIC_RELAXED);
   return fail(JJA_EHIP, "a column barrier of a split launch gave up waiting; its results are invalid");
+}
+
+int jja_plan_poll(jja_plan* p) {
+  Plan* plan = reinterpret_cast<Plan*>(p);
+  if (!plan) return fail(JJA_EINVAL, "jja_plan_poll: invalid arguments");
+  if (!plan->host_err || !__atomic_load_n(plan->host_err, __ATOMIC_RELAXED)) return JJA_OK;
+  return jja_plan_status(p);
 }
 
 int64_t jja_plan_one_xcd_parts(jja_plan* p) {

@@ -184,3 +184,44 @@ def test_gpu_plans_with_different_lds_interleave():
         es.close()
     np.testing.assert_array_equal(th_big[:, :, -1], big.compute().get_theta()[:, :, -1])
     np.testing.assert_array_equal(th_small[:, :, -1], small.compute().get_theta()[:, :, -1])
+
+
+@pytest.mark.parametrize("make", [lambda: pa.SquareArray(64, 64), lambda: pa.HoneycombArray(16, 16)], ids=["slabs", "domains"])
+def test_gpu_passes_in_parts_do_not_block(make):
+    """A pass in slabs or subdomains returns while its launch runs, as one of a single
+    workgroup does. One whose parts give up waiting for each other (wait limit zero, every
+    kernel still running to its end) leaves NaN in phases and gradients, a later call
+    raises, and the next is exact."""
+    import torch
+    c, W, Nt = make(), 2, 8000
+    put = lambda a: torch.tensor(a, dtype=torch.float64, device="cuda")
+    X = [put(np.ones(c.junction_count())), put(np.full(c.face_count(), 0.1)), put(0.6 * c.current_base(0.0))]
+    print(f"[errors] {c.junction_count()} junctions in parts, asynchronous", flush=True)
+    with pa.DifferentiableEvolution(c, time_step=0.05, time_step_count=Nt, problem_count=W, store_time_steps=[9],
+                                    checkpoint_every=Nt) as evo:
+        assert evo.eng.host.parts > 1
+        with torch.no_grad():
+            want = evo(*X)
+            torch.cuda.synchronize()
+            out = evo(*X)
+            running = not torch.cuda.current_stream().query()
+            torch.cuda.synchronize()
+        assert running and torch.equal(out, want)
+    kw = dict(time_step=0.05, time_step_count=15, problem_count=W, store_time_steps=[14], checkpoint_every=8)
+    with pa.DifferentiableEvolution(c, **kw) as evo:
+        leaves = [x.clone().requires_grad_(True) for x in X]
+        th = evo(*leaves)
+        want = (th.detach().clone(),) + torch.autograd.grad(th, leaves, torch.ones_like(th))
+        th = evo(*leaves)
+        torch.cuda.synchronize()
+        _native.check(evo.eng.lib.jja_plan_set_wait_limit(evo.eng.handle, 0))
+        grads = torch.autograd.grad(th, leaves, torch.ones_like(th), retain_graph=True)
+        _native.check(evo.eng.lib.jja_plan_set_wait_limit(evo.eng.handle, 1 << 21))
+        torch.cuda.synchronize()
+        assert all(torch.isnan(g).any() for g in grads)
+        with pytest.raises(_native.NativeError, match="gave up"):
+            torch.autograd.grad(th, leaves, torch.ones_like(th))
+        th = evo(*leaves)
+        got = (th.detach().clone(),) + torch.autograd.grad(th, leaves, torch.ones_like(th))
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
