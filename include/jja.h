@@ -279,6 +279,12 @@ typedef struct jja_problem_desc {
  * a device (jja_plan_create runs the same checks before it uploads anything).
  */
 int jja_plan_validate(int32_t n_problems, const jja_problem_desc* problems);
+/*
+ * Whether a plan of this problem alone would run its columns as row slabs
+ * (lattice_slabs): 1, 0 where they do not fit (its columns would then meet at column
+ * barriers), or a negative JJA_E* code. Touches no device.
+ */
+int jja_slabs_fit(const jja_problem_desc* problem);
 /* Create a plan for n_problems circuits on the current HIP device. */
 int jja_plan_create(int32_t n_problems, const jja_problem_desc* problems, jja_plan** out);
 int jja_plan_destroy(jja_plan* plan);

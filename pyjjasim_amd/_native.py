@@ -105,7 +105,7 @@ _lib = None
 
 EXPORTS = ["jja_cholesky", "jja_factor_get", "jja_factor_free", "jja_factor_last_error",
            "jja_plan_validate", "jja_plan_create", "jja_plan_destroy", "jja_plan_lds_bytes",
-           "jja_plan_zbuf_doubles", "jja_plan_status", "jja_plan_poll", "jja_plan_set_wait_limit",
+           "jja_plan_zbuf_doubles", "jja_plan_status", "jja_plan_poll", "jja_slabs_fit", "jja_plan_set_wait_limit",
            "jja_plan_one_xcd_parts", "jja_evolve",
            "jja_vortex", "jja_adjoint", "jja_solve", "jja_solve_noalloc", "jja_last_error"]
 
@@ -132,6 +132,8 @@ def lib():
     L.jja_plan_zbuf_doubles.restype = C.c_int64
     L.jja_plan_status.argtypes = [C.c_void_p]
     L.jja_plan_status.restype = C.c_int
+    L.jja_slabs_fit.argtypes = [C.POINTER(ProblemDesc)]
+    L.jja_slabs_fit.restype = C.c_int
     L.jja_plan_poll.argtypes = [C.c_void_p]
     L.jja_plan_poll.restype = C.c_int
     L.jja_plan_set_wait_limit.argtypes = [C.c_void_p, C.c_uint32]

@@ -406,13 +406,17 @@ int upload(Plan* plan, const T* host, size_t n, const T** out) {
   return JJA_OK;
 }
 
+// Whether a plan of this problem alone is asked for row slabs.
+bool wants_slabs(const jja_problem_desc& d) {
+  return d.lattice_slabs && d.lattice_rows && d.n_junctions > 0 && d.parts >= 2 && d.block_size == d.parts * kPartBlock;
+}
+
 // The slab form of a split lattice problem, where it asks for it and fits.
 int create_slabs(Plan* plan, const jja_problem_desc& d) {
-  if (!d.lattice_slabs || !d.lattice_rows || plan->parts < 2 || plan->block_size != kPartBlock) return JJA_OK;
+  if (!wants_slabs(d)) return JJA_OK;
   SlabHost h;
   if (!build_slabs(d, plan->parts, kSplitLdsMax, &h)) return JJA_OK;
   const int32_t per = (std::max(h.d.pairs, h.d.faces) + kPartBlock - 1) / kPartBlock;
-  if (per > kSlabPairs) return JJA_OK;
   const std::vector<double> table = dst_table(d.lattice_cols);
   int rc;
   if ((rc = upload(plan, h.pair.data(), h.pair.size(), &h.d.pair))) return rc;
@@ -1336,6 +1340,13 @@ int jja_plan_validate(int32_t n_problems, const jja_problem_desc* descs) {
   for (int32_t p = 0; p < n_problems; ++p)
     if (int rc = validate(descs[p])) return rc;
   return JJA_OK;
+}
+
+int jja_slabs_fit(const jja_problem_desc* d) {
+  if (!d) return fail(JJA_EINVAL, "jja_slabs_fit: invalid arguments");
+  if (int rc = check_plan_shapes(1, d)) return rc;
+  if (int rc = validate(*d)) return rc;
+  return wants_slabs(*d) && slabs_fit(*d, d->parts, kSplitLdsMax) ? 1 : 0;
 }
 
 int jja_plan_create(int32_t n_problems, const jja_problem_desc* descs, jja_plan** out) {

@@ -43,9 +43,10 @@ struct SlabHost {
 // Doubles of dynamic LDS one workgroup of a slab launch takes.
 int64_t slab_lds_doubles(const SlabDev& d, int32_t cols);
 
-// Cuts the lattice problem into `parts` slabs; false (with a reason) when a
-// junction joins faces that are not neighbours, a face has more than four
-// junctions, or a local index does not fit.
+// Whether the lattice problem can be cut into `parts` slabs: every junction joins
+// neighbours, no face has more than four, the slabs fit in LDS, a thread's registers and
+// local indices. build_slabs cuts it and makes the tables.
+bool slabs_fit(const jja_problem_desc& desc, int32_t parts, int64_t lds_bytes);
 bool build_slabs(const jja_problem_desc& desc, int32_t parts, int64_t lds_bytes, SlabHost* out);
 
 // Kernels (workgroups of kPartBlock threads) whose threads hold at most `pairs`

@@ -371,7 +371,10 @@ int64_t slab_lds_doubles(const SlabDev& d, int32_t cols) {
          (d.table_lds ? DstShape(cols).entries() : 0) + 1;
 }
 
-bool build_slabs(const jja_problem_desc& desc, int32_t parts, int64_t lds_bytes, SlabHost* out) {
+namespace {
+
+// The parts' junctions and faces and what LDS holds: everything but the tables.
+bool cut_slabs(const jja_problem_desc& desc, int32_t parts, int64_t lds_bytes, SlabHost* out) {
   const int32_t R = desc.lattice_rows, C = desc.lattice_cols, Nj = desc.n_junctions, G = parts;
   if (R < 2 * G || C < 8 || G < 2) return false;  // two rows a part: its first and its last
   SlabDev& d = out->d;
@@ -414,7 +417,15 @@ bool build_slabs(const jja_problem_desc& desc, int32_t parts, int64_t lds_bytes,
     for (int32_t v : mask[p]) n += v != 0;
     d.pairs = std::max(d.pairs, n);
   }
-  if (2 * d.pairs > 32767 || Nj >= (1 << 27)) return false;
+  d.ends_rows = (2 * G + 3) / 4 * 4;
+  if (2 * d.pairs > 32767 || Nj >= (1 << 27) || std::max(d.pairs, d.faces) > kSlabPairs * kPartBlock) return false;
+  // LDS: the pivots, then the sine table, where there is room
+  d.inv_lds = d.table_lds = 0;
+  if (8 * slab_lds_doubles(d, C) > lds_bytes) return false;
+  d.inv_lds = 1;
+  if (8 * slab_lds_doubles(d, C) > lds_bytes) d.inv_lds = 0;
+  d.table_lds = 1;
+  if (8 * slab_lds_doubles(d, C) > lds_bytes) d.table_lds = 0;
   out->pair.assign(static_cast<size_t>(G) * d.pairs, -1);
   out->pair_code.assign(2 * static_cast<size_t>(G) * d.pairs, 0xffffffffu);
   out->face_id.assign(static_cast<size_t>(G) * d.faces, -1);
@@ -461,20 +472,26 @@ bool build_slabs(const jja_problem_desc& desc, int32_t parts, int64_t lds_bytes,
                                      static_cast<uint32_t>(fcode[4 * static_cast<size_t>(e) + 2 * i + 1]) << 16;
     }
   }
+  return true;
+}
+
+}  // namespace
+
+bool slabs_fit(const jja_problem_desc& desc, int32_t parts, int64_t lds_bytes) {
+  SlabHost h;
+  return cut_slabs(desc, parts, lds_bytes, &h);
+}
+
+bool build_slabs(const jja_problem_desc& desc, int32_t parts, int64_t lds_bytes, SlabHost* out) {
+  if (!cut_slabs(desc, parts, lds_bytes, out)) return false;
+  const int32_t R = desc.lattice_rows, C = desc.lattice_cols, G = parts;
+  SlabDev& d = out->d;
   std::vector<double> reduced;
   row_part_tables(R, C, G, desc.lattice_g, desc.lattice_gc, &out->inv, &out->spike, &reduced);
-  d.ends_rows = (2 * G + 3) / 4 * 4;
   out->reduced.assign(2 * static_cast<size_t>(G) * d.ends_rows * C, 0.0);
   for (int32_t r = 0; r < 2 * G; ++r)
     std::copy_n(&reduced[2 * static_cast<size_t>(r) * G * C], 2 * static_cast<size_t>(G) * C,
                 &out->reduced[static_cast<size_t>(r) * d.ends_rows * C]);
-  // LDS: the pivots, then the sine table, where there is room
-  d.inv_lds = d.table_lds = 0;
-  if (8 * slab_lds_doubles(d, C) > lds_bytes) return false;
-  d.inv_lds = 1;
-  if (8 * slab_lds_doubles(d, C) > lds_bytes) d.inv_lds = 0;
-  d.table_lds = 1;
-  if (8 * slab_lds_doubles(d, C) > lds_bytes) d.table_lds = 0;
   return true;
 }
 

@@ -187,6 +187,20 @@ def slab_parts(host, columns, n_cu, max_parts=16):
     return 1 if parts == 2 and host.Nj <= RESIDENT_JUNCTIONS else parts
 
 
+def slab_layout(host, parts):
+    """The plan laid out for ``parts`` row slabs a column; where they do not fit (a long
+    narrow lattice takes more LDS than its junctions suggest), None if one workgroup holds
+    the column's faces, else as many parts with column barriers (us a step in one workgroup
+    and in such parts: 9x701, 100 columns 51 / 122; 11x1501, 40 columns 180 / 104). None
+    for one part."""
+    if parts == 1:
+        return None
+    sliced = host.relayout(SLAB_BLOCK, parts, slabs=True)
+    if _native.lib().jja_slabs_fit(C.byref(sliced.desc())) == 1:
+        return sliced
+    return host.relayout(SLAB_BLOCK, parts) if host.global_store else None
+
+
 # subdomains of any other circuit (jja_domain.hip): the fewest faces a part has, and
 # the most faces of a circuit that two parts take (us a step: a 10x10 honeycomb array
 # 14.7 in one workgroup, 11 in 2 to 4; 30x30 with 64 columns 39.3 in one, 33.7 in 2,
@@ -252,9 +266,9 @@ class Engine:
             self.block_size = self.host.block_size
             parts = getattr(problem, "parts", None)
             slabs = slab_parts(self.host, W, device_compute_units()) if parts_open else 1
-            if slabs > 1:
-                self.block_size = SLAB_BLOCK
-                self.host = self.host.relayout(SLAB_BLOCK, slabs, slabs=True)
+            sliced = slab_layout(self.host, slabs)
+            if sliced is not None:
+                self.block_size, self.host = SLAB_BLOCK, sliced
                 parts = 1
             elif self.host.domains is not None:
                 parts = 1
