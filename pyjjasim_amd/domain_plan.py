@@ -102,6 +102,7 @@ class DomainPlan:
     def __init__(self, K, xy, junc_code, parts):
         self.parts = parts
         self.ok = False
+        self._desc = None
         K = scipy.sparse.csr_matrix(K)
         Nf, Nj = K.shape[0], len(junc_code) // 2
         self.Nf, self.Nj = Nf, Nj
@@ -346,7 +347,10 @@ class DomainPlan:
             self.source[g, :len(s)] = s
 
     def desc(self):
-        """ctypes jja_domains pointing at this object's arrays (keep it alive)."""
+        """ctypes jja_domains pointing at this object's arrays (keep it alive); the same
+        one on every call, since problem descriptors hold its address."""
+        if self._desc is not None:
+            return self._desc
         d, C = _native.Domains(), _native.C
         d.parts, d.pairs, d.faces, d.n_gamma = self.parts, self.pairs, self.n_local, len(self.gamma)
         d.sources, d.n_published, d.n_records = self.sources, int(self.pub_ptr[-1]), len(self.slices)
@@ -358,7 +362,14 @@ class DomainPlan:
             setattr(self, name, a)
             setattr(d, name, a.ctypes.data)
         d.n_slice_rows, d.n_entries, d.n_index = len(self.slice_rows), len(self.ent_val), len(self.ent_off)
+        self._desc = d
         return d
+
+    def __getstate__(self):
+        # pointers to this object's arrays: made again on the other side
+        state = dict(self.__dict__, _desc=None)
+        state.pop("_records", None)
+        return state
 
     # ----------------------------------------------------------- host emulation
     def emulate(self, b):

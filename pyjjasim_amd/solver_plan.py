@@ -1131,8 +1131,7 @@ class CircuitPlan:
             self.lattice.set_desc(d)
             d.lattice_slabs = int(self.slabs)
         if getattr(self, "domains", None) is not None:
-            self._domain_desc = self.domains.desc()
-            d.domains = C.addressof(self._domain_desc)
+            d.domains = C.addressof(self.domains.desc())
         return d
 
     def lds_bytes(self):

@@ -114,3 +114,23 @@ def test_domain_plans_stand_alone():
         setattr(d, name, 0)
         d.n_face_slices = 0
         assert lib.jja_plan_validate(1, C.byref(d)) == -1, name
+
+
+def test_domain_plan_pickles_and_keeps_its_descriptors():
+    """A plan with subdomains pickles after its descriptor was made, as every plan does, and
+    a descriptor stays valid when another is made of the same plan."""
+    import ctypes as C
+    import pickle
+    from pyjjasim_amd import _native
+    plan = CircuitPlan(pa.HoneycombArray(11, 9), 0.05, domains=4)
+    first = plan.desc(max_columns=2)
+    head = C.cast(first.domains, C.POINTER(_native.Domains)).contents
+    records = head.records
+    second = plan.desc(max_columns=3)
+    assert first.domains == second.domains and head.records == records
+    lib = _native.lib()
+    assert lib.jja_plan_validate(1, C.byref(first)) == 0 and lib.jja_plan_validate(1, C.byref(second)) == 0
+    copy = pickle.loads(pickle.dumps(plan))
+    assert lib.jja_plan_validate(1, C.byref(copy.desc(max_columns=2))) == 0
+    b = np.random.default_rng(0).standard_normal(plan.Nf)
+    np.testing.assert_array_equal(copy.domains.emulate(b), plan.domains.emulate(b))
