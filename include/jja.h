@@ -264,7 +264,9 @@ typedef struct jja_problem_desc {
    * x_r = d_r - ((-g) inv[r][k]) x_{r+1} */
   const double* lattice_inv;
   double lattice_g;            /* g */
-  double lattice_gc;           /* g_c */
+  /* g_c, or 0 where it is not given: the tables above then solve every column, and none
+   * of the forms that keep a lattice's column on chip is taken */
+  double lattice_gc;
   /* NULL, or the subdomains that solve the face system of a plan of this problem
    * alone (parts >= 2 equal to theirs, block_size 512 * parts, index_bytes 4,
    * lattice_rows 0, solve positions in circuit order). There are then no solve

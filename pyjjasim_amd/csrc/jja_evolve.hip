@@ -408,7 +408,7 @@ int upload(Plan* plan, const T* host, size_t n, const T** out) {
 
 // Whether a plan of this problem alone is asked for row slabs.
 bool wants_slabs(const jja_problem_desc& d) {
-  return d.lattice_slabs && d.lattice_rows && d.n_junctions > 0 && d.parts >= 2 && d.block_size == d.parts * kPartBlock;
+  return d.lattice_slabs && d.lattice_rows && d.lattice_gc > 0.0 && d.n_junctions > 0 && d.parts >= 2 && d.block_size == d.parts * kPartBlock;
 }
 
 // The slab form of a split lattice problem, where it asks for it and fits.
@@ -456,7 +456,7 @@ int create_wide(Plan* plan, const jja_problem_desc* descs, int32_t n) {
   std::vector<WideHost> h(n);
   int64_t lds = 0;
   for (int32_t i = 0; i < n; ++i) {
-    if (!descs[i].lattice_rows || plan->problems[i].lat_ld || plan->problems[i].index_bytes != 2 ||
+    if (!descs[i].lattice_rows || !(descs[i].lattice_gc > 0.0) || plan->problems[i].lat_ld || plan->problems[i].index_bytes != 2 ||
         !build_wide(descs[i], plan->lds_limit, &h[i]))
       return JJA_OK;
     lds = std::max(lds, 8 * wide_lds_doubles(h[i].d, descs[i].n_junctions));
@@ -857,8 +857,8 @@ int validate(const jja_problem_desc& d) {
     if (ms < (Nf & 1) + std::max(2 * R * EF, 4 * B * C))
       return fail(JJA_EINVAL, "max_stage_rows too small for the lattice solve");
     if (!(d.lattice_g > 0.0) || !std::isfinite(d.lattice_g)) return fail(JJA_EINVAL, "lattice_g must be finite and > 0");
-    if (!(d.lattice_gc > 0.0) || !std::isfinite(d.lattice_gc))
-      return fail(JJA_EINVAL, "lattice_gc must be finite and > 0");
+    if (!(d.lattice_gc >= 0.0) || !std::isfinite(d.lattice_gc))
+      return fail(JJA_EINVAL, "lattice_gc must be finite and > 0, or 0 where it is not given");
     return JJA_OK;
   }
   if (d.domains) return validate_domains(d);
@@ -1424,7 +1424,8 @@ int jja_plan_create(int32_t n_problems, const jja_problem_desc* descs, jja_plan*
       const int32_t ld = dc.padded() + 4;
       const int64_t buf = static_cast<int64_t>(dr.padded()) * ld;
       const int64_t tables = dc.entries() + (R == C ? 0 : dr.entries());
-      if (d.index_bytes == 2 && R <= TileShape::kSide && C <= TileShape::kSide) {
+      const bool solve_in_modes = d.lattice_gc > 0.0;  // both factors known
+      if (solve_in_modes && d.index_bytes == 2 && R <= TileShape::kSide && C <= TileShape::kSide) {
         dp.lat_tile = 1;
         dp.lat_ld = TileShape::kLd;
         dp.lat_buf = TileShape::kSide * TileShape::kLd;
@@ -1432,7 +1433,7 @@ int jja_plan_create(int32_t n_problems, const jja_problem_desc* descs, jja_plan*
         dp.store_doubles = dp.lat_tab + 3 * TileShape::kTable;
         const std::vector<double> t = tile_table(R, C, d.lattice_g, d.lattice_gc);
         if ((rc = upload(plan, t.data(), t.size(), &dp.lat_table))) break;
-      } else if (d.index_bytes == 2 && R >= 8 && C >= 8 && 8 * (2 * buf + tables) <= plan->lds_limit) {
+      } else if (solve_in_modes && d.index_bytes == 2 && R >= 8 && C >= 8 && 8 * (2 * buf + tables) <= plan->lds_limit) {
         dp.lat_ld = ld;
         dp.lat_buf = static_cast<int32_t>(buf);
         dp.lat_tab = static_cast<int32_t>(2 * buf);

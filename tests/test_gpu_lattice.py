@@ -189,3 +189,23 @@ def test_gpu_split_lattice_with_idle_parts_matches_oracle():
     th = res.get_theta()
     assert np.abs(th - ref["theta"]).max() <= 1e-9 * np.abs(ref["theta"]).max()
     np.testing.assert_array_equal(res.get_vortex_configuration(), to.vortex(c.get_cycle_matrix(), ref["theta"]))
+
+
+# sides a wave, the padded products and large columns in registers would take
+@pytest.mark.parametrize("n,m,block_size", [(9, 8, None), (20, 24, None), (66, 66, 1024)])
+def test_gpu_lattice_without_its_column_factor(monkeypatch, n, m, block_size):
+    """A lattice whose descriptor does not give lattice_gc is solved by its tables alone."""
+    from pyjjasim_amd.lattice_solve import LatticeSolve
+    c = pa.SquareArray(n, m)
+    kw = dict(time_step=0.05, time_step_count=30, external_flux=0.1, store_time_steps=[0, 29], solver="lattice", parts=1,
+              block_size=block_size, current_sources=c.current_base(0.0)[:, None, None] * np.array([0.6, 1.3])[None, :, None])
+    print(f"[lattice] {n}x{m} without its column factor", flush=True)
+    want = pa.TimeEvolutionProblem(c, **kw).compute().get_theta()
+    given = LatticeSolve.set_desc
+
+    def without(self, d):
+        given(self, d)
+        d.lattice_gc = 0.0
+    monkeypatch.setattr(LatticeSolve, "set_desc", without)
+    got = pa.TimeEvolutionProblem(c, **kw).compute().get_theta()
+    assert np.abs(got - want).max() <= 1e-9 * np.abs(want).max()

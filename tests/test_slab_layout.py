@@ -43,3 +43,16 @@ def test_slabs_fit_checks_its_problem():
     d = plan.desc()
     d.max_columns = 0
     assert lib.jja_slabs_fit(C.byref(d)) == -1                     # JJA_EINVAL
+
+
+def test_lattice_without_its_column_factor_is_accepted():
+    """A lattice descriptor that leaves lattice_gc at 0 (its tables solve it) passes the
+    checks and gets no slabs; a wrong one does not pass."""
+    lib, host = _native.lib(), _plan(64, 64)
+    plan = host.relayout(512, 8, slabs=True)
+    d = plan.desc()
+    d.lattice_gc = 0.0
+    assert lib.jja_plan_validate(1, C.byref(d)) == 0 and lib.jja_slabs_fit(C.byref(d)) == 0
+    for wrong in (-1.0, float("nan"), float("inf")):
+        d.lattice_gc = wrong
+        assert lib.jja_plan_validate(1, C.byref(d)) == -1
