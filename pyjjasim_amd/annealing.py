@@ -157,6 +157,7 @@ class AnnealingProblem:
             _native.check(end.lib.jja_vortex(end.handle, end.index, th.data_ptr(), W, n.data_ptr(),
                                              torch.cuda.current_stream().cuda_stream))
             n = n.cpu().numpy().T.astype(int)
+            _native.check(end.lib.jja_plan_status(end.handle))
         finally:
             end.close()
         f = np.atleast_1d(self.external_flux)[:, None, None]

@@ -54,3 +54,23 @@ def test_gpu_annealing_philox_lowers_temperature():
         if st == 0:
             assert cfg.is_solution()
             assert abs(cfg.get_vortex_configuration().sum() - round(0.2 * c.face_count())) <= 2
+
+
+def test_gpu_annealing_reports_a_wait_that_gave_up(monkeypatch):
+    """The closing runs at zero temperature are checked as the annealing itself is: parts
+    that stop waiting for each other there (wait limit zero) raise."""
+    from pyjjasim_amd import _native, annealing
+    made = []
+
+    class Impatient(annealing.Engine):
+        def __init__(self, *a, **k):
+            super().__init__(*a, **k)
+            made.append(self.host.parts)
+            if len(made) == 2:
+                _native.check(self.lib.jja_plan_set_wait_limit(self.handle, 0))
+    monkeypatch.setattr(annealing, "Engine", Impatient)
+    c = pa.HoneycombArray(16, 16)
+    print("[annealing] give-up in the closing runs", flush=True)
+    with pytest.raises(_native.NativeError, match="gave up"):
+        pa.AnnealingProblem(c, time_step=0.5, interval_steps=10, external_flux=0.1, interval_count=3, seed=1).compute()
+    assert made[1] > 1
