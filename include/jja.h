@@ -176,6 +176,20 @@ typedef struct jja_domains {
   const uint16_t* ent_off;
 } jja_domains;
 
+/*
+ * The records of subdomains from phases given as rows (HOST code, no device): program p
+ * runs phases program_ptr[p] .. program_ptr[p + 1] - 1, phase h rows phase_ptr[h] ..
+ * phase_ptr[h + 1] - 1 with flags[h] (JJA_SLICE_BLOCK or 0), row r writes address rows[r]
+ * from entries row_ptr[r] .. row_ptr[r + 1] - 1 (val, and idx below 65536). With records
+ * NULL only the sizes are set: records, entries of ent_val and of ent_off, slice_rows.
+ * Otherwise sizes holds them on entry and the arrays receive the programs of `waves` waves
+ * each, wave_ptr [n_programs][waves + 1].
+ */
+int jja_domain_programs(int32_t n_programs, int32_t waves, const int32_t* program_ptr, const int64_t* phase_ptr,
+                        const int32_t* flags, const int32_t* rows, const int64_t* row_ptr, const int32_t* idx,
+                        const double* val, int64_t* sizes, jja_slice* records, int32_t* wave_ptr, double* ent_val,
+                        uint16_t* ent_off, int32_t* slice_rows);
+
 typedef struct jja_problem_desc {
   int32_t n_junctions;
   int32_t n_faces;

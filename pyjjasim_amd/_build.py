@@ -24,7 +24,7 @@ HIPCC_FLAGS = [
 
 
 def sources():
-    return [os.path.join(CSRC, name) for name in ("jja_evolve.hip", "jja_resident.hip", "jja_slab.hip", "jja_wide.hip", "jja_domain.hip", "jja_factor.cpp")]
+    return [os.path.join(CSRC, name) for name in ("jja_evolve.hip", "jja_resident.hip", "jja_slab.hip", "jja_wide.hip", "jja_domain.hip", "jja_factor.cpp", "jja_program.cpp")]
 
 
 def build_library(verbose=False):

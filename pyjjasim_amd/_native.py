@@ -103,7 +103,7 @@ class NativeError(RuntimeError):
 
 _lib = None
 
-EXPORTS = ["jja_cholesky", "jja_factor_get", "jja_factor_free", "jja_factor_last_error",
+EXPORTS = ["jja_domain_programs", "jja_cholesky", "jja_factor_get", "jja_factor_free", "jja_factor_last_error",
            "jja_plan_validate", "jja_plan_create", "jja_plan_destroy", "jja_plan_lds_bytes",
            "jja_plan_zbuf_doubles", "jja_plan_status", "jja_plan_poll", "jja_slabs_fit", "jja_plan_set_wait_limit",
            "jja_plan_one_xcd_parts", "jja_evolve",
@@ -120,6 +120,7 @@ def lib():
     L = C.CDLL(LIB_PATH)
     L.jja_cholesky.argtypes = [C.c_int32, i64p, i32p, f64p, C.POINTER(C.c_void_p), i64p]
     L.jja_factor_get.argtypes = [C.c_void_p, i64p, i32p, f64p]
+    L.jja_domain_programs.argtypes = [C.c_int32, C.c_int32] + 13 * [C.c_void_p]
     L.jja_factor_free.argtypes = [C.c_void_p]
     L.jja_factor_free.restype = None
     L.jja_factor_last_error.restype = C.c_char_p

@@ -30,7 +30,7 @@ import numpy as np
 import scipy.sparse
 
 from . import _native
-from .solver_plan import MAX_ITER, WAVE, CircuitPlan
+from .solver_plan import WAVE
 
 BLOCK = 512                 # threads of a workgroup
 MAX_PAIRS = 4 * BLOCK       # junction pairs of one workgroup
@@ -39,6 +39,8 @@ MAX_GAMMA = 4096            # separator faces
 FACE_CODES = 8              # junctions of a face
 LDS_DOUBLES = 163840 // 8 - 32
 CELLS = (1, 2, 4, 8, 16, 32)
+# jja_slice
+RECORD = np.dtype([("base", "<i8"), ("ibase", "<i8"), ("rowbase", "<i4"), ("r0", "<i4"), ("n_iter", "<i4"), ("flags", "<i4")])
 
 
 def bisect(faces, xy, touched, levels):
@@ -72,26 +74,16 @@ def spd_inverse(M):
     return inv
 
 
-class _Programs(CircuitPlan):
-    """The wave-program builder of CircuitPlan on phases given as rows."""
-
-    def __init__(self, phases):
-        self.block_size, self.parts = BLOCK, 1
-        self.global_store, self.index_bytes = False, 2
-        self._build_wave_program(phases, MAX_ITER)
-
-
 def _phase(rows, blocks, kind):
-    """A phase for the builder: row i sums dense blocks (row numbers, column
-    addresses, matrix) in turn."""
+    """A phase of a program: row i sums dense blocks (row numbers, column addresses,
+    matrix) in turn."""
     n = len(rows)
     who = np.concatenate([np.repeat(r, len(c)) for r, c, _ in blocks])
     order = np.argsort(who, kind="stable")
     idx = np.concatenate([np.tile(c, len(r)) for r, c, _ in blocks])[order]
     val = np.concatenate([M.ravel() for _, _, M in blocks])[order]
     lens = np.bincount(who, minlength=n)
-    ptr = np.concatenate(([0], np.cumsum(lens)))
-    return (0, np.asarray(rows, dtype=np.int64), ptr, idx, val, kind, None, "col", "col")
+    return np.asarray(rows, dtype=np.int32), lens, idx, val, kind
 
 
 class DomainPlan:
@@ -129,14 +121,19 @@ class DomainPlan:
         # separator faces that border each interior, then those of the junctions it is given
         border = [set(gamma[touched(f)[gamma]].tolist()) for f in interiors]
         load = np.bincount(owner[owner >= 0], minlength=parts)
+        beside = {int(g): {p for p in range(parts) if int(g) in border[p]} for g in gamma}   # the parts that border it
         for j in np.flatnonzero(owner < 0):
             mine = [int(f) for f in face[j] if f >= 0]
-            fits = [p for p in range(parts) if all(f in border[p] for f in mine)] or \
-                [p for p in range(parts) if any(f in border[p] for f in mine)] or list(range(parts))
-            p = min(fits, key=lambda q: load[q])
+            held = [beside[f] for f in mine]
+            # a part that borders all of them, else any of them, else any part; the
+            # least loaded, the first among equals
+            fits = (set.intersection(*held) or set.union(*held)) if held else set()
+            p = min(sorted(fits) or range(parts), key=lambda q: load[q])
             owner[j] = p
             load[p] += 1
             border[p].update(mine)
+            for f in mine:
+                beside[f].add(p)
         # a separator face that no part borders would never be published
         for f in gamma:
             if not any(f in b for b in border):
@@ -312,27 +309,28 @@ class DomainPlan:
         return before, after
 
     def _programs(self):
-        slices, vals, offs, rows, wave_ptr = [], [], [], [], []
-        n_val = n_off = n_row = n_rec = 0
-        self.entries = 0
-        for p in range(self.parts):
-            for phases in self._phases(p):
-                self.entries += sum(len(ph[4]) for ph in phases)
-                prog = _Programs(phases)
-                wave_ptr.append(prog.wave_ptr + n_rec)
-                slices += [(b + n_val, ib + n_off, rb + n_row, r0, it, fl)
-                           for b, ib, rb, r0, it, fl in prog.solve_slices]
-                vals.append(prog.ent_val)
-                offs.append(prog.ent_off)
-                rows.append(prog.slice_rows)
-                n_rec += len(prog.solve_slices)
-                n_val += len(prog.ent_val)
-                n_off += len(prog.ent_off)
-                n_row += len(prog.slice_rows)
-        self.slices = slices
-        self.ent_val, self.ent_off = np.concatenate(vals), np.concatenate(offs)
-        self.slice_rows = np.concatenate(rows)
-        self.wave_ptr = np.ascontiguousarray(np.concatenate(wave_ptr), dtype=np.int32)
+        programs = [half for p in range(self.parts) for half in self._phases(p)]
+        phases = [ph for half in programs for ph in half]
+        self.entries = sum(len(ph[2]) for ph in phases)
+        ends = lambda counts, t: np.concatenate(([0], np.cumsum(counts))).astype(t)
+        given = [ends([len(half) for half in programs], np.int32), ends([len(ph[0]) for ph in phases], np.int64),
+                 np.array([ph[4] for ph in phases], dtype=np.int32), np.concatenate([ph[0] for ph in phases]),
+                 ends(np.concatenate([ph[1] for ph in phases]), np.int64),
+                 np.concatenate([ph[2] for ph in phases]).astype(np.int32), np.concatenate([ph[3] for ph in phases])]
+        sizes = np.zeros(3, dtype=np.int64)
+        waves = BLOCK // WAVE
+
+        def build(*made):
+            args = [a.ctypes.data for a in given] + [sizes.ctypes.data] + [a.ctypes.data if a is not None else None for a in made]
+            rc = _native.lib().jja_domain_programs(len(programs), waves, *args)
+            if rc != _native.JJA_OK:
+                raise _native.NativeError(f"jja_domain_programs: libjja error {rc}")
+        build(None, None, None, None, None)
+        self.records = np.empty(sizes[0], dtype=RECORD)
+        self.wave_ptr = np.empty(len(programs) * (waves + 1), dtype=np.int32)
+        self.ent_val, self.ent_off = np.empty(sizes[1]), np.empty(sizes[1], dtype=np.uint16)
+        self.slice_rows = np.empty(sizes[2], dtype=np.int32)
+        build(self.records, self.wave_ptr, self.ent_val, self.ent_off, self.slice_rows)
         # published contributions: part by part, the border in order; their sources
         # per separator face
         self.pub_ptr = np.concatenate(([0], np.cumsum([len(b) for b in self.border]))).astype(np.int32)
@@ -351,12 +349,10 @@ class DomainPlan:
         one on every call, since problem descriptors hold its address."""
         if self._desc is not None:
             return self._desc
-        d, C = _native.Domains(), _native.C
+        d = _native.Domains()
         d.parts, d.pairs, d.faces, d.n_gamma = self.parts, self.pairs, self.n_local, len(self.gamma)
-        d.sources, d.n_published, d.n_records = self.sources, int(self.pub_ptr[-1]), len(self.slices)
-        self._records = CircuitPlan._slice_array(self.slices)
-        d.records = C.cast(self._records, C.c_void_p)
-        for name in ("pair", "pair_code", "face_code", "face_id", "face_used", "pub_ptr", "pub_at", "source", "wave_ptr",
+        d.sources, d.n_published, d.n_records = self.sources, int(self.pub_ptr[-1]), len(self.records)
+        for name in ("records", "pair", "pair_code", "face_code", "face_id", "face_used", "pub_ptr", "pub_at", "source", "wave_ptr",
                      "slice_rows", "ent_val", "ent_off"):
             a = np.ascontiguousarray(getattr(self, name))
             setattr(self, name, a)
@@ -367,9 +363,7 @@ class DomainPlan:
 
     def __getstate__(self):
         # pointers to this object's arrays: made again on the other side
-        state = dict(self.__dict__, _desc=None)
-        state.pop("_records", None)
-        return state
+        return dict(self.__dict__, _desc=None)
 
     # ----------------------------------------------------------- host emulation
     def emulate(self, b):
@@ -379,7 +373,8 @@ class DomainPlan:
         phases = [self._phases(p) for p in range(self.parts)]
 
         def run(m, ph):
-            _, rows, ptr, idx, val, kind, _, _, _ = ph
+            rows, lens, idx, val, kind = ph
+            ptr = np.concatenate(([0], np.cumsum(lens)))
             sums = np.array([np.dot(val[ptr[i]:ptr[i + 1]], m[idx[ptr[i]:ptr[i + 1]]]) for i in range(len(rows))])
             m[rows] = sums if kind else m[rows] - sums
         pub = np.zeros(int(self.pub_ptr[-1]))

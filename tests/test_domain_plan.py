@@ -134,3 +134,40 @@ def test_domain_plan_pickles_and_keeps_its_descriptors():
     assert lib.jja_plan_validate(1, C.byref(copy.desc(max_columns=2))) == 0
     b = np.random.default_rng(0).standard_normal(plan.Nf)
     np.testing.assert_array_equal(copy.domains.emulate(b), plan.domains.emulate(b))
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_domain_programs_match_the_plan_builder(seed):
+    """The library's programs for phases given as rows are those of the builder of the
+    staged factor, record by record: rows of no entry, of one, of a lane's eight and one
+    more, of all lanes' 512 and more; phases without rows and waves without work."""
+    import ctypes as C
+    from pyjjasim_amd import _native
+    rng = np.random.default_rng(seed)
+    lens = [rng.permutation([0, 1, 7, 8, 9, 63, 64, 65, 511, 512, 513, 1100, *rng.integers(0, 700, n)])[:n] for n in (0, 1, 5, 150)]
+    rows = [rng.permutation(2000)[:len(l)].astype(np.int32) for l in lens]
+    kinds = [0, _native.SLICE_BLOCK, _native.SLICE_BLOCK, 0]
+    idx = [rng.integers(0, 65536, int(l.sum())).astype(np.int32) for l in lens]
+    val = [rng.standard_normal(int(l.sum())) for l in lens]
+
+    class Builder(CircuitPlan):
+        def __init__(self):
+            self.block_size, self.parts, self.global_store, self.index_bytes = 512, 1, False, 2
+            self._build_wave_program([(0, r, np.concatenate(([0], np.cumsum(l))), i, v, k, None, "col", "col")
+                                      for r, l, i, v, k in zip(rows, lens, idx, val, kinds)], 8)
+    want = Builder()
+    ends = lambda counts, t: np.concatenate(([0], np.cumsum(counts))).astype(t)
+    given = [ends([4], np.int32), ends([len(l) for l in lens], np.int64), np.array(kinds, np.int32), np.concatenate(rows),
+             ends(np.concatenate(lens), np.int64), np.concatenate(idx), np.concatenate(val)]
+    sizes = np.zeros(3, np.int64)
+    point = lambda *arrays: [a.ctypes.data for a in arrays]
+    lib = _native.lib()
+    assert lib.jja_domain_programs(1, 8, *point(*given, sizes), *[None] * 5) == 0
+    made = [np.empty((sizes[0], 8), np.int32), np.empty(9, np.int32), np.empty(sizes[1]), np.empty(sizes[1], np.uint16),
+            np.empty(sizes[2], np.int32)]
+    assert lib.jja_domain_programs(1, 8, *point(*given, sizes, *made)) == 0
+    np.testing.assert_array_equal(made[0].view(np.int64)[:, :2], [s[:2] for s in want.solve_slices])
+    np.testing.assert_array_equal(made[0][:, 4:], [s[2:] for s in want.solve_slices])
+    for got, name in zip(made[1:], ("wave_ptr", "ent_val", "ent_off", "slice_rows")):
+        np.testing.assert_array_equal(got, getattr(want, name), err_msg=name)
+    assert lib.jja_domain_programs(1, 0, *point(*given, sizes), *[None] * 5) == -1
