@@ -12,9 +12,12 @@ run's host set-up and its warmup (its GPU work also brings the device to its
 working clock). Reported:
 
   value      junction-steps/s = Nj * W * steps / wall time
-  roofline   algorithmic HBM bytes per launch / mean launch time (HIP events on the
-             launch stream) against the 8 TB/s HBM peak
-  plain      the one-problem-at-a-time GPU loop (W = 1) on the same circuit
+  roofline   what bounds the kernel that ran, by mean launch time (HIP events on the launch
+             stream): operations of the step against the FP64 peak where the columns
+             stay on chip, algorithmic HBM bytes against 8 TB/s where they lie in memory.
+             scheme_bytes: those bytes in either case, moved or not
+  plain      the one-problem-at-a-time GPU loop (W = 1) on the same circuit, in the
+             fastest of the layout it gets by itself and the explicit ones
   cpu_baseline  the FP64 numpy/scipy restatement of the reference scheme (same
              library calls), timed on this host on a bounded sample of steps
 
@@ -39,6 +42,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
+FP64_PEAK_TFLOPS = 78.6
 WORKLOAD = "batched_iv_sweep_square100_W256"
 
 
@@ -108,6 +112,7 @@ def run_gpu(pa, torch, n, W, steps, warmup, steps_per_launch, block_size, events
                 stored_in_window=int(th_mask[warmup:].sum()),
                 nnz_factor=int(len(sp.lo_val) + len(sp.inv_cm)), nnz_L=int(sp.nnz_L),
                 n_stages=sp.n_stages, block_size=eng.block_size, parts=eng.host.parts,
+                on_chip_parts=eng.host.slabs or eng.host.domains is not None, global_store=eng.host.global_store,
                 steps_per_launch=eng.steps_per_launch,
                 solver="lattice" if lat is not None else "cholesky",
                 lattice=None if lat is None else {"rows": lat.R, "cols": lat.C,
@@ -468,19 +473,41 @@ def host_info():
             "scipy": scipy.__version__, "thread_env": env}
 
 
-def plain_best(pa, torch, n, steps, amplitude=1.0, parts_options=(1, 2, 4, 8, 16)):
+def step_flops(info, W):
+    """Operations a step cannot do without, as far as they can be counted without saying
+    how: 150 a junction (stencil and sine 90, thermal deviate 60) and 60 a face (its
+    sum and a fast direct solve)."""
+    return W * (150 * info["Nj"] + 60 * info["Nf"])
+
+
+def kernel_of(info):
+    """The step kernel that a run with this layout takes (usual step, no other problem in
+    its plan) and the threads of one workgroup of it."""
+    if info["on_chip_parts"]:
+        return "evolve_parts_kernel", info["block_size"]
+    if info["parts"] == 1 and not info["global_store"]:
+        if info["block_size"] <= 512:
+            return "evolve_resident_kernel", info["block_size"]
+        # lattices with a side that leaves no room for the padded solve
+        if info["lattice"] and max(info["lattice"]["rows"], info["lattice"]["cols"]) > 64:
+            return "evolve_wide_kernel", 512
+    return ("evolve_kernel" if info["parts"] == 1 else "evolve_split_kernel"), info["block_size"]
+
+
+def plain_best(pa, torch, n, steps, amplitude=1.0, parts_options=(None, 1, 2, 4, 8, 16)):
     """The plain loop: one problem (one bias point, W = 1) at a time, in its
-    fastest single-problem layout: one workgroup with the LDS face store (the
-    lattice solve), or the column split over 2..16 workgroups with the global
-    face store (the factor). Returns the best rate and every layout's ms/step."""
+    fastest single-problem layout: the one it gets by itself (row slabs), one
+    workgroup with the LDS face store, or the column split over 2..16 workgroups with
+    column barriers. Returns the best rate and every layout's ms/step."""
     per = {}
     for parts in parts_options:
-        opts = {"parts": parts} if parts > 1 else {"parts": 1}
-        if parts > 1:
+        opts = {} if parts is None else {"parts": parts}
+        if parts is not None and parts > 1:
             opts["face_store"] = "global"
         wall, _, _, _, c, info = run_gpu(pa, torch, n, 1, steps, 100, None, None, events=False,
                                          amplitudes=[amplitude], **opts)
-        per[f"parts{parts}_{info['solver']}"] = wall / steps * 1e3
+        name = f"parts{info['parts']}_{info['solver']}"
+        per["auto_" + name if parts is None else name] = wall / steps * 1e3
     best = min(per, key=per.get)
     Nj = 2 * n * (n - 1)
     return {"value": Nj / (per[best] * 1e-3), "unit": "junction-steps/s", "layout": best,
@@ -594,9 +621,8 @@ def main():
                                                prelude=prelude, solver=args.solver)
     Nj, W, K = info["Nj"], args.W, args.steps
     value = Nj * W * K / wall
-    # dominant kernel: evolve_kernel; one launch advances k steps of the whole
-    # batch. Algorithmic bytes of the timed launches: B_step per step plus the
-    # theta rows stored within them
+    # one launch of the step kernel advances k steps of the whole batch. Algorithmic
+    # bytes of the timed launches: B_step per step plus the theta rows stored within them
     tot_steps = sum(k for k, _ in launch_ms)
     tot_ms = sum(ms for _, ms in launch_ms)
     n_launch = len(launch_ms)
@@ -604,6 +630,18 @@ def main():
     bytes_timed = info["bytes_per_step"] * tot_steps + info["bytes_per_stored_step"] * info["stored_in_window"]
     bytes_per_launch = bytes_timed / n_launch
     achieved = bytes_per_launch / (mean_launch_ms * 1e-3) / 1e9
+    kernel, threads = kernel_of(info)
+    tflops = step_flops(info, W) * tot_steps / (tot_ms * 1e-3) / 1e12
+    scheme_bytes = {"per_step": info["bytes_per_step"], "per_launch": bytes_per_launch, "GB_per_s": achieved,
+                    "of_hbm_peak": achieved / HBM_PEAK_GBS,
+                    "note": "bytes of the scheme with its state in memory; a kernel that keeps the state on chip "
+                            "does not move them (traffic: measured)"}
+    if kernel in ("evolve_kernel", "evolve_split_kernel"):
+        bound = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                 "frac": achieved / HBM_PEAK_GBS}
+    else:
+        bound = {"bound": "fp64", "achieved": tflops, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
+                 "frac": tflops / FP64_PEAK_TFLOPS, "flops_per_step": step_flops(info, W)}
     traffic = traffic_note = None
     if (args.n, W) == (100, 256):
         mt = measured_traffic()
@@ -635,13 +673,12 @@ def main():
                    "junctions": Nj, "faces": info["Nf"], "W": W, "dt": 0.05, "T": 0.01,
                    "beta_C": 1.0, "f": 0.25, "Nt": args.warmup + K,
                    "bias": "SeparableSource(current_base(0), linspace(0, 2, W))",
-                   "steps_per_launch": info["steps_per_launch"], "block_size": info["block_size"],
+                   "steps_per_launch": info["steps_per_launch"], "block_size": threads,
                    "parts": info["parts"], "solver": info["solver"],
                    "solve_stages": info["n_stages"] if info["solver"] == "cholesky" else None},
-        "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "traffic_source": traffic_note,
-                     "kernel": "evolve_wide_kernel", "bytes_per_step": info["bytes_per_step"],
-                     "bytes_per_launch": bytes_per_launch, "stored_steps_in_window": info["stored_in_window"],
+        "roofline": {**bound, "traffic": traffic, "traffic_source": traffic_note,
+                     "kernel": kernel, "scheme_bytes": scheme_bytes,
+                     "stored_steps_in_window": info["stored_in_window"],
                      "mean_launch_ms": mean_launch_ms, "launches": n_launch},
         "plain": plain,
     }
