@@ -1,10 +1,12 @@
 """Many time-evolution problems in one launch per chunk of steps.
 
 ``TimeEvolutionBatch(problems).compute()`` returns one TimeEvolutionResult per
-problem, each identical to ``problem.compute()`` run with the layout the batch
-gave it (``layouts``: workgroup size, parts per column, face store; the factor
-gives the same bits in any layout, while the lattice solve's rounding depends
-on the face store and the part count): the problems (any circuits,
+problem, as ``problem.compute()`` run with the layout the batch gave it
+(``layouts``: workgroup size, parts per column, face store) would: bit for bit with
+the factor, whose bits do not depend on the layout, and where both runs take the
+same kernel; the lattice solve's rounding depends on the face store, the part
+count and on whether large lattices stay in registers (with workgroups of 1024
+threads, if every problem of the launch allows it). The problems (any circuits,
 sizes and column counts; one stencil width and step count) share one libjja
 plan, and every launch advances the columns of all of them. By default a
 column is one workgroup: circuits whose face vector fits in LDS keep it there,

@@ -29,6 +29,10 @@ __device__ __forceinline__ T stream_offset(const GAS T* base, uint32_t bytes) {
   return __builtin_nontemporal_load(reinterpret_cast<const GAS T*>(reinterpret_cast<const GAS char*>(base) + bytes));
 }
 
+// The transforms here are those of jja_rowdst.h (whose header says why they are as they
+// are) without its blocks of four rows: with that code in this kernel, which holds 160
+// registers of state, its forms spilled 46 to 138 registers.
+//
 // The table's values of four steps are loaded together, a batch ahead of the products
 // (and the next task's first ones before the last steps of a task): they come from the
 // L2, which answers in 1000 to 2000 cycles here, and the matrix pipe works on a batch

@@ -127,7 +127,10 @@ TURN_BYTES = 1 << 28
 # junctions up to which a column's whole state fits in one workgroup's LDS
 # beside the face vector (or in registers): the kernels for that take at most
 # 512 threads, which then have 256 registers each (1024 threads spilled over 100
-# of their 128). Larger lattices take 1024, or the registers of jja_wide.hip
+# of their 128). Larger lattices take 1024, or the registers of jja_wide.hip. Runs that
+# those kernels refuse lose nothing by the smaller workgroups (us a step with 1024 / 512
+# threads, 256 columns, stencil 4: 25x25 16.4 / 9.7, 55x55 34.6 / 28.9, 20x20 honeycomb
+# 31.5 / 25.4, 30x30 triangular 55.7 / 51.8; voltage sources there 55.5 / 56.1)
 RESIDENT_JUNCTIONS = 6144
 
 
