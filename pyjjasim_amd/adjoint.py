@@ -57,6 +57,10 @@ def _term(tensor, n, W, name):
 class DifferentiableEvolution:
     """Differentiable stencil-3 time evolution of one circuit for W columns.
 
+    A call returns while the device works, forward and backward, except where parts meet
+    at column barriers. Passes share the evolution's state: they run one after the other,
+    replays of captured ones among them.
+
     Arguments follow TimeEvolutionProblem (time_evolution.py:94-103); the
     external flux and the bias currents are the call's tensors and are constant
     in time. ``checkpoint_every`` steps are recomputed per backward segment.
@@ -90,6 +94,7 @@ class DifferentiableEvolution:
         pos = self.eng.host.face_of_pos.astype(np.int64)
         self.face_of_pos = torch.from_numpy(pos).to(self.eng.dev)
         self.n_seg = -(-self.Nt // self.C)
+        self._stream = None                          # of the last eager pass in parts
 
     def __call__(self, Ic, f, Is):
         return _apply(Ic, f, Is, self)
@@ -114,9 +119,14 @@ class DifferentiableEvolution:
 
     def _check_finished(self):
         """Raise NativeError if a finished pass in slabs or subdomains gave up waiting
-        between its parts (it left NaN); waits for nothing."""
-        eng = self.eng
-        if self._on_chip() and not self.torch.cuda.is_current_stream_capturing():
+        between its parts (it left NaN). Waits for nothing, unless the last pass went to
+        another stream: the passes share the evolution's state."""
+        eng, cuda = self.eng, self.torch.cuda
+        if self._on_chip() and not cuda.is_current_stream_capturing():
+            stream = cuda.current_stream()
+            if self._stream is not None and self._stream != stream:
+                self._stream.synchronize()
+            self._stream = stream
             _native.check(eng.lib.jja_plan_poll(eng.handle))
 
     def _check_status(self):

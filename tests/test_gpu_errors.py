@@ -225,3 +225,36 @@ def test_gpu_passes_in_parts_do_not_block(make):
         got = (th.detach().clone(),) + torch.autograd.grad(th, leaves, torch.ones_like(th))
         for a, b in zip(got, want):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("make", [lambda: pa.SquareArray(64, 64), lambda: pa.HoneycombArray(16, 16)], ids=["slabs", "domains"])
+def test_gpu_passes_in_parts_change_streams(make):
+    """Passes in slabs or subdomains that follow each other on different streams, forward
+    and backward, wait for each other: they share the evolution's state."""
+    import torch
+    c, W, Nt = make(), 2, 3000
+    put = lambda a: torch.tensor(a, dtype=torch.float64, device="cuda")
+    inputs = [[put(np.ones(c.junction_count())), put(np.full(c.face_count(), 0.1)), put(b * c.current_base(0.0))] for b in (0.6, 0.9)]
+    print(f"[errors] {c.junction_count()} junctions in parts, two streams", flush=True)
+    with pa.DifferentiableEvolution(c, time_step=0.05, time_step_count=Nt, problem_count=W, store_time_steps=[9, Nt - 1],
+                                    checkpoint_every=Nt // 2) as evo:
+        assert evo.eng.host.parts > 1
+        want = []
+        for X in inputs:
+            leaves = [x.clone().requires_grad_(True) for x in X]
+            th = evo(*leaves)
+            want.append([th.detach().clone()] + [g.clone() for g in torch.autograd.grad(th, leaves, torch.ones_like(th))])
+        torch.cuda.synchronize()
+        streams = [torch.cuda.Stream() for _ in range(2)]
+        got, held = [], []
+        for k in range(4):
+            with torch.cuda.stream(streams[k % 2]):
+                leaves = [x.clone().requires_grad_(True) for x in inputs[k % 2]]
+                th = evo(*leaves)
+                ones = torch.ones_like(th)
+                got.append([th.detach().clone(), *torch.autograd.grad(th, leaves, ones)])
+                held.append((leaves, th, ones))
+        torch.cuda.synchronize()
+        for k, outs in enumerate(got):
+            for a, b in zip(outs, want[k % 2]):
+                assert torch.equal(a, b)
