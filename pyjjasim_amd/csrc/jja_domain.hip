@@ -114,7 +114,7 @@ struct DomainSolver {
           }
         if (__all(ready)) break;
         if (++spins > wait_limit) {
-          // gives up for the rest of the launch; the verdict kernel after it tells the host
+          // gives up for the rest of the launch; a kernel after it (evolve_spoil_kernel) tells the host
           // and spoils the results
           *stopped = 1;
           __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

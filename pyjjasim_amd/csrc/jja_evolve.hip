@@ -37,6 +37,7 @@
 #include <cstdint>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -179,37 +180,37 @@ __global__ __launch_bounds__(BS) void adjoint_split_kernel(const DevProblem* __r
 // host is told through pinned memory, which it reads without waiting (jja_plan_poll). A kernel of
 // its own, one workgroup a column: the same in the step kernels cost them 1 to 3% in
 // spilled scalar registers (256x256, 16 columns), this one some two microseconds a launch.
-constexpr int kVerdictBlock = 256;
-__global__ __launch_bounds__(kVerdictBlock) void evolve_verdict_kernel(const jja_problem_run* __restrict__ runs, int32_t Nj,
-                                                                       const int32_t* __restrict__ err, int32_t* host_err,
-                                                                       int32_t n_steps, int64_t step0) {
+constexpr int kSpoilBlock = 256;
+__global__ __launch_bounds__(kSpoilBlock) void evolve_spoil_kernel(const jja_problem_run* __restrict__ runs, int32_t Nj,
+                                                                   const int32_t* __restrict__ err, int32_t* host_err,
+                                                                   int32_t n_steps, int64_t step0) {
   if (!err[0]) return;
   if (blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(host_err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   const jja_problem_run& R = runs[0];
   const size_t stride = static_cast<size_t>(R.W) * Nj, col = static_cast<size_t>(blockIdx.x) * Nj;
   const double bad = __builtin_nan("");
-  for (int32_t j = threadIdx.x; j < Nj; j += kVerdictBlock) R.theta[col + j] = R.theta[stride + col + j] = bad;
+  for (int32_t j = threadIdx.x; j < Nj; j += kSpoilBlock) R.theta[col + j] = R.theta[stride + col + j] = bad;
   for (int64_t i = 0; i < n_steps; ++i) {
     const int64_t at = step0 + i - R.slot_t0;
     const int32_t tho = R.th_slot ? R.th_slot[at] : -1, Io = R.I_slot ? R.I_slot[at] : -1;
-    for (int32_t j = threadIdx.x; j < Nj; j += kVerdictBlock) {
+    for (int32_t j = threadIdx.x; j < Nj; j += kSpoilBlock) {
       if (tho >= 0) R.th_out[tho * stride + col + j] = bad;
       if (Io >= 0) R.I_out[Io * stride + col + j] = bad;
     }
   }
 }
 
-__global__ __launch_bounds__(kVerdictBlock) void adjoint_verdict_kernel(const jja_adjoint_run* __restrict__ runs, int32_t Nj,
-                                                                        int32_t Nf, const int32_t* __restrict__ err,
-                                                                        int32_t* host_err) {
+__global__ __launch_bounds__(kSpoilBlock) void adjoint_spoil_kernel(const jja_adjoint_run* __restrict__ runs, int32_t Nj,
+                                                                    int32_t Nf, const int32_t* __restrict__ err,
+                                                                    int32_t* host_err) {
   if (!err[0]) return;
   if (blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(host_err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   const jja_adjoint_run& A = runs[0];
   const size_t stride = static_cast<size_t>(A.W) * Nj, w = blockIdx.x;
   const double bad = __builtin_nan("");
-  for (int32_t j = threadIdx.x; j < Nj; j += kVerdictBlock)
+  for (int32_t j = threadIdx.x; j < Nj; j += kSpoilBlock)
     A.grad_Ic[w * Nj + j] = A.grad_Is[w * Nj + j] = A.lam[w * Nj + j] = A.lam[stride + w * Nj + j] = bad;
-  for (int32_t f = threadIdx.x; f < Nf; f += kVerdictBlock) A.grad_f[w * Nf + f] = bad;
+  for (int32_t f = threadIdx.x; f < Nf; f += kSpoilBlock) A.grad_f[w * Nf + f] = bad;
 }
 
 // n[col][f] = -sum_j A[f,j] rint(theta_j / 2pi) (time_evolution.py:734-755): one
@@ -619,8 +620,12 @@ int keep_copy(Plan* plan, const void* host, size_t bytes, const void** out) {
   if (e == hipSuccess) e = hipStreamSynchronize(side);
   (void)hipStreamDestroy(side);
   if (e != hipSuccess) return fail(JJA_EHIP, std::string("captured launch: copy of its descriptors: ") + hipGetErrorString(e));
-  const char* bytes0 = static_cast<const char*>(host);
-  plan->kept.push_back({std::vector<char>(bytes0, bytes0 + bytes), d});
+  try {
+    const char* first = static_cast<const char*>(host);
+    plan->kept.push_back({std::vector<char>(first, first + bytes), d});
+  } catch (const std::bad_alloc&) {
+    return fail(JJA_ENOMEM, "captured launch: out of host memory");
+  }
   plan->kept_chunk += room;
   plan->kept_left -= room;
   plan->kept_bytes += room;
@@ -1236,7 +1241,7 @@ int launch_evolve_parts(Plan* plan, int32_t n, int32_t n_steps, int64_t step0, h
   if (int rc = launch_cooperative(plan, plan->parts_evolve, plan->block_size, n, plan->parts_lds, stream, probs, runs, work,
                                   tables, n_steps, step0, plan->d_parts_seq, plan->d_err, plan->wait_limit))
     return rc;
-  hipLaunchKernelGGL(evolve_verdict_kernel, dim3(n / plan->parts), dim3(kVerdictBlock), 0, stream, runs,
+  hipLaunchKernelGGL(evolve_spoil_kernel, dim3(n / plan->parts), dim3(kSpoilBlock), 0, stream, runs,
                      plan->problems[0].Nj, plan->d_err, plan->host_err, n_steps, step0);
   JJA_HIP(hipGetLastError());
   return JJA_OK;
@@ -1250,7 +1255,7 @@ int launch_adjoint_parts(Plan* plan, int32_t n, int64_t k_hi, int64_t k_lo, hipS
   if (int rc = launch_cooperative(plan, plan->parts_adjoint, plan->block_size, n, plan->parts_lds, stream, probs, runs, work,
                                   tables, k_hi, k_lo, plan->d_parts_seq, plan->d_err, plan->wait_limit))
     return rc;
-  hipLaunchKernelGGL(adjoint_verdict_kernel, dim3(n / plan->parts), dim3(kVerdictBlock), 0, stream, runs,
+  hipLaunchKernelGGL(adjoint_spoil_kernel, dim3(n / plan->parts), dim3(kSpoilBlock), 0, stream, runs,
                      plan->problems[0].Nj, plan->problems[0].Nf, plan->d_err, plan->host_err);
   JJA_HIP(hipGetLastError());
   return JJA_OK;
@@ -1344,9 +1349,13 @@ int jja_plan_validate(int32_t n_problems, const jja_problem_desc* descs) {
 
 int jja_slabs_fit(const jja_problem_desc* d) {
   if (!d) return fail(JJA_EINVAL, "jja_slabs_fit: invalid arguments");
-  if (int rc = check_plan_shapes(1, d)) return rc;
-  if (int rc = validate(*d)) return rc;
-  return wants_slabs(*d) && slabs_fit(*d, d->parts, kSplitLdsMax) ? 1 : 0;
+  try {
+    if (int rc = check_plan_shapes(1, d)) return rc;
+    if (int rc = validate(*d)) return rc;
+    return wants_slabs(*d) && slabs_fit(*d, d->parts, kSplitLdsMax) ? 1 : 0;
+  } catch (const std::bad_alloc&) {
+    return fail(JJA_ENOMEM, "jja_slabs_fit: out of host memory");
+  }
 }
 
 int jja_plan_create(int32_t n_problems, const jja_problem_desc* descs, jja_plan** out) {

@@ -285,7 +285,7 @@ __device__ __forceinline__ void SlabSolver<AHEAD>::solve(const DevProblem& P, co
         const uint32_t v = __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (__all(static_cast<int32_t>(v - seq) >= 0)) break;
         if (++spins > wait_limit) {
-          // gives up for the rest of the launch; the verdict kernel after it tells the host
+          // gives up for the rest of the launch; a kernel after it (evolve_spoil_kernel) tells the host
           // and spoils the results
           *stopped = 1;
           __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -378,7 +378,8 @@ namespace {
 // The parts' junctions and faces and what LDS holds: everything but the tables.
 bool cut_slabs(const jja_problem_desc& desc, int32_t parts, int64_t lds_bytes, SlabHost* out) {
   const int32_t R = desc.lattice_rows, C = desc.lattice_cols, Nj = desc.n_junctions, G = parts;
-  if (R < 2 * G || C < 8 || G < 2) return false;  // two rows a part: its first and its last
+  // two rows a part: its first and its last; more columns, rows or junctions fit in no way
+  if (R < 2 * G || C < 8 || G < 2 || 2 * C > kPartBlock || R / G > 32767 || Nj >= (1 << 27)) return false;
   SlabDev& d = out->d;
   d.parts = G;
   d.base = R / G;
@@ -420,7 +421,7 @@ bool cut_slabs(const jja_problem_desc& desc, int32_t parts, int64_t lds_bytes, S
     d.pairs = std::max(d.pairs, n);
   }
   d.ends_rows = (2 * G + 3) / 4 * 4;
-  if (2 * d.pairs > 32767 || Nj >= (1 << 27) || std::max(d.pairs, d.faces) > kSlabPairs * kPartBlock) return false;
+  if (2 * d.pairs > 32767 || std::max(d.pairs, d.faces) > kSlabPairs * kPartBlock) return false;
   // LDS: the pivots, then the sine table, where there is room
   d.inv_lds = d.table_lds = 0;
   if (8 * slab_lds_doubles(d, C) > lds_bytes) return false;
